@@ -33,7 +33,11 @@ FLAGS = [
 # per-file flags: the FFT kernels feed literal zeros into their register DFTs
 # for the grid slots outside the sphere, and x + 0 folds to x only when the
 # sign of zero may be ignored
-EXTRA_FLAGS = {"qepw_fft.hip": ["-fno-signed-zeros"]}
+EXTRA_FLAGS = {"qepw_fft.hip": ["-fno-signed-zeros"],
+               # contraction off: the grouped and one-problem plane kernels agree
+               # bit for bit (their fused multiply-adds are written out)
+               "qepw_plane_c128.hip": ["-fno-signed-zeros", "-ffp-contract=off"],
+               "qepw_plane_c64.hip": ["-fno-signed-zeros", "-ffp-contract=off"]}
 
 
 def _compile(src: Path) -> Path:

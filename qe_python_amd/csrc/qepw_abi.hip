@@ -96,6 +96,12 @@ void free_plan(qepw::Plan& p) {
     p.d_tw64[a] = nullptr;
     p.d_tw32[a] = nullptr;
   }
+  for (int a = 0; a < 2; ++a) {
+    hipFree(p.d_ltw64[a]);
+    hipFree(p.d_ltw32[a]);
+    p.d_ltw64[a] = nullptr;
+    p.d_ltw32[a] = nullptr;
+  }
   hipFree(p.d_perm);
   p.d_perm = nullptr;
 }
@@ -218,11 +224,10 @@ static int plan_create_impl(const int32_t* miller, int64_t npw, int n1, int n2, 
   for (int a = 0; a < 3; ++a) p.line[a] = lp[a];
   p.sphere.nst = nst;
   p.sphere.nxcols = (int)sphere.xcols.size();
-  if (n1 == n2) {
-    std::vector<int> stick_y(nst);
-    for (int s = 0; s < nst; ++s) stick_y[s] = sphere.plane[s] % n2;
-    p.sphere.slot_mask = qepw::team_slot_mask(n1, sphere.xcols, stick_y);
-  }
+  std::vector<int> stick_y(nst);
+  for (int s = 0; s < nst; ++s) stick_y[s] = sphere.plane[s] % n2;
+  p.sphere.xmask = qepw::team_slot_mask(n1, sphere.xcols);
+  p.sphere.ymask = qepw::team_slot_mask(n2, stick_y);
   p.sphere.npoints = npw;
   p.sphere.group = qepw::stick_group_for(n3, nst);
   p.sphere.ngroups = (nst + p.sphere.group - 1) / p.sphere.group;
@@ -252,6 +257,25 @@ static int plan_create_impl(const int32_t* miller, int64_t npw, int n1, int n2, 
     }
     e = upload(&p.d_tw64[a], t64);
     if (e == hipSuccess) e = upload(&p.d_tw32[a], t32);
+    const int l = qepw::team_L(n);
+    if (a < 2 && l > 0) {
+      // the same w^(t k) in the order of a team's lanes
+      const int m = n / l;
+      std::vector<double2> lane64((size_t)2 * n);
+      std::vector<float2> lane32((size_t)2 * n);
+      for (int k = 0; k < l; ++k)
+        for (int t = 0; t < m; ++t) {
+          lane64[(size_t)k * m + t] = t64[(size_t)(t * k) % n];
+          lane32[(size_t)k * m + t] = t32[(size_t)(t * k) % n];
+        }
+      for (int k = 0; k < m; ++k)
+        for (int t = 0; t < l; ++t) {
+          lane64[(size_t)n + k * l + t] = t64[(size_t)(t * k) % n];
+          lane32[(size_t)n + k * l + t] = t32[(size_t)(t * k) % n];
+        }
+      if (qepw::plane_lane_table(n, true) && e == hipSuccess) e = upload(&p.d_ltw64[a], lane64);
+      if (qepw::plane_lane_table(n, false) && e == hipSuccess) e = upload(&p.d_ltw32[a], lane32);
+    }
   }
   hipSetDevice(prev);
   if (e != hipSuccess) {
@@ -259,6 +283,8 @@ static int plan_create_impl(const int32_t* miller, int64_t npw, int n1, int n2, 
     delete plan;
     return fail_hip(e, "qepw_plan_create");
   }
+  p.sphere.plane64 = qepw::plane_choice<double>(p, p.sphere);
+  p.sphere.plane32 = qepw::plane_choice<float>(p, p.sphere);
   *out = plan;
   return QEPW_OK;
 }

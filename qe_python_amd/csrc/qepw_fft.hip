@@ -282,14 +282,10 @@ static void launch_split(bool real_mode, const Plan& p, const StickTables& st, c
   const size_t lc = (size_t)gc * p.n2 * sizeof(cplx<T>);
   const size_t lr = (size_t)gr * p.n1 * sizeof(cplx<T>);
   const int64_t tband = split_band_elems(p, st);
-  hipFuncSetAttribute(reinterpret_cast<const void*>(&k_split_cols_inverse<T>),
-                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lc);
-  hipFuncSetAttribute(reinterpret_cast<const void*>(&k_split_cols_forward<T>),
-                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lc);
-  hipFuncSetAttribute(reinterpret_cast<const void*>(&k_split_rows<T, kPlaneApply>),
-                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lr);
-  hipFuncSetAttribute(reinterpret_cast<const void*>(&k_split_rows<T, kPlaneReal>),
-                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lr);
+  allow_lds(reinterpret_cast<const void*>(&k_split_cols_inverse<T>), lc);
+  allow_lds(reinterpret_cast<const void*>(&k_split_cols_forward<T>), lc);
+  allow_lds(reinterpret_cast<const void*>(&k_split_rows<T, kPlaneApply>), lr);
+  allow_lds(reinterpret_cast<const void*>(&k_split_rows<T, kPlaneReal>), lr);
   const dim3 gcols((unsigned)((st.nxcols + gc - 1) / gc), (unsigned)p.n3, (unsigned)nb);
   const dim3 grows((unsigned)((p.n2 + gr - 1) / gr), (unsigned)p.n3, (unsigned)nb);
   hipLaunchKernelGGL(k_split_cols_inverse<T>, gcols, dim3(kSplitThreads), lc, stream, work,
@@ -309,35 +305,7 @@ static void launch_split(bool real_mode, const Plan& p, const StickTables& st, c
                      gc, p.line[1], twiddles<T>(p, 1));
 }
 
-// Fast xy-plane kernel for square planes (n1 = n2 = N): the LDS holds only
-// the nxc active x columns of the plane, Q[c * NP + y], plus one all-zero
-// column; every 1-D FFT is a register "team" FFT (qepw_regfft.h).
-//
-// The backward transforms are decimation-in-frequency team FFTs, whose input
-// slot s of lane t is position t + M s: the sphere's x and y extents leave
-// whole slots empty for every lane (with the usual grids only s = 0, 1, L-2,
-// L-1 hold sticks), so with KEEP naming the occupied slots the empty inputs
-// are literal zeros that the compiler folds away (this file is built with
-// -fno-signed-zeros for that), and the loads of them disappear.  The forward
-// transforms are decimation-in-time team FFTs, whose output slot s of lane t
-// is again position t + M s: only the kept slots are computed and stored.
-// The row pass chains backward x-FFT (DIF), V(r) multiply and forward x-FFT
-// (DIT) in registers -- the DIT consumes the DIF's output order -- at two
-// team exchanges per row.
-//
-// LDS holds the plane and nothing else, so that more workgroups share a CU
-// (FP64 at the 72^3 workload: 42 KB, three per CU): a column FFT exchanges
-// through its own column (its values are in registers by then), and the row
-// pass reads a batch of rows into registers, after which the plane's storage
-// is free and each team exchanges through a line of it; the outputs wait in
-// registers until every team is done, then go back to their rows.
 constexpr int kTeamThreads = 256;
-constexpr int kPlaneTeamThreads = 256;
-
-// Column stride padding of the plane kernel's LDS plane (one element in
-// both precisions: strides of N + 2, 3, 5 and 9 FP32 elements measured the
-// same at the 72^3 workload).
-template <typename T> constexpr int plane_pad() { return 1; }
 
 template <int N> struct TeamGeom {
   static constexpr int L = team_L(N);
@@ -347,206 +315,16 @@ template <int N> struct TeamGeom {
   // input slots kept by the pruned kernel: the first two and the last two
   static constexpr unsigned all = (1u << L) - 1u;
   static constexpr unsigned pruned = L >= 6 ? (0x3u | (0x3u << (L - 2))) : all;
-  // the plane kernel's workgroup: kPlaneTeamThreads threads, plane_teams
-  // teams -- enough for the usual sphere's active columns in one round of
-  // each column pass and the rows in two rounds
-  static constexpr int plane_teams = (kPlaneTeamThreads / 64) * per_wave;
-  // rows a team holds in registers per batch of the plane kernel's row pass:
-  // all of its rows when there are at most three, and then the row pass
-  // exchanges through the plane's own storage; else one, with exchange lines
-  // of their own after the plane
-  static constexpr int rows = (N + plane_teams - 1) / plane_teams;
-  static constexpr bool rows_in_place = rows <= 3;
-  static constexpr int row_batch = rows_in_place ? rows : 1;
 };
 
-template <typename T, int N, bool PRUNE>
-__device__ __forceinline__ void planes_team_body(
-    int z, int64_t b, cplx<T>* __restrict__ work, int64_t band_stride, int nst,
-    const int* __restrict__ colpos, const int* __restrict__ colmap, int nxc,
-    const T* __restrict__ V, const cplx<T>* __restrict__ tw) {
-  using G = TeamGeom<N>;
-  constexpr int L = G::L, M = G::M, RB = G::row_batch;
-  constexpr unsigned KEEP = PRUNE ? G::pruned : G::all;
-  extern __shared__ unsigned char smem_raw[];
-  // Q[c * NP + y]: active column c, padded stride NP = N + 1 so that the
-  // columns start on different LDS banks.  Column nxc stays zero through the
-  // column passes: the row pass reads the inactive x positions from it and
-  // writes their (discarded) outputs to it.
-  constexpr int NP = N + plane_pad<T>();
-  cplx<T>* Q = reinterpret_cast<cplx<T>*>(smem_raw);
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
-  const int team_in_wave = lane / M;
-  const int t = lane - team_in_wave * M;
-  const bool in_team = team_in_wave < G::per_wave;
-  const int team = wave * G::per_wave + team_in_wave;
-  const int nq = (nxc + 1) * NP;
-  // the team's exchange line of the row pass: in the plane's storage when
-  // one batch holds every row, else after it
-  cplx<T>* E = Q + (G::rows_in_place ? 0 : nq) + team * NP;
-  const cplx<T> zero = mk<T>(T(0), T(0));
-  cplx<T>* w = work + b * band_stride + (int64_t)z * nst;
-
-  // per-lane tables, the same for every row of the plane: twiddles, and the
-  // Q offsets of this lane's row slots x = t + M s (lanes t < M, kept s),
-  // which are both the backward inputs and the forward outputs
-  TeamTwiddles<T, N> twr;
-  twr.load(t, tw);
-  int cq[L];
-#pragma unroll
-  for (int s = 0; s < L; ++s) {
-    const int c = (t < M && ((KEEP >> s) & 1u)) ? colmap[t + M * s] : -1;
-    cq[s] = (c < 0 ? nxc : c) * NP;
-  }
-
-  // the zero column (ordered before the row pass by the barrier after the
-  // column pass, which does not touch it)
-  for (int i = tid; i < NP; i += kPlaneTeamThreads) Q[nxc * NP + i] = zero;
-
-  // backward y-FFT of every active column, its inputs read straight from the
-  // stick buffer (colpos: the stick at (c, y), or -1), in place in LDS: the
-  // column is the team's exchange line
-  if (in_team) {
-    for (int c = team; c < nxc; c += G::plane_teams) {
-      cplx<T>* col = Q + c * NP;
-      const int* pos = colpos + c * N;
-      cplx<T> bb[L], a[M];
-      if (t < M) {
-        // every position first, then every stick load (from element 0 where
-        // the slot holds no stick, replaced by zero): two memory round trips
-        // per column instead of two per slot
-        int st[L];
-#pragma unroll
-        for (int s = 0; s < L; ++s) st[s] = ((KEEP >> s) & 1u) ? pos[t + M * s] : -1;
-#pragma unroll
-        for (int s = 0; s < L; ++s) {
-          bb[s] = zero;
-          if ((KEEP >> s) & 1u) {
-            const cplx<T> v = w[st[s] >= 0 ? st[s] : 0];
-            bb[s] = st[s] >= 0 ? v : zero;
-          }
-        }
-      }
-      dif_front<T, N, +1>(t, col, twr, bb);
-      wave_lds_sync();
-      dif_back<T, N, +1>(t, col, a);
-      wave_lds_sync();
-      if (t < L) {
-#pragma unroll
-        for (int k = 0; k < M; ++k) col[t + L * k] = a[k];
-      }
-    }
-  }
-  __syncthreads();
-
-  // rows, RB per team and batch: backward x-FFT (inputs only at active
-  // columns), V, forward x-FFT (outputs only at active columns)
-  const T* vz = V + (int64_t)z * N * N;
-  for (int y0 = 0; y0 < N; y0 += RB * G::plane_teams) {
-    cplx<T> rows[RB][L];
-#pragma unroll
-    for (int r = 0; r < RB; ++r) {
-      const int y = y0 + team + r * G::plane_teams;
-      if (in_team && y < N && t < M) {
-#pragma unroll
-        for (int s = 0; s < L; ++s) rows[r][s] = ((KEEP >> s) & 1u) ? Q[cq[s] + y] : zero;
-      }
-    }
-    __syncthreads();
-    if (in_team) {
-#pragma unroll
-      for (int r = 0; r < RB; ++r) {
-        const int y = y0 + team + r * G::plane_teams;
-        if (y < N) {
-          // V(r) at this lane's backward outputs x = t + L k, fetched first
-          T vv[M];
-#pragma unroll
-          for (int k = 0; k < M; ++k) vv[k] = t < L ? vz[y * N + t + L * k] : T(0);
-          cplx<T> a[M];
-          // consecutive rows reuse the line: a DIF after a DIT writes only
-          // the slots the same lane read last
-          dif_front<T, N, +1>(t, E, twr, rows[r]);
-          wave_lds_sync();
-          dif_back<T, N, +1>(t, E, a);
-          if (t < L) {
-#pragma unroll
-            for (int k = 0; k < M; ++k) a[k] = cscale(a[k], vv[k]);
-          }
-          dit_front<T, N, -1>(t, E, twr, a);
-          wave_lds_sync();
-          dit_back<T, N, -1>(t, E, rows[r]);
-        }
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < RB; ++r) {
-      const int y = y0 + team + r * G::plane_teams;
-      if (in_team && y < N && t < M) {
-#pragma unroll
-        for (int s = 0; s < L; ++s)
-          if ((KEEP >> s) & 1u) Q[cq[s] + y] = rows[r][s];
-      }
-    }
-    __syncthreads();
-  }
-
-  // forward y-FFT of every active column, in place; only the kept y slots,
-  // which hold every stick, are computed, and the sticks among them go
-  // straight to the stick buffer
-  if (in_team) {
-    for (int c = team; c < nxc; c += G::plane_teams) {
-      cplx<T>* col = Q + c * NP;
-      const int* pos = colpos + c * N;
-      cplx<T> a[M], bb[L];
-      // the stick positions are fetched before the transform, so that the
-      // stores below wait for nothing
-      int st[L];
-#pragma unroll
-      for (int k = 0; k < L; ++k) st[k] = ((KEEP >> k) & 1u) ? pos[t + M * k] : -1;
-      if (t < L) {
-#pragma unroll
-        for (int s = 0; s < M; ++s) a[s] = col[t + L * s];
-      }
-      wave_lds_sync();
-      dit_front<T, N, -1>(t, col, twr, a);
-      wave_lds_sync();
-      dit_back<T, N, -1>(t, col, bb);
-      if (t < M) {
-        // every position is consumed before the first store: one wait for
-        // the loads above, none between the stores (stores count in vmcnt)
-#pragma unroll
-        for (int k = 0; k < L; ++k)
-          if ((KEEP >> k) & 1u) asm volatile("" ::"v"(st[k]));
-#pragma unroll
-        for (int k = 0; k < L; ++k)
-          if (((KEEP >> k) & 1u) && st[k] >= 0) w[st[k]] = bb[k];
-      }
-    }
-  }
-}
-
-// at least three waves per SIMD: the FP64 plane's LDS admits three workgroups
-// per CU, and its registers are held to that
-template <typename T, int N, bool PRUNE>
-__global__ __launch_bounds__(kPlaneTeamThreads, 3) void k_planes_team(
-    cplx<T>* __restrict__ work, int64_t band_stride, int nst,
-    const int* __restrict__ colpos, const int* __restrict__ colmap, int nxc,
-    const T* __restrict__ V, const cplx<T>* __restrict__ tw) {
-  planes_team_body<T, N, PRUNE>(blockIdx.x, blockIdx.y, work, band_stride, nst, colpos,
-                                colmap, nxc, V, tw);
-}
-
-// Slots of the team FFT of length n that hold any active x column or stick y
-// (bit s: positions t + M s, t < M); 0 when n has no team FFT.
-unsigned team_slot_mask(int n, const std::vector<int>& xs, const std::vector<int>& ys) {
+// Slots of the team FFT of length n that hold any of the positions (bit s:
+// positions t + M s, t < M); 0 when n has no team FFT.
+unsigned team_slot_mask(int n, const std::vector<int>& positions) {
   const int l = team_L(n);
   if (l <= 0) return 0u;
   const int m = n / l;
   unsigned mask = 0u;
-  for (int x : xs) mask |= 1u << (x / m);
-  for (int y : ys) mask |= 1u << (y / m);
+  for (int p : positions) mask |= 1u << (p / m);
   return mask;
 }
 
@@ -667,8 +445,6 @@ __global__ __launch_bounds__(kTeamThreads) void k_sticks_forward_team(
 // problem from that prefix, then runs the same register team FFT body as the
 // one-problem kernels for its grid length, chosen at run time among
 // QEPW_GROUP_SIZES.
-#define QEPW_GROUP_SIZES(X) X(36) X(48) X(54) X(60) X(64) X(72) X(80) X(96)
-constexpr int kMaxFftGroup = 24;
 
 template <typename T> struct StickGroupArgs {
   int count;
@@ -688,28 +464,6 @@ template <typename T> struct StickGroupArgs {
   int64_t ldout[kMaxFftGroup];
   T inv_n[kMaxFftGroup];
 };
-
-template <typename T> struct PlaneGroupArgs {
-  int count;
-  int start[kMaxFftGroup + 1];
-  int n[kMaxFftGroup];             // plane side (n1 = n2)
-  int n3[kMaxFftGroup];
-  int prune[kMaxFftGroup];
-  int nst[kMaxFftGroup];
-  int nxc[kMaxFftGroup];
-  cplx<T>* work[kMaxFftGroup];
-  int64_t bstride[kMaxFftGroup];
-  const int* colpos[kMaxFftGroup];
-  const int* colmap[kMaxFftGroup];
-  const T* V[kMaxFftGroup];
-  const cplx<T>* tw[kMaxFftGroup];
-};
-
-__device__ __forceinline__ int group_of(const int* start, int count, int bx) {
-  int p = 0;
-  while (p + 1 < count && start[p + 1] <= bx) ++p;
-  return p;
-}
 
 template <typename T, bool FORWARD>
 __global__ __launch_bounds__(kTeamThreads) void k_sticks_group(const StickGroupArgs<T> g) {
@@ -734,30 +488,8 @@ __global__ __launch_bounds__(kTeamThreads) void k_sticks_group(const StickGroupA
   }
 }
 
-template <typename T>
-__global__ __launch_bounds__(kPlaneTeamThreads, 3) void k_planes_group(const PlaneGroupArgs<T> g) {
-  const int p = group_of(g.start, g.count, blockIdx.x);
-  const int l = blockIdx.x - g.start[p];
-  const int z = l % g.n3[p];
-  const int64_t b = l / g.n3[p];
-  switch (g.n[p]) {
-#define QEPW_PLANE_CASE(NN)                                                                     \
-  case NN:                                                                                      \
-    if (g.prune[p])                                                                             \
-      planes_team_body<T, NN, true>(z, b, g.work[p], g.bstride[p], g.nst[p], g.colpos[p],       \
-                                    g.colmap[p], g.nxc[p], g.V[p], g.tw[p]);                    \
-    else                                                                                        \
-      planes_team_body<T, NN, false>(z, b, g.work[p], g.bstride[p], g.nst[p], g.colpos[p],      \
-                                     g.colmap[p], g.nxc[p], g.V[p], g.tw[p]);                   \
-    break;
-    QEPW_GROUP_SIZES(QEPW_PLANE_CASE)
-#undef QEPW_PLANE_CASE
-    default: break;
-  }
-}
-
-// Square plane sizes with an instantiated fast kernel.
-#define QEPW_TEAM_SIZES(X) \
+// z lengths and density plane sides with a team kernel.
+#define QEPW_LINE_SIZES(X) \
   X(16) X(18) X(20) X(24) X(25) X(27) X(30) X(32) X(36) X(40) X(45) X(48) X(50) X(54) \
   X(60) X(64) X(72) X(75) X(80) X(81) X(90) X(96) X(100) X(108) X(120)
 
@@ -765,81 +497,21 @@ __global__ __launch_bounds__(kPlaneTeamThreads, 3) void k_planes_group(const Pla
 static int team_teams(int n) {
   int teams = 0;
 #define QEPW_TEAMS_N(NN) if (n == NN) teams = TeamGeom<NN>::teams;
-  QEPW_TEAM_SIZES(QEPW_TEAMS_N)
+  QEPW_LINE_SIZES(QEPW_TEAMS_N)
 #undef QEPW_TEAMS_N
   return teams;
-}
-
-// Whether the pruned plane kernel (only the first two and last two slots
-// occupied) serves a plan whose occupied slots are ``mask``.
-static bool team_prunable(int n, unsigned mask) {
-  bool ok = false;
-#define QEPW_PRUNE_N(NN) if (n == NN) ok = (mask & ~TeamGeom<NN>::pruned) == 0u;
-  QEPW_TEAM_SIZES(QEPW_PRUNE_N)
-#undef QEPW_PRUNE_N
-  return ok;
-}
-
-// LDS of the plane kernel (k_planes_team / k_planes_group): the active
-// columns and the zero column, holding an exchange line per team when the
-// row pass exchanges in place, else followed by them.
-template <typename T>
-static size_t plane_team_lds_bytes(int n, int nxc) {
-  size_t teams = 0;
-  bool in_place = false;
-#define QEPW_TEAMS_OF(NN)                  \
-  if (n == NN) {                           \
-    teams = TeamGeom<NN>::plane_teams;     \
-    in_place = TeamGeom<NN>::rows_in_place; \
-  }
-  QEPW_TEAM_SIZES(QEPW_TEAMS_OF)
-#undef QEPW_TEAMS_OF
-  if (teams == 0) return 0;
-  const size_t lines = in_place ? std::max((size_t)nxc + 1, teams) : (size_t)nxc + 1 + teams;
-  return lines * (size_t)(n + plane_pad<T>()) * sizeof(cplx<T>);
 }
 
 template <typename T>
 static size_t team_lds_bytes(int n, int nxc) {
   size_t teams = 0;
 #define QEPW_TEAMS_OF(NN) if (n == NN) teams = TeamGeom<NN>::teams;
-  QEPW_TEAM_SIZES(QEPW_TEAMS_OF)
+  QEPW_LINE_SIZES(QEPW_TEAMS_OF)
 #undef QEPW_TEAMS_OF
   // no team kernel for this length: the generic kernels run
   if (teams == 0) return 0;
   // active columns, the zero column of k_planes_team, one scratch line per team
   return ((size_t)nxc + 1 + teams) * (size_t)(n + 1) * sizeof(cplx<T>);
-}
-
-// Launches the fast plane kernel if one exists for this plane; returns false
-// otherwise (the generic kernel is used).
-template <typename T>
-static bool launch_planes_team(const Plan& p, const StickTables& st, cplx<T>* work,
-                               int64_t bstride, const T* V, const cplx<T>* tw, int nb,
-                               hipStream_t stream) {
-  if (p.n1 != p.n2 || !st.d_colpos || !st.d_colmap) return false;
-  const size_t lds = plane_team_lds_bytes<T>(p.n1, st.nxcols);
-  if (lds == 0 || lds > (size_t)kMaxLdsBytes) return false;
-  const dim3 grid(p.n3, nb);
-#define QEPW_LAUNCH_TEAM_K(NN, PR)                                                           \
-  do {                                                                                       \
-    hipFuncSetAttribute(reinterpret_cast<const void*>(&k_planes_team<T, NN, PR>),           \
-                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);               \
-    hipLaunchKernelGGL((k_planes_team<T, NN, PR>), grid, dim3(kPlaneTeamThreads), lds, stream, \
-                       work, bstride, st.nst, st.d_colpos, st.d_colmap, st.nxcols, V, tw);  \
-  } while (0)
-#define QEPW_LAUNCH_TEAM(NN)                                                                 \
-  if (p.n1 == NN) {                                                                          \
-    if ((st.slot_mask & ~TeamGeom<NN>::pruned) == 0u)                                        \
-      QEPW_LAUNCH_TEAM_K(NN, true);                                                          \
-    else                                                                                     \
-      QEPW_LAUNCH_TEAM_K(NN, false);                                                         \
-    return true;                                                                             \
-  }
-  QEPW_TEAM_SIZES(QEPW_LAUNCH_TEAM)
-#undef QEPW_LAUNCH_TEAM
-#undef QEPW_LAUNCH_TEAM_K
-  return false;
 }
 
 // Launches the team z-stage kernel for n3 if one exists; false otherwise.
@@ -862,7 +534,7 @@ static bool launch_sticks_team(bool inverse, const Plan& p, const StickTables& s
                          st.d_off, st.d_gpos, tw, inv_n);                                    \
     return true;                                                                             \
   }
-  QEPW_TEAM_SIZES(QEPW_LAUNCH_STICKS)
+  QEPW_LINE_SIZES(QEPW_LAUNCH_STICKS)
 #undef QEPW_LAUNCH_STICKS
   return false;
 }
@@ -892,22 +564,11 @@ int stick_group_for(int n3, int nst) {
 
 template <typename T>
 static void set_lds_attrs(size_t stick_bytes, size_t plane_bytes) {
-  hipFuncSetAttribute(reinterpret_cast<const void*>(&k_sticks_inverse<T>),
-                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)stick_bytes);
-  hipFuncSetAttribute(reinterpret_cast<const void*>(&k_sticks_forward<T>),
-                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)stick_bytes);
+  allow_lds(reinterpret_cast<const void*>(&k_sticks_inverse<T>), stick_bytes);
+  allow_lds(reinterpret_cast<const void*>(&k_sticks_forward<T>), stick_bytes);
   if (plane_bytes == 0 || plane_bytes > (size_t)kMaxLdsBytes) return;
-  hipFuncSetAttribute(reinterpret_cast<const void*>(&k_planes<T, kPlaneApply>),
-                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)plane_bytes);
-  hipFuncSetAttribute(reinterpret_cast<const void*>(&k_planes<T, kPlaneReal>),
-                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)plane_bytes);
-}
-
-template <typename T>
-static bool team_available(const Plan& p, const StickTables& st) {
-  if (p.n1 != p.n2 || !st.d_colpos || !st.d_colmap) return false;
-  const size_t lds = plane_team_lds_bytes<T>(p.n1, st.nxcols);
-  return lds > 0 && lds <= (size_t)kMaxLdsBytes;
+  allow_lds(reinterpret_cast<const void*>(&k_planes<T, kPlaneApply>), plane_bytes);
+  allow_lds(reinterpret_cast<const void*>(&k_planes<T, kPlaneReal>), plane_bytes);
 }
 
 // How the xy-plane stage of a plan runs.
@@ -924,7 +585,7 @@ static bool generic_plane_fits(const Plan& p) {
 template <typename T>
 static int plane_path(const Plan& p, const StickTables& st) {
   if (st.group * p.n3 > lds_fft_capacity(p.line[2], kStickThreads, kStickPts)) return kPathNone;
-  if (team_available<T>(p, st)) return kPathTeam;
+  if ((sizeof(T) == 8 ? st.plane64 : st.plane32).waves > 0) return kPathTeam;
   if (generic_plane_fits<T>(p)) return kPathGeneric;
   if (split_available<T>(p, st)) return kPathSplit;
   return kPathNone;
@@ -978,8 +639,8 @@ int apply_local_t(const Plan& p, const void* vectors, int64_t ldv, int nb,
       launch_split<T>(false, p, st, work, bstride, tbuf, static_cast<const T*>(potential),
                       nullptr, nbc, stream);
     else if (path != kPathTeam ||
-             !launch_planes_team<T>(p, st, work, bstride, static_cast<const T*>(potential),
-                                    twiddles<T>(p, 0), nbc, stream))
+             !launch_plane_stage<T>(p, st, work, bstride, static_cast<const T*>(potential),
+                                    nbc, stream))
       hipLaunchKernelGGL((k_planes<T, kPlaneApply>), gp, dim3(kPlaneThreads), plane_lds,
                          stream, work, bstride, st.nst, st.d_plane, st.d_xcols, st.nxcols,
                          static_cast<const T*>(potential), static_cast<T*>(nullptr), p.n1,
@@ -1021,7 +682,7 @@ template <typename T>
 static bool group_eligible(const Plan& p, int nb, size_t ws_bytes) {
   const StickTables& st = p.sphere;
   if (!(p.n1 == p.n2 && group_size(p.n1) && group_size(p.n3))) return false;
-  if (plane_path<T>(p, st) != kPathTeam || !team_available<T>(p, st)) return false;
+  if (plane_path<T>(p, st) != kPathTeam) return false;
   return (size_t)nb * band_bytes_t<T>(p, st) <= ws_bytes && nb <= 65535;
 }
 
@@ -1047,10 +708,12 @@ int apply_local_group_t(int count, const Plan* const* plans, const void* const* 
   for (size_t g0 = 0; g0 < members.size(); g0 += kMaxFftGroup) {
     const int m = (int)std::min<size_t>(kMaxFftGroup, members.size() - g0);
     StickGroupArgs<T> sa{};
-    PlaneGroupArgs<T> pa{};
-    sa.count = pa.count = m;
-    size_t stick_lds = 0, plane_lds = 0;
-    int64_t stotal = 0, ptotal = 0;
+    sa.count = m;
+    size_t stick_lds = 0;
+    int64_t stotal = 0;
+    const Plan* gplan[kMaxFftGroup];
+    const T* gV[kMaxFftGroup];
+    int gnb[kMaxFftGroup];
     for (int j = 0; j < m; ++j) {
       const int i = members[g0 + j];
       const Plan& p = *plans[i];
@@ -1073,34 +736,18 @@ int apply_local_group_t(int count, const Plan* const* plans, const void* const* 
       sa.inv_n[j] = T(1.0 / ((double)p.n1 * p.n2 * p.n3));
       stotal += (int64_t)sa.groups[j] * nb[i];
       stick_lds = std::max(stick_lds, (size_t)teams_z * (p.n3 + 1) * sizeof(cplx<T>));
-      pa.start[j] = (int)ptotal;
-      pa.n[j] = p.n1;
-      pa.n3[j] = p.n3;
-      pa.prune[j] = team_prunable(p.n1, st.slot_mask) ? 1 : 0;
-      pa.nst[j] = st.nst;
-      pa.nxc[j] = st.nxcols;
-      pa.work[j] = sa.work[j];
-      pa.bstride[j] = sa.bstride[j];
-      pa.colpos[j] = st.d_colpos;
-      pa.colmap[j] = st.d_colmap;
-      pa.V[j] = static_cast<const T*>(potentials[i]);
-      pa.tw[j] = twiddles<T>(p, 0);
-      ptotal += (int64_t)p.n3 * nb[i];
-      plane_lds = std::max(plane_lds, plane_team_lds_bytes<T>(p.n1, st.nxcols));
+      gplan[j] = &p;
+      gV[j] = static_cast<const T*>(potentials[i]);
+      gnb[j] = nb[i];
     }
     sa.start[m] = (int)stotal;
-    pa.start[m] = (int)ptotal;
-    if (stotal > 0x7fffffff || ptotal > 0x7fffffff) return QEPW_ERR_UNSUPPORTED;
-    hipFuncSetAttribute(reinterpret_cast<const void*>(&k_sticks_group<T, false>),
-                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)stick_lds);
-    hipFuncSetAttribute(reinterpret_cast<const void*>(&k_sticks_group<T, true>),
-                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)stick_lds);
-    hipFuncSetAttribute(reinterpret_cast<const void*>(&k_planes_group<T>),
-                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)plane_lds);
+    if (stotal > 0x7fffffff) return QEPW_ERR_UNSUPPORTED;
+    allow_lds(reinterpret_cast<const void*>(&k_sticks_group<T, false>), stick_lds);
+    allow_lds(reinterpret_cast<const void*>(&k_sticks_group<T, true>), stick_lds);
     hipLaunchKernelGGL((k_sticks_group<T, false>), dim3((unsigned)stotal), dim3(kTeamThreads),
                        stick_lds, stream, sa);
-    hipLaunchKernelGGL(k_planes_group<T>, dim3((unsigned)ptotal), dim3(kPlaneTeamThreads),
-                       plane_lds, stream, pa);
+    const int rc = launch_plane_group<T>(m, gplan, sa.work, sa.bstride, gV, gnb, stream);
+    if (rc != QEPW_OK) return rc;
     hipLaunchKernelGGL((k_sticks_group<T, true>), dim3((unsigned)stotal), dim3(kTeamThreads),
                        stick_lds, stream, sa);
   }
@@ -1418,17 +1065,14 @@ int accumulate_density_t(const Plan& p, const void* vectors, int64_t ldv, int nb
   const size_t plane_lds = np * sizeof(cplx<T>);
   set_lds_attrs<T>(stick_lds, 0);
   if (!team && !split)
-    hipFuncSetAttribute(reinterpret_cast<const void*>(&k_density_plane<T>),
-                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)plane_lds);
+    allow_lds(reinterpret_cast<const void*>(&k_density_plane<T>), plane_lds);
   const int gc = split ? split_group<T>(p.line[1]) : 0;
   const int gr = split ? split_group<T>(p.line[0]) : 0;
   const size_t lc = (size_t)gc * p.n2 * sizeof(cplx<T>);
   const size_t lr = (size_t)gr * p.n1 * sizeof(cplx<T>);
   if (split) {
-    hipFuncSetAttribute(reinterpret_cast<const void*>(&k_split_cols_inverse<T>),
-                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lc);
-    hipFuncSetAttribute(reinterpret_cast<const void*>(&k_split_rows_density<T>),
-                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lr);
+    allow_lds(reinterpret_cast<const void*>(&k_split_cols_inverse<T>), lc);
+    allow_lds(reinterpret_cast<const void*>(&k_split_rows_density<T>), lr);
   }
   const int64_t bstride = (int64_t)p.n3 * st.nst;
   if (nb <= 0) {
@@ -1452,21 +1096,20 @@ int accumulate_density_t(const Plan& p, const void* vectors, int64_t ldv, int nb
     if (team) {
 #define QEPW_LAUNCH_DENSITY_K(NN, PR)                                                        \
   do {                                                                                       \
-    hipFuncSetAttribute(reinterpret_cast<const void*>(&k_density_team<T, NN, PR>),          \
-                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)team_lds);          \
+    allow_lds(reinterpret_cast<const void*>(&k_density_team<T, NN, PR>), team_lds);          \
     hipLaunchKernelGGL((k_density_team<T, NN, PR>), grid, dim3(kTeamThreads), team_lds,     \
                        stream, work, bstride, st.nst, st.d_colpos, st.d_colmap, st.nxcols,  \
                        nbc, per, weights + b0, partial, acc, twiddles<T>(p, 0));             \
   } while (0)
 #define QEPW_LAUNCH_DENSITY(NN)                                                              \
   if (!launched && p.n1 == NN) {                                                             \
-    if ((st.slot_mask & ~TeamGeom<NN>::pruned) == 0u)                                        \
+    if (((st.xmask | st.ymask) & ~TeamGeom<NN>::pruned) == 0u)                                        \
       QEPW_LAUNCH_DENSITY_K(NN, true);                                                       \
     else                                                                                     \
       QEPW_LAUNCH_DENSITY_K(NN, false);                                                      \
     launched = true;                                                                         \
   }
-      QEPW_TEAM_SIZES(QEPW_LAUNCH_DENSITY)
+      QEPW_LINE_SIZES(QEPW_LAUNCH_DENSITY)
 #undef QEPW_LAUNCH_DENSITY
 #undef QEPW_LAUNCH_DENSITY_K
     }

@@ -35,11 +35,11 @@ template <typename T> struct SmallDft<T, 3> {
   static __device__ __forceinline__ void run(cplx<T> (&v)[3], int sign) {
     const T h = T(0.866025403784438646763723170752936183);  // sqrt(3)/2
     cplx<T> t1 = cadd(v[1], v[2]);
-    cplx<T> t2 = csub(v[0], cscale(t1, T(0.5)));
-    cplx<T> t3 = cmuli(cscale(csub(v[1], v[2]), h), sign);
+    cplx<T> t2 = caxpy(t1, T(-0.5), v[0]);
+    cplx<T> t3 = cmuli(csub(v[1], v[2]), sign);
     v[0] = cadd(v[0], t1);
-    v[1] = cadd(t2, t3);
-    v[2] = csub(t2, t3);
+    v[1] = caxpy(t3, h, t2);
+    v[2] = caxmy(t3, h, t2);
   }
 };
 
@@ -62,10 +62,10 @@ template <typename T> struct SmallDft<T, 5> {
     const T s2 = T(0.587785252292473129168705954639072769);   // sin(4pi/5)
     cplx<T> a1 = cadd(v[1], v[4]), b1 = csub(v[1], v[4]);
     cplx<T> a2 = cadd(v[2], v[3]), b2 = csub(v[2], v[3]);
-    cplx<T> r1 = cadd(v[0], cadd(cscale(a1, c1), cscale(a2, c2)));
-    cplx<T> r2 = cadd(v[0], cadd(cscale(a1, c2), cscale(a2, c1)));
-    cplx<T> i1 = cmuli(cadd(cscale(b1, s1), cscale(b2, s2)), sign);
-    cplx<T> i2 = cmuli(csub(cscale(b1, s2), cscale(b2, s1)), sign);
+    cplx<T> r1 = caxpy(a2, c2, caxpy(a1, c1, v[0]));
+    cplx<T> r2 = caxpy(a2, c1, caxpy(a1, c2, v[0]));
+    cplx<T> i1 = cmuli(caxpy(b2, s2, cscale(b1, s1)), sign);
+    cplx<T> i2 = cmuli(caxmy(b2, s1, cscale(b1, s2)), sign);
     v[0] = cadd(v[0], cadd(a1, a2));
     v[1] = cadd(r1, i1);
     v[4] = csub(r1, i1);

@@ -11,6 +11,24 @@ namespace qepw {
 
 constexpr int kMaxLdsBytes = 160 * 1024;
 
+// Raises a kernel's dynamic LDS limit where a launch needs more than the 64 KB
+// every kernel may use (the call costs a microsecond of a launch).
+inline void allow_lds(const void* kernel, size_t bytes) {
+  if (bytes > 64 * 1024)
+    (void)hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+}
+
+// Grouped launches (qepw_apply_local_group): up to kMaxFftGroup problems whose
+// plane side and z length are among QEPW_GROUP_SIZES.
+#define QEPW_GROUP_SIZES(X) X(36) X(48) X(54) X(60) X(64) X(72) X(80) X(96)
+constexpr int kMaxFftGroup = 24;
+
+__device__ __forceinline__ int group_of(const int* start, int count, int bx) {
+  int p = 0;
+  while (p + 1 < count && start[p + 1] <= bx) ++p;
+  return p;
+}
+
 // qepw_fft.hip
 int stick_group_for(int n3, int nst);
 size_t apply_local_band_bytes(const Plan& p, int precision);
@@ -26,10 +44,28 @@ size_t density_workspace_bytes(const Plan& p, int precision, int nb);
 int accumulate_density(const Plan& p, int precision, const void* vectors, int64_t ldv, int nb,
                        const double* weights, double scale, double* out, void* workspace,
                        size_t ws_bytes, hipStream_t stream);
-unsigned team_slot_mask(int n, const std::vector<int>& xs, const std::vector<int>& ys);
+unsigned team_slot_mask(int n, const std::vector<int>& positions);
 size_t inverse_real_bytes(const Plan& p);
 int inverse_real(const Plan& p, const void* grid_g, void* out_real, void* workspace,
                  size_t ws_bytes, hipStream_t stream);
+
+// qepw_plane_c128.hip, qepw_plane_c64.hip (the xy-plane stage, qepw_plane.h)
+// Whether the lines of length n load their twiddles instead of holding them:
+// held, FP64 lines spill or halve the waves a CU runs (96^2, 110 bands: 46 of
+// 168 registers' worth spilled); nine twiddles of lines up to 72 still fit (72^2,
+// 128 bands: 280 us held, 292 us loaded; 60^2: 216 and 209 us).
+constexpr bool plane_lane_table(int n, bool fp64) {
+  const int m = team_L(n) > 0 ? n / team_L(n) : 0;
+  return fp64 ? !(m == 9 && n <= 72) : m >= 15;
+}
+template <typename T> PlaneChoice plane_choice(const Plan& p, const StickTables& st);
+template <typename T>
+bool launch_plane_stage(const Plan& p, const StickTables& st, cplx<T>* work, int64_t bstride,
+                        const T* V, int nb, hipStream_t stream);
+template <typename T>
+int launch_plane_group(int count, const Plan* const* plans, cplx<T>* const* work,
+                       const int64_t* bstride, const T* const* V, const int* nb,
+                       hipStream_t stream);
 
 // qepw_gemm.hip
 size_t gemm_workspace_bytes(int precision, int op_a, int64_t m, int64_t n, int64_t k);

@@ -18,6 +18,15 @@
 
 namespace qepw {
 
+// How the xy planes of a plan run in one precision (plane_choice,
+// qepw_plane.h): waves of the workgroup (0: the team stage does not serve it),
+// its kernel and its LDS.
+struct PlaneChoice {
+  int waves = 0;
+  bool square = false, prune = false;
+  size_t lds = 0;
+};
+
 struct StickTables {
   int nst = 0;          // active sticks
   int nxcols = 0;       // distinct x among active sticks
@@ -33,7 +42,9 @@ struct StickTables {
   int* d_colstart = nullptr;  // nxcols+1: first stick of each active column (sticks
                               // are sorted by x, then y)
   int* d_colpos = nullptr;  // nxcols * n2: stick at (column c, y), or -1
-  unsigned slot_mask = 0;   // team-FFT input slots holding an active x or stick y
+  unsigned xmask = 0;       // team-FFT input slots holding an active x
+  unsigned ymask = 0;       // ... a stick's y
+  PlaneChoice plane64, plane32;
 };
 
 struct Plan {
@@ -44,6 +55,10 @@ struct Plan {
   StickTables full;     // every stick of the grid (prepare_potential)
   double2* d_tw64[3] = {nullptr, nullptr, nullptr};
   float2* d_tw32[3] = {nullptr, nullptr, nullptr};
+  // w_n^(t k) of the x and y lines in lane order (PlaneTwiddles, qepw_plane.h)
+  // where plane_lane_table(n); null else
+  double2* d_ltw64[2] = {nullptr, nullptr};
+  float2* d_ltw32[2] = {nullptr, nullptr};
   int* d_perm = nullptr;
   std::vector<int> h_perm;
   int device = 0;

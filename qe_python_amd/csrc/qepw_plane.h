@@ -1,0 +1,603 @@
+// The xy-plane stage on register "team" FFTs (qepw_regfft.h): one workgroup
+// per (z-plane, band), any pair of team lengths n1 (x) and n2 (y).
+//
+// LDS holds only the nxc occupied x columns of the plane, Q[c * NP2 + y], plus
+// one all-zero column:
+//   columns : backward y-FFT of every occupied column, its sticks read
+//             straight from the stick buffer;
+//   rows    : backward x-FFT, times V(r), forward x-FFT, in registers;
+//   columns : forward y-FFT, the sticks written straight back.
+//
+// The backward transforms are decimation-in-frequency team FFTs, whose input
+// slot s of lane t is position t + M s: the sphere's x and y extents leave
+// whole slots empty for every lane (the extents of a sphere reach about a
+// quarter of the grid to either side), so with KEEP naming the occupied slots
+// the empty inputs are literal zeros that the compiler folds away (these files
+// are built with -fno-signed-zeros for that), and the loads of them disappear.
+// The forward transforms are decimation-in-time team FFTs, whose output slot s
+// of lane t is again position t + M s: only the kept slots are computed and
+// stored.  The row pass chains backward x-FFT (DIF), V(r) multiply and forward
+// x-FFT (DIT) in registers -- the DIT consumes the DIF's output order -- at two
+// team exchanges per row.
+//
+// LDS holds the plane and nothing else, so that more workgroups share a CU
+// (FP64 at the 72^3 workload: 42 KB, three per CU): a column FFT exchanges
+// through its own column (its values are in registers by then), and the row
+// pass reads all its rows into registers, after which the plane's storage is
+// free and each team exchanges through a line of it; the outputs wait in
+// registers until every team is done, then go back to their rows.
+#pragma once
+
+#include <algorithm>
+
+#include "qepw_internal.h"
+#include "qepw_regfft.h"
+
+namespace qepw {
+
+// Team geometry of a line length.
+template <int N> struct PlaneLine {
+  static constexpr int L = team_L(N);
+  static constexpr int M = N / L;
+  static constexpr int per_wave = 64 / M;
+  static constexpr unsigned all = (1u << L) - 1u;
+  // input slots of the pruned kernels: those within a quarter of the line of
+  // either end
+  static constexpr int kept = ((N + 3) / 4 + M - 1) / M;
+  static constexpr bool prunes = 2 * kept < L;
+  static constexpr unsigned pruned =
+      prunes ? (((1u << kept) - 1u) | (((1u << kept) - 1u) << (L - kept))) : all;
+};
+
+// The twiddles between the two halves of a team FFT, w_N^(t k) for lane t.
+// Held in registers (TeamTwiddles), or loaded where they are used from a table
+// in the order of the lanes ([k M + t] for the DIF half's k < L, N + [k L + t]
+// for the DIT half's k < M) that stays in the L1 (plane_lane_table).
+template <typename T, int N, bool LOAD = plane_lane_table(N, sizeof(T) == 8)>
+struct PlaneTwiddles {
+  TeamTwiddles<T, N> reg;
+  __device__ __forceinline__ void load(int t, const cplx<T>* __restrict__ tw) { reg.load(t, tw); }
+  __device__ __forceinline__ void fresh() {}
+  __device__ __forceinline__ cplx<T> dif(int, int k) const { return reg.w[k]; }
+  __device__ __forceinline__ cplx<T> dit(int, int k) const { return reg.w[k]; }
+};
+template <typename T, int N> struct PlaneTwiddles<T, N, true> {
+  const cplx<T>* tab;
+  int zero;
+  __device__ __forceinline__ void load(int, const cplx<T>* __restrict__ tw) { tab = tw; }
+  // keeps the loads after this point after it (an offset, so that they stay
+  // global loads)
+  __device__ __forceinline__ void fresh() {
+    zero = 0;
+    asm volatile("" : "+s"(zero));
+  }
+  __device__ __forceinline__ cplx<T> dif(int t, int k) const {
+    return (tab + zero)[k * PlaneLine<N>::M + t];
+  }
+  __device__ __forceinline__ cplx<T> dit(int t, int k) const {
+    return (tab + zero)[N + k * PlaneLine<N>::L + t];
+  }
+};
+
+// Backward (DIF) and forward (DIT) team FFTs of one line through its LDS line
+// S, split as in qepw_regfft.h: b, slots t + M s of lanes t < M; a, slots
+// t + L k of lanes t < L.
+template <typename T, int N>
+__device__ __forceinline__ void plane_backward(int t, cplx<T>* S, PlaneTwiddles<T, N>& tw,
+                                               cplx<T> (&b)[PlaneLine<N>::L],
+                                               cplx<T> (&a)[PlaneLine<N>::M]) {
+  constexpr int L = PlaneLine<N>::L, M = PlaneLine<N>::M;
+  if (t < M) {
+    tw.fresh();
+    RegDft<T, L, +1>::run(b);
+#pragma unroll
+    for (int k = 1; k < L; ++k) b[k] = cmulc(b[k], tw.dif(t, k));
+#pragma unroll
+    for (int k = 0; k < L; ++k) S[k * M + t] = b[k];
+  }
+  wave_lds_sync();
+  if (t < L) {
+#pragma unroll
+    for (int j = 0; j < M; ++j) a[j] = S[t * M + j];
+    RegDft<T, M, +1>::run(a);
+  }
+}
+
+template <typename T, int N>
+__device__ __forceinline__ void plane_forward(int t, cplx<T>* S, PlaneTwiddles<T, N>& tw,
+                                              cplx<T> (&a)[PlaneLine<N>::M],
+                                              cplx<T> (&b)[PlaneLine<N>::L]) {
+  constexpr int L = PlaneLine<N>::L, M = PlaneLine<N>::M;
+  if (t < L) {
+    tw.fresh();
+    RegDft<T, M, -1>::run(a);
+#pragma unroll
+    for (int k = 1; k < M; ++k) a[k] = cmul(a[k], tw.dit(t, k));
+#pragma unroll
+    for (int k = 0; k < M; ++k) S[t * M + k] = a[k];
+  }
+  wave_lds_sync();
+  if (t < M) {
+#pragma unroll
+    for (int j = 0; j < L; ++j) b[j] = S[j * M + t];
+    RegDft<T, L, -1>::run(b);
+  }
+}
+
+// One problem's plane stage.
+template <typename T> struct PlaneArgs {
+  cplx<T>* work;        // stick buffers (band, z, stick)
+  int64_t bstride;
+  int nst, n1, n2, nxc;
+  const int* colpos;    // (nxc, n2): stick at (column c, y), or -1
+  const int* colmap;    // n1: rank of x among the occupied columns, or -1
+  const T* V;           // (n3, n2, n1)
+  const cplx<T>* tw1;
+  const cplx<T>* tw2;
+};
+
+template <int N> struct PlaneLane {
+  int t, team;
+  bool on;
+  __device__ __forceinline__ PlaneLane() {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int i = lane / PlaneLine<N>::M;
+    t = lane - i * PlaneLine<N>::M;
+    on = i < PlaneLine<N>::per_wave;
+    team = wave * PlaneLine<N>::per_wave + i;
+  }
+};
+
+// Backward y-FFT of every occupied column, in place in LDS: the column is the
+// team's exchange line.  Column nxc is zeroed: the row pass reads the
+// unoccupied x positions from it (and writes their discarded outputs to it).
+template <typename T, int N2, bool PRUNE>
+__device__ __forceinline__ void plane_cols_backward(const PlaneArgs<T>& g, const cplx<T>* w,
+                                                    cplx<T>* Q, int waves,
+                                                    PlaneTwiddles<T, N2>& tw) {
+  using G = PlaneLine<N2>;
+  constexpr int L = G::L, M = G::M, NP = N2 + 1;
+  constexpr unsigned KEEP = PRUNE ? G::pruned : G::all;
+  const PlaneLane<N2> ln;
+  const int t = ln.t;
+  const cplx<T> zero = mk<T>(T(0), T(0));
+  for (int i = threadIdx.x; i < NP; i += waves * 64) Q[g.nxc * NP + i] = zero;
+  if (!ln.on) return;
+  for (int c = ln.team; c < g.nxc; c += waves * G::per_wave) {
+    cplx<T>* col = Q + c * NP;
+    const int* pos = g.colpos + c * N2;
+    cplx<T> bb[L], a[M];
+    if (t < M) {
+      // every position first, then every stick load (from element 0 where
+      // the slot holds no stick, replaced by zero): two memory round trips
+      // per column instead of two per slot
+      int st[L];
+#pragma unroll
+      for (int s = 0; s < L; ++s) st[s] = ((KEEP >> s) & 1u) ? pos[t + M * s] : -1;
+#pragma unroll
+      for (int s = 0; s < L; ++s) {
+        bb[s] = zero;
+        if ((KEEP >> s) & 1u) {
+          const cplx<T> v = w[st[s] >= 0 ? st[s] : 0];
+          bb[s] = st[s] >= 0 ? v : zero;
+        }
+      }
+    }
+    plane_backward<T, N2>(t, col, tw, bb, a);
+    wave_lds_sync();
+    if (t < L) {
+#pragma unroll
+      for (int k = 0; k < M; ++k) col[t + L * k] = a[k];
+    }
+  }
+}
+
+// The LDS offsets of this lane's row slots x = t + M s (lanes t < M, kept s),
+// which are both the backward inputs and the forward outputs: its column's,
+// or the zero column's.  The same for every row of the plane.
+template <typename T, int N1, bool PRUNE>
+__device__ __forceinline__ void plane_row_slots(const PlaneArgs<T>& g, int np2,
+                                                int (&cq)[PlaneLine<N1>::L]) {
+  using G = PlaneLine<N1>;
+  constexpr unsigned KEEP = PRUNE ? G::pruned : G::all;
+  const PlaneLane<N1> ln;
+#pragma unroll
+  for (int s = 0; s < G::L; ++s) {
+    const int c =
+        (ln.on && ln.t < G::M && ((KEEP >> s) & 1u)) ? g.colmap[ln.t + G::M * s] : -1;
+    cq[s] = (c < 0 ? g.nxc : c) * np2;
+  }
+}
+
+// Rows, RB per team (RB teams >= n2): backward x-FFT (inputs only at occupied
+// columns), V, forward x-FFT (outputs only at occupied columns).  np2: the
+// LDS column stride.  Called by the whole workgroup (it synchronises).
+template <typename T, int N1, bool PRUNE, int RB>
+__device__ __forceinline__ void plane_rows(const PlaneArgs<T>& g, int z, cplx<T>* Q, int n2,
+                                           int np2, int waves, PlaneTwiddles<T, N1>& tw,
+                                           const int (&cq)[PlaneLine<N1>::L]) {
+  using G = PlaneLine<N1>;
+  constexpr int L = G::L, M = G::M, NP = N1 + 1;
+  constexpr unsigned KEEP = PRUNE ? G::pruned : G::all;
+  const PlaneLane<N1> ln;
+  const int t = ln.t, team = ln.team, teams = waves * G::per_wave;
+  const cplx<T> zero = mk<T>(T(0), T(0));
+  cplx<T>* E = Q + team * NP;
+  const T* vz = g.V + (int64_t)z * n2 * N1;
+  cplx<T> rows[RB][L];
+#pragma unroll
+  for (int r = 0; r < RB; ++r) {
+    const int y = team + r * teams;
+    if (ln.on && y < n2 && t < M) {
+#pragma unroll
+      for (int s = 0; s < L; ++s) rows[r][s] = ((KEEP >> s) & 1u) ? Q[cq[s] + y] : zero;
+    }
+  }
+  __syncthreads();
+  if (ln.on) {
+#pragma unroll
+    for (int r = 0; r < RB; ++r) {
+      const int y = team + r * teams;
+      if (y < n2) {
+        // V(r) at this lane's backward outputs x = t + L k, fetched first
+        T vv[M];
+#pragma unroll
+        for (int k = 0; k < M; ++k) vv[k] = t < L ? vz[y * N1 + t + L * k] : T(0);
+        cplx<T> a[M];
+        // consecutive rows reuse the line: a DIF after a DIT writes only
+        // the slots the same lane read last
+        plane_backward<T, N1>(t, E, tw, rows[r], a);
+        if (t < L) {
+#pragma unroll
+          for (int k = 0; k < M; ++k) a[k] = cscale(a[k], vv[k]);
+        }
+        plane_forward<T, N1>(t, E, tw, a, rows[r]);
+      }
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < RB; ++r) {
+    const int y = team + r * teams;
+    if (ln.on && y < n2 && t < M) {
+#pragma unroll
+      for (int s = 0; s < L; ++s)
+        if ((KEEP >> s) & 1u) Q[cq[s] + y] = rows[r][s];
+    }
+  }
+}
+
+// Forward y-FFT of every occupied column, in place; only the kept y slots,
+// which hold every stick, are computed, and the sticks among them go straight
+// to the stick buffer.
+template <typename T, int N2, bool PRUNE>
+__device__ __forceinline__ void plane_cols_forward(const PlaneArgs<T>& g, cplx<T>* w, cplx<T>* Q,
+                                                   int waves, PlaneTwiddles<T, N2>& tw) {
+  using G = PlaneLine<N2>;
+  constexpr int L = G::L, M = G::M, NP = N2 + 1;
+  constexpr unsigned KEEP = PRUNE ? G::pruned : G::all;
+  const PlaneLane<N2> ln;
+  if (!ln.on) return;
+  const int t = ln.t;
+  for (int c = ln.team; c < g.nxc; c += waves * G::per_wave) {
+    cplx<T>* col = Q + c * NP;
+    const int* pos = g.colpos + c * N2;
+    cplx<T> a[M], bb[L];
+    // the stick positions are fetched before the transform, so that the
+    // stores below wait for nothing
+    int st[L];
+#pragma unroll
+    for (int k = 0; k < L; ++k) st[k] = ((KEEP >> k) & 1u) ? pos[t + M * k] : -1;
+    if (t < L) {
+#pragma unroll
+      for (int s = 0; s < M; ++s) a[s] = col[t + L * s];
+    }
+    wave_lds_sync();
+    plane_forward<T, N2>(t, col, tw, a, bb);
+    if (t < M) {
+      // every position is consumed before the first store: one wait for
+      // the loads above, none between the stores (stores count in vmcnt)
+#pragma unroll
+      for (int k = 0; k < L; ++k)
+        if ((KEEP >> k) & 1u) asm volatile("" ::"v"(st[k]));
+#pragma unroll
+      for (int k = 0; k < L; ++k)
+        if (((KEEP >> k) & 1u) && st[k] >= 0) w[st[k]] = bb[k];
+    }
+  }
+}
+
+// Line lengths with a team FFT.
+#define QEPW_TEAM_SIZES(X) \
+  X(16) X(18) X(20) X(24) X(25) X(27) X(30) X(32) X(36) X(40) X(45) X(48) X(50) X(54) \
+  X(60) X(64) X(72) X(75) X(80) X(81) X(90) X(96) X(100) X(108) X(120) X(128) X(135) \
+  X(144) X(150) X(160) X(180) X(192)
+
+// Elements of row data a lane may hold across the row pass.
+template <typename T> constexpr int plane_row_budget() { return sizeof(T) == 8 ? 16 : 36; }
+
+template <int N, bool PRUNE> constexpr int plane_kept() {
+  return PRUNE && PlaneLine<N>::prunes ? 2 * PlaneLine<N>::kept : PlaneLine<N>::L;
+}
+
+// Waves of the square N x N kernel's workgroup, measured over 2 .. 12 (FFT phase
+// of 128 bands, or as many as 3e8 bytes of sticks hold).  Whole quads of waves
+// win (they load the four SIMDs evenly: 72^2 in FP64 takes 292 us with four
+// waves, 403 with six): four while several workgroups share a CU (two are up to
+// 5% faster below 64^2, and slower for a few bands), twelve where an FP64
+// plane's LDS admits one or two per CU and four waves' rows would not fit
+// their registers (96^2: 864 us, 894 with three).  The kernels of four waves
+// before, with exchange lines of their own above 72^2, took: FP64 75^2 1007 us
+// (now 732), 80^2 662 (541), 90^2 1029 (797), 100^2 1298 (773), 108^2 1441
+// (890), 120^2 1348 (822), 128^2 in the split stage 3323 (1034); FP32 90^2 386
+// (322), 108^2 502 (380), 120^2 464 (361), 128^2 2640 (684).
+template <typename T, int N, bool PRUNE> constexpr int plane_waves() {
+  constexpr int kept = plane_kept<N, PRUNE>();
+  constexpr bool fp64 = sizeof(T) == 8;
+  int w = fp64 ? (N <= 80 && N != 75 ? 4 : 12) : (N < 120 ? 4 : 8);
+  while (w < 16) {
+    const int teams = w * PlaneLine<N>::per_wave;
+    const int rows = (N + teams - 1) / teams;
+    if (rows <= 6 && rows * kept <= plane_row_budget<T>()) break;
+    w += w < 4 ? 1 : 4;
+  }
+  return w;
+}
+
+template <typename T, int N, bool PRUNE, int W>
+__device__ __forceinline__ void plane_square_body(const PlaneArgs<T>& g, int z, int64_t b) {
+  extern __shared__ unsigned char smem_raw[];
+  cplx<T>* Q = reinterpret_cast<cplx<T>*>(smem_raw);
+  cplx<T>* w = g.work + b * g.bstride + (int64_t)z * g.nst;
+  constexpr int teams = W * PlaneLine<N>::per_wave;
+  // the per-lane tables of all passes, fetched while the sticks are
+  PlaneTwiddles<T, N> tw;
+  tw.load(PlaneLane<N>().t, g.tw1);
+  int cq[PlaneLine<N>::L];
+  plane_row_slots<T, N, PRUNE>(g, N + 1, cq);
+  plane_cols_backward<T, N, PRUNE>(g, w, Q, W, tw);
+  __syncthreads();
+  plane_rows<T, N, PRUNE, (N + teams - 1) / teams>(g, z, Q, N, N + 1, W, tw, cq);
+  __syncthreads();
+  plane_cols_forward<T, N, PRUNE>(g, w, Q, W, tw);
+}
+
+template <typename T, int N, bool PRUNE, int W>
+__global__ __launch_bounds__(64 * W, W > 12 ? 4 : 3) void k_plane_square(PlaneArgs<T> g) {
+  plane_square_body<T, N, PRUNE, W>(g, blockIdx.x, blockIdx.y);
+}
+
+// Any two lengths: the passes are chosen at run time (uniform branches).  Two
+// kernels: the lengths whose halves need few registers, and all.  Against the
+// Stockham plane kernel that served them (128 bands, FP64 / FP32): 48 x 60 x 80
+// 1069 / 925 us -> 221 / 127 us, 36 x 40 x 160 1731 / 1551 -> 263 / 190, 72 x 75
+// x 90 1751 / 1440 -> 458 / 277, 108 x 120 x 60 3857 / 3192 -> 926 / 386.
+constexpr int kPlaneAnyWaves = 12;
+// Rows per team of the run-time kernels: with six kept slots three FP64 rows
+// spill (90 x 108 x 60, 128 bands: 913 us with three, 685 us with two).
+template <typename T, int N1> constexpr int plane_any_rows() {
+  return sizeof(T) == 8 && plane_kept<N1, true>() > 4 ? 2 : 3;
+}
+constexpr bool plane_any_small(int n) { return n <= 108 && n / team_L(n) <= 12; }
+
+template <typename T, bool SMALL>
+__global__ __launch_bounds__(64 * kPlaneAnyWaves, 3) void k_plane_any(PlaneArgs<T> g) {
+  extern __shared__ unsigned char smem_raw[];
+  cplx<T>* Q = reinterpret_cast<cplx<T>*>(smem_raw);
+  cplx<T>* w = g.work + blockIdx.y * g.bstride + (int64_t)blockIdx.x * g.nst;
+  const int waves = blockDim.x >> 6;
+  switch (g.n2) {
+#define QEPW_PLANE_CASE(NN)                                                               \
+  case NN:                                                                                \
+    if constexpr (!SMALL || plane_any_small(NN)) {                                        \
+      PlaneTwiddles<T, NN> tw;                                                            \
+      tw.load(PlaneLane<NN>().t, g.tw2);                                                  \
+      plane_cols_backward<T, NN, true>(g, w, Q, waves, tw);                               \
+    }                                                                                     \
+    break;
+    QEPW_TEAM_SIZES(QEPW_PLANE_CASE)
+#undef QEPW_PLANE_CASE
+    default: break;
+  }
+  __syncthreads();
+  switch (g.n1) {
+#define QEPW_PLANE_CASE(NN)                                                               \
+  case NN:                                                                                \
+    if constexpr (!SMALL || plane_any_small(NN)) {                                        \
+      PlaneTwiddles<T, NN> tw;                                                            \
+      tw.load(PlaneLane<NN>().t, g.tw1);                                                  \
+      int cq[PlaneLine<NN>::L];                                                           \
+      plane_row_slots<T, NN, true>(g, g.n2 + 1, cq);                                      \
+      plane_rows<T, NN, true, plane_any_rows<T, NN>()>(g, blockIdx.x, Q, g.n2, g.n2 + 1,  \
+                                                       waves, tw, cq);                    \
+    }                                                                                     \
+    break;
+    QEPW_TEAM_SIZES(QEPW_PLANE_CASE)
+#undef QEPW_PLANE_CASE
+    default: break;
+  }
+  __syncthreads();
+  switch (g.n2) {
+#define QEPW_PLANE_CASE(NN)                                                               \
+  case NN:                                                                                \
+    if constexpr (!SMALL || plane_any_small(NN)) {                                        \
+      PlaneTwiddles<T, NN> tw;                                                            \
+      tw.load(PlaneLane<NN>().t, g.tw2);                                                  \
+      plane_cols_forward<T, NN, true>(g, w, Q, waves, tw);                                \
+    }                                                                                     \
+    break;
+    QEPW_TEAM_SIZES(QEPW_PLANE_CASE)
+#undef QEPW_PLANE_CASE
+    default: break;
+  }
+}
+
+// ---- one launch for many problems ---------------------------------------------
+// The plane stage of up to kMaxFftGroup square problems: workgroups of all
+// problems end to end along x, each finding its problem in a prefix table and
+// running the one-problem body of its length.
+template <typename T> struct PlaneGroup {
+  int count;
+  int start[kMaxFftGroup + 1];
+  int n3[kMaxFftGroup];
+  int prune[kMaxFftGroup];
+  PlaneArgs<T> plane[kMaxFftGroup];
+};
+
+template <typename T> constexpr int plane_group_waves() {
+  int w = 0;
+#define QEPW_PLANE_CASE(NN)                            \
+  w = std::max(w, plane_waves<T, NN, true>());         \
+  w = std::max(w, plane_waves<T, NN, false>());
+  QEPW_GROUP_SIZES(QEPW_PLANE_CASE)
+#undef QEPW_PLANE_CASE
+  return w;
+}
+
+template <typename T>
+__global__ __launch_bounds__(64 * plane_group_waves<T>(), 3) void k_plane_group(
+    const PlaneGroup<T> g) {
+  constexpr int W = plane_group_waves<T>();
+  const int p = group_of(g.start, g.count, blockIdx.x);
+  const int l = blockIdx.x - g.start[p];
+  const int z = l % g.n3[p];
+  const int64_t b = l / g.n3[p];
+  switch (g.plane[p].n1) {
+#define QEPW_PLANE_CASE(NN)                                                       \
+  case NN:                                                                        \
+    if (g.prune[p]) plane_square_body<T, NN, true, W>(g.plane[p], z, b);          \
+    else plane_square_body<T, NN, false, W>(g.plane[p], z, b);                    \
+    break;
+    QEPW_GROUP_SIZES(QEPW_PLANE_CASE)
+#undef QEPW_PLANE_CASE
+    default: break;
+  }
+}
+
+// ---- host side ------------------------------------------------------------------
+template <typename T> const cplx<T>* plane_twiddles(const Plan& p, int axis);
+
+template <typename T>
+static PlaneArgs<T> plane_args(const Plan& p, const StickTables& st, cplx<T>* work,
+                               int64_t bstride, const T* V) {
+  PlaneArgs<T> g{};
+  g.work = work;
+  g.bstride = bstride;
+  g.nst = st.nst;
+  g.n1 = p.n1;
+  g.n2 = p.n2;
+  g.nxc = st.nxcols;
+  g.colpos = st.d_colpos;
+  g.colmap = st.d_colmap;
+  g.V = V;
+  g.tw1 = plane_twiddles<T>(p, 0);
+  g.tw2 = plane_twiddles<T>(p, 1);
+  return g;
+}
+
+template <typename T> PlaneChoice plane_choice(const Plan& p, const StickTables& st) {
+  PlaneChoice c;
+  if (!st.d_colpos || !st.d_colmap || !plane_twiddles<T>(p, 0) || !plane_twiddles<T>(p, 1))
+    return c;
+  int per1 = 0, per2 = 0, wprune = 0, wfull = 0, any_rows = 0;
+  bool prune1 = false, prune2 = false;
+#define QEPW_PLANE_N(NN)                                                     \
+  if (p.n1 == NN) {                                                          \
+    per1 = PlaneLine<NN>::per_wave;                                          \
+    any_rows = plane_any_rows<T, NN>();                                      \
+    prune1 = (st.xmask & ~PlaneLine<NN>::pruned) == 0u;                      \
+    wprune = plane_waves<T, NN, true>();                                     \
+    wfull = plane_waves<T, NN, false>();                                     \
+  }                                                                          \
+  if (p.n2 == NN) {                                                          \
+    per2 = PlaneLine<NN>::per_wave;                                          \
+    prune2 = (st.ymask & ~PlaneLine<NN>::pruned) == 0u;                      \
+  }
+  QEPW_TEAM_SIZES(QEPW_PLANE_N)
+#undef QEPW_PLANE_N
+  if (per1 == 0 || per2 == 0) return c;
+  c.prune = prune1 && prune2;
+  c.square = p.n1 == p.n2 && p.n1 <= 128;
+  if (c.square) {
+    c.waves = c.prune ? wprune : wfull;
+  } else if (c.prune) {
+    // whole quads of waves where more than two are needed: a workgroup's waves
+    // then share the four SIMDs evenly
+    for (int w : {2, 4, 8, 12}) {
+      if (p.n2 > any_rows * w * per1) continue;
+      c.waves = w;
+      break;
+    }
+  }
+  c.lds = std::max((size_t)(st.nxcols + 1) * (p.n2 + 1), (size_t)c.waves * per1 * (p.n1 + 1)) *
+          sizeof(cplx<T>);
+  if (c.lds > (size_t)kMaxLdsBytes) c.waves = 0;
+  return c;
+}
+
+template <typename T>
+bool launch_plane_stage(const Plan& p, const StickTables& st, cplx<T>* work, int64_t bstride,
+                        const T* V, int nb, hipStream_t stream) {
+  const PlaneChoice& c = sizeof(T) == 8 ? st.plane64 : st.plane32;
+  if (c.waves == 0) return false;
+  const PlaneArgs<T> g = plane_args<T>(p, st, work, bstride, V);
+  const dim3 grid(p.n3, nb);
+#define QEPW_PLANE_LAUNCH(K)                                                            \
+  do {                                                                                  \
+    allow_lds(reinterpret_cast<const void*>(&K), c.lds);                                \
+    hipLaunchKernelGGL(K, grid, dim3(64 * c.waves), c.lds, stream, g);                  \
+    return true;                                                                        \
+  } while (0)
+  if (c.square) {
+#define QEPW_PLANE_SQUARE(NN)                                                           \
+  if constexpr (NN <= 128) {                                                            \
+    if (p.n1 == NN && c.prune)                                                          \
+      QEPW_PLANE_LAUNCH((k_plane_square<T, NN, true, plane_waves<T, NN, true>()>));     \
+    if (p.n1 == NN)                                                                     \
+      QEPW_PLANE_LAUNCH((k_plane_square<T, NN, false, plane_waves<T, NN, false>()>));   \
+  }
+    QEPW_TEAM_SIZES(QEPW_PLANE_SQUARE)
+#undef QEPW_PLANE_SQUARE
+    return false;
+  }
+  if (plane_any_small(p.n1) && plane_any_small(p.n2)) QEPW_PLANE_LAUNCH((k_plane_any<T, true>));
+  QEPW_PLANE_LAUNCH((k_plane_any<T, false>));
+#undef QEPW_PLANE_LAUNCH
+  return false;
+}
+
+// The grouped plane stage of ``count`` square problems whose lengths are among
+// QEPW_GROUP_SIZES (nb bands each).
+template <typename T>
+int launch_plane_group(int count, const Plan* const* plans, cplx<T>* const* work,
+                       const int64_t* bstride, const T* const* V, const int* nb,
+                       hipStream_t stream) {
+  PlaneGroup<T> g{};
+  g.count = count;
+  int64_t total = 0;
+  size_t lds = 0;
+  for (int j = 0; j < count; ++j) {
+    const Plan& p = *plans[j];
+    const PlaneChoice& c = sizeof(T) == 8 ? p.sphere.plane64 : p.sphere.plane32;
+    g.start[j] = (int)total;
+    g.n3[j] = p.n3;
+    g.prune[j] = c.prune ? 1 : 0;
+    g.plane[j] = plane_args<T>(p, p.sphere, work[j], bstride[j], V[j]);
+    total += (int64_t)p.n3 * nb[j];
+    int per = 0;
+#define QEPW_PLANE_N(NN) if (p.n1 == NN) per = PlaneLine<NN>::per_wave;
+    QEPW_GROUP_SIZES(QEPW_PLANE_N)
+#undef QEPW_PLANE_N
+    lds = std::max(lds, std::max((size_t)(p.sphere.nxcols + 1),
+                                 (size_t)plane_group_waves<T>() * per) *
+                            (p.n1 + 1) * sizeof(cplx<T>));
+  }
+  if (total > 0x7fffffff || lds > (size_t)kMaxLdsBytes) return QEPW_ERR_UNSUPPORTED;
+  g.start[count] = (int)total;
+  allow_lds(reinterpret_cast<const void*>(&k_plane_group<T>), lds);
+  hipLaunchKernelGGL(k_plane_group<T>, dim3((unsigned)total), dim3(64 * plane_group_waves<T>()),
+                     lds, stream, g);
+  return QEPW_OK;
+}
+
+}  // namespace qepw

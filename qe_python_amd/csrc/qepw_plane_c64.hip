@@ -1,0 +1,18 @@
+// The xy-plane stage in complex64 (qepw_plane.h).
+#include "qepw_plane.h"
+
+namespace qepw {
+
+template <> const float2* plane_twiddles<float>(const Plan& p, int axis) {
+  return plane_lane_table(axis == 0 ? p.n1 : p.n2, false) ? p.d_ltw32[axis] : p.d_tw32[axis];
+}
+
+template PlaneChoice plane_choice<float>(const Plan& p, const StickTables& st);
+template bool launch_plane_stage<float>(const Plan& p, const StickTables& st, float2* work,
+                                         int64_t bstride, const float* V, int nb,
+                                         hipStream_t stream);
+template int launch_plane_group<float>(int count, const Plan* const* plans, float2* const* work,
+                                        const int64_t* bstride, const float* const* V,
+                                        const int* nb, hipStream_t stream);
+
+}  // namespace qepw

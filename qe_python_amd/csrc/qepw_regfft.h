@@ -128,13 +128,6 @@ template <typename T, int SIGN> struct RegDft<T, 1, SIGN> {
   static __device__ __forceinline__ void run(cplx<T>*) {}
 };
 
-constexpr int team_L(int n) {
-  int best = 0;
-  for (int l = 1; l <= 16; ++l)
-    if (n % l == 0 && n / l <= 16 && n / l >= l) best = l;
-  return best;
-}
-
 // Orders this wave's LDS accesses around a team exchange (no workgroup sync).
 __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");

@@ -328,3 +328,35 @@ def test_timed_apply_matches_and_times_the_phase(medium):
     assert torch.equal(got, ref)
     inner = start.elapsed_time(stop)
     assert 0.0 < inner <= outer0.elapsed_time(outer1) + 1e-3
+
+
+@pytest.mark.parametrize("shape,dense", [
+    ((16, 18, 20), False), ((20, 16, 18), False), ((27, 45, 24), False), ((36, 40, 54), False),
+    ((60, 48, 30), False), ((75, 96, 20), False), ((128, 120, 16), False),
+    ((120, 128, 16), False), ((90, 160, 18), False), ((192, 50, 16), False),
+    ((96, 96, 16), False), ((128, 128, 16), False), ((24, 30, 20), True), ((40, 40, 20), True)])
+def test_plane_stage_of_any_two_lengths(shape, dense):
+    """The xy-plane stage for rectangular planes, at its largest sides, with the
+    k-point pushing the sphere across the pruned slots, and (``dense``) for
+    bases that fill the axes, which the pruned kernels cannot take."""
+    from qe_python_amd.basis import PlaneWaveBasis
+    from qe_python_amd.diagonalization import PlaneWaveHamiltonian
+    rng = np.random.default_rng(37)
+    ax = [np.arange(-((n - 1) // 2), n // 2 + 1) if dense
+          else np.arange(-((n + 1) // 4), (n - 1) // 4 + 1) for n in shape]
+    m = np.stack(np.meshgrid(*ax, indexing="ij"), -1).reshape(-1, 3)
+    if not dense:   # an ellipsoid reaching the ends of each axis
+        half = np.array([len(a) / 2.0 for a in ax])
+        mid = np.array([(a[0] + a[-1]) / 2.0 for a in ax])
+        m = m[(((m - mid) / half) ** 2).sum(1) <= 1.0]
+    m = m[rng.permutation(len(m))].astype(np.int32)
+    kin = 0.5 * (m.astype(float) ** 2).sum(1) / 100.0
+    basis = PlaneWaveBasis(m, m.astype(float), kin)
+    vr = rng.uniform(-1.0, 0.5, shape)
+    x = rng.standard_normal((len(m), 2)) + 1j * rng.standard_normal((len(m), 2))
+    ref = OracleHamiltonian(m, kin, shape, vr).apply(x)
+    ham = PlaneWaveHamiltonian(basis, np.zeros(shape, complex), (), real_potential=vr)
+    assert rel(ham.apply(x), ref) <= 1e-12
+    ham32 = PlaneWaveHamiltonian(basis, np.zeros(shape, complex), (), real_potential=vr,
+                                 precision="fp32")
+    assert rel(ham32.apply(x), ref) <= 2e-6
