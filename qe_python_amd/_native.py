@@ -181,8 +181,8 @@ def load() -> ctypes.CDLL:
         fn.argtypes = argtypes
     _LIB = lib
     _register_host_lapack(lib)
-    # the committed GEMM tile table (qe_python_amd.autotune); QEPW_GEMM_TABLE
-    # names another table, or "none" for the built-in choice
+    # a tuned GEMM tile table (qe_python_amd.autotune), if there is one;
+    # QEPW_GEMM_TABLE names another, or "none" for the built-in choice
     table = os.environ.get("QEPW_GEMM_TABLE")
     if table != "none":
         from . import autotune

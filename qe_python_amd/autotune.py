@@ -2,12 +2,14 @@
 
 ``qepw_gemm`` has a handful of tile variants (TM x TN output tiles per
 workgroup) and splits K over workgroups for the tall A^H B products over the
-plane waves.  The built-in choice is a heuristic; this module times every
-variant (and, for the split products, a range of split counts) on the
-device for the shape classes a Davidson solve produces, and writes the
-winners as rules into a JSON table that ``load_table`` installs in the
-library (``qepw_gemm_set_rule``).  The table committed next to this module
-(``tuning/gemm_gfx950.json``) is loaded automatically with the library.
+plane waves.  The built-in choice is the cheapest of a cost model fitted to
+measured times (within 3% of the best tile and split in the mean), so that no
+table is needed; this module times every variant (and, for the split
+products, a range of split counts) on the device for the shape classes a
+Davidson solve produces, and writes the winners as rules into a JSON table
+that ``load_table`` installs in the library (``qepw_gemm_set_rule``).  A
+table at ``tuning/gemm_gfx950.json`` next to this module, or one that
+``QEPW_GEMM_TABLE`` names, is loaded with the library.
 
 Shape classes (per precision):
 

@@ -113,6 +113,38 @@ def test_every_gemm_tile_variant_matches_numpy(prec, op):
         autotune.load_table()
 
 
+@pytest.mark.parametrize("prec", ["c128", "c64"])
+@pytest.mark.parametrize("op", ["N", "C"])
+def test_gemm_chosen_plans_at_tile_and_step_edges(prec, op):
+    """The built-in tile and split at the edges of tiles (columns 2, 15..17,
+    a row more than a tile) and of K steps (depths 1, 15, 17, a split's ragged
+    end), against NumPy, with the partials inside the static scratch."""
+    import ctypes
+
+    from qe_python_amd import _native as nat
+    from qe_python_amd import device as dv
+    lib = nat.load()
+    dtype = torch.complex128 if prec == "c128" else torch.complex64
+    size = 16 if prec == "c128" else 8
+    code = nat.OP_N if op == "N" else nat.OP_C
+    ws = dv.Workspace(torch.device(DEV))
+    for m, n, k in [(65, 2, 1), (33, 15, 15), (1, 16, 17), (129, 17, 2950), (64, 16, 4097),
+                    (2951, 16, 31), (4097, 13, 257), (8, 8, 2950), (257, 40, 2049)]:
+        rng = np.random.default_rng(m + n + k)
+        a = rand(rng, m, k) if op == "N" else rand(rng, k, m)
+        b = rand(rng, k, n)
+        ta, tb = dev_block(a, dtype), dev_block(b, dtype)
+        tc = dev_block(np.zeros((m, n), complex), dtype)
+        plan = (ctypes.c_int64 * 4)()
+        nat.check(lib.qepw_gemm_plan(dv.precision_code(dtype), code, m, n, k, plan), "plan")
+        assert plan[1] == 1 or plan[1] * m * n * size <= lib.qepw_gemm_static_scratch_bytes()
+        dv.gemm(code, m, n, k, 1.0, ta, tb, 0.0, tc, ws)
+        ref = (a if op == "N" else a.conj().T) @ b
+        tol = 1e-12 if prec == "c128" else 2e-6 + 1e-7 * np.sqrt(k)
+        err = np.linalg.norm(host_block(tc) - ref) / np.linalg.norm(ref)
+        assert err < tol, (m, n, k, list(plan), err)
+
+
 def test_gemm_split_k_is_deterministic():
     from qe_python_amd import _native as nat
     from qe_python_amd import device as dv
