@@ -411,6 +411,22 @@ int qepw_projector_forces(int precision, const void* dO, int64_t lddo, int64_t d
                           const int32_t* off, int natom, double* out, void* stream);
 
 /*
+ * The same dE/dtau from psi, the packed projectors and D O in one product over
+ * the bands (no dO blocks): out[a, c] = 2 sum_g q[g, c] sum_{i in atom a}
+ * Im(B[g, i] conj(W[g, i])), W = psi diag(f) (D O)^H.  psi: (npw x nb), proj:
+ * (npw x nproj), coupled: (nproj x nb), column-major device arrays of the
+ * precision; q: device double (npw, 3); f: device double (nb).
+ * Replaces: the force branch of _nonlocal_derivatives
+ *   (qepy_pw/pw/scf.py:1521-1631).
+ */
+size_t qepw_position_gradient_workspace(int precision, int64_t npw, int64_t nproj, int nb);
+int qepw_position_gradient(int precision, const void* psi, int64_t ldpsi, int nb,
+                           const void* proj, int64_t ldproj, int64_t nproj,
+                           const void* coupled, int64_t ldc, const double* f, const double* q,
+                           int64_t npw, const int32_t* off, int natom, double* out,
+                           void* workspace, size_t ws_bytes, void* stream);
+
+/*
  * Pieces of the device Rayleigh-Ritz that replaces the host zhegvd call of
  * davidson (generalized_eigh, qepy_pw/_native_fft.pyx:667-691, via
  * _lowest_generalized_eigh, qepy_pw/diagonalization.py:83-110).  All operate

@@ -101,6 +101,10 @@ SIGNATURES = [
     ("qepw_projector_basis", c_int, [c_void_p, c_int64, c_void_p, c_int64, c_int, c_double,
                                      c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int64,
                                      c_void_p]),
+    ("qepw_position_gradient_workspace", c_size_t, [c_int, c_int64, c_int64, c_int]),
+    ("qepw_position_gradient", c_int, [c_int, c_void_p, c_int64, c_int, c_void_p, c_int64,
+                                       c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_int64,
+                                       c_void_p, c_int, c_void_p, c_void_p, c_size_t, c_void_p]),
     ("qepw_projector_forces", c_int, [c_int, c_void_p, c_int64, c_int64, c_void_p, c_int64,
                                       c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p]),
     ("qepw_hermitian_complete", c_int, [c_void_p, c_int64, c_int, c_int, c_void_p]),

@@ -780,6 +780,29 @@ int qepw_projector_forces(int precision, const void* dO, int64_t lddo, int64_t d
                 "qepw_projector_forces");
 }
 
+size_t qepw_position_gradient_workspace(int precision, int64_t npw, int64_t nproj, int nb) {
+  return qepw::position_gradient_bytes(precision, npw, nproj, nb);
+}
+
+int qepw_position_gradient(int precision, const void* psi, int64_t ldpsi, int nb,
+                           const void* proj, int64_t ldproj, int64_t nproj,
+                           const void* coupled, int64_t ldc, const double* f, const double* q,
+                           int64_t npw, const int32_t* off, int natom, double* out,
+                           void* workspace, size_t ws_bytes, void* stream) {
+  if (nb < 0 || npw < 0 || nproj < 0)
+    return fail(QEPW_ERR_ARG, "qepw_position_gradient: negative size");
+  if (natom > 0 && (!off || !out))
+    return fail(QEPW_ERR_ARG, "qepw_position_gradient: bad argument");
+  if (natom > 0 && npw > 0 && nproj > 0 &&
+      (!proj || !q || !workspace || ldproj < npw ||
+       (nb > 0 && (!psi || !coupled || !f || ldpsi < npw || ldc < nproj))))
+    return fail(QEPW_ERR_ARG, "qepw_position_gradient: bad argument");
+  return finish(qepw::position_gradient(precision, npw, nproj, nb, psi, ldpsi, coupled, ldc, f,
+                                        proj, ldproj, q, off, natom, out, workspace, ws_bytes,
+                                        static_cast<hipStream_t>(stream)),
+                "qepw_position_gradient");
+}
+
 }  // extern "C"
 
 extern "C" {

@@ -110,36 +110,34 @@ __device__ __forceinline__ void gemm_tile(unsigned b, unsigned mt, unsigned nt, 
 // every load checked: FP64 78 805 x 192 x 512 1114 -> 983 us (63 TFLOP/s, at
 // the power limit), 512 x 192 x 78 805 (A^H B) 1136 -> 1010; FP32 695 -> 548
 // (113 TFLOP/s) and 740 -> 560; FP64 23 847 x 13 x 256 35 -> 28.
-template <typename T, bool CONJ_A, bool CONJ_B, int TM, int TN, int WAVES_M>
-__global__ __launch_bounds__(kGemmThreads, 2) void k_cgemm(
-    int64_t M, int64_t N, int64_t K, int64_t kchunk, unsigned mt, unsigned nt, unsigned splits,
-    const cplx<T>* __restrict__ A, int64_t lda, const cplx<T>* __restrict__ B, int64_t ldb,
-    cplx<T>* __restrict__ C, int64_t ldc, cplx<T>* __restrict__ partial, T alpha_r, T alpha_i,
-    T beta_r, T beta_i) {
-  using Acc = typename Mfma<T>::acc;
-  using Pair = typename Mfma<T>::pair;
-  constexpr int BK = gemm_bk<T, TM, TN>();
-  constexpr int WAVES_N = 4 / WAVES_M;
-  constexpr int WTM = TM / WAVES_M;  // wave tile
-  constexpr int WTN = TN / WAVES_N;
-  constexpr int NBM = WTM / 16;      // MFMA blocks per wave and dimension
-  constexpr int NBN = WTN / 16;
+template <typename T, int TM, int TN, int WAVES_M> struct GemmTile {
+  static constexpr int BK = gemm_bk<T, TM, TN>();
+  static constexpr int NBUF = gemm_buffers<T, TM, TN>();
+  static constexpr int WAVES_N = 4 / WAVES_M;
+  static constexpr int WTM = TM / WAVES_M;  // wave tile
+  static constexpr int WTN = TN / WAVES_N;
+  static constexpr int NBM = WTM / 16;      // MFMA blocks per wave and dimension
+  static constexpr int NBN = WTN / 16;
   static_assert(NBM >= 1 && NBN >= 1 && WAVES_M * WAVES_N == 4, "tile shape");
-  constexpr int NBUF = gemm_buffers<T, TM, TN>();
+};
+
+// re, im = the wave's part of op(A) op(B) over K in [kbeg, kend), at rows m0,
+// columns n0 of the output
+template <typename T, bool CONJ_A, bool CONJ_B, int TM, int TN, int WAVES_M, int NBM, int NBN>
+__device__ __forceinline__ void gemm_accumulate(
+    int64_t M, int64_t N, int64_t m0, int64_t n0, int64_t kbeg, int64_t kend,
+    const cplx<T>* __restrict__ A, int64_t lda, const cplx<T>* __restrict__ B, int64_t ldb,
+    typename Mfma<T>::acc (&re)[NBM][NBN], typename Mfma<T>::acc (&im)[NBM][NBN]) {
+  using Pair = typename Mfma<T>::pair;
+  using G = GemmTile<T, TM, TN, WAVES_M>;
+  constexpr int BK = G::BK, NBUF = G::NBUF;
   __shared__ Pair As[NBUF][BK][TM + kPad];
   __shared__ Pair Bs[NBUF][BK][TN + kPad];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
-  const int wm = (wave % WAVES_M) * WTM;
-  const int wn = (wave / WAVES_M) * WTN;
-  unsigned bm, bn, bs;
-  gemm_tile(blockIdx.x, mt, nt, splits, bm, bn, bs);
-  const int64_t m0 = (int64_t)bm * TM;
-  const int64_t n0 = (int64_t)bn * TN;
-  const int64_t kbeg = (int64_t)bs * kchunk;
-  const int64_t kend = (kbeg + kchunk) < K ? (kbeg + kchunk) : K;
-  Acc re[NBM][NBN], im[NBM][NBN];
+  const int wm = (wave % WAVES_M) * G::WTM;
+  const int wn = (wave / WAVES_M) * G::WTN;
 #pragma unroll
   for (int i = 0; i < NBM; ++i)
 #pragma unroll
@@ -256,7 +254,30 @@ __global__ __launch_bounds__(kGemmThreads, 2) void k_cgemm(
     if (more) store(buf);
     __syncthreads();
   }
+}
 
+template <typename T, bool CONJ_A, bool CONJ_B, int TM, int TN, int WAVES_M>
+__global__ __launch_bounds__(kGemmThreads, 2) void k_cgemm(
+    int64_t M, int64_t N, int64_t K, int64_t kchunk, unsigned mt, unsigned nt, unsigned splits,
+    const cplx<T>* __restrict__ A, int64_t lda, const cplx<T>* __restrict__ B, int64_t ldb,
+    cplx<T>* __restrict__ C, int64_t ldc, cplx<T>* __restrict__ partial, T alpha_r, T alpha_i,
+    T beta_r, T beta_i) {
+  using G = GemmTile<T, TM, TN, WAVES_M>;
+  constexpr int NBM = G::NBM, NBN = G::NBN;
+  unsigned bm, bn, bs;
+  gemm_tile(blockIdx.x, mt, nt, splits, bm, bn, bs);
+  const int64_t m0 = (int64_t)bm * TM;
+  const int64_t n0 = (int64_t)bn * TN;
+  const int64_t kbeg = (int64_t)bs * kchunk;
+  const int64_t kend = (kbeg + kchunk) < K ? (kbeg + kchunk) : K;
+  typename Mfma<T>::acc re[NBM][NBN], im[NBM][NBN];
+  gemm_accumulate<T, CONJ_A, CONJ_B, TM, TN, WAVES_M>(M, N, m0, n0, kbeg, kend, A, lda, B, ldb,
+                                                      re, im);
+
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const int wm = (wave % WAVES_M) * G::WTM;
+  const int wn = (wave / WAVES_M) * G::WTN;
   const bool direct = splits == 1;
 #pragma unroll
   for (int i = 0; i < NBM; ++i)
@@ -414,6 +435,96 @@ static GemvPlan gemv_plan(bool ca, int64_t m, int64_t k) {
 }
 
 // Tile variants of k_cgemm: (TM, TN, WAVES_M).
+// The projector force, dE/dtau_a,c = 2 sum_n f_n Re sum_{i in a} conj(dO_c[i,n])
+// (D O)[i,n] with dO_c = i B^H (q_c psi), in one product over the bands instead of
+// three over the plane waves: with W = psi (f D O)^H (npw x P),
+//   dE/dtau_a,c = 2 sum_G q_c(G) sum_{i in a} Im(B[G,i] conj(W[G,i])),
+// so W is contracted with B and q in the tile's epilogue and never stored.  Each
+// wave writes the sums of its rows, in FP64 for both precisions, to
+// partial[(c P + i) parts + part]; k_force_sum adds them in a fixed order.
+//
+// Bound by the product's FP64 MFMAs (8 npw P nb flops, a third of the former
+// ones, which also read psi, scaled, three times).  23 847 x 256 projectors x
+// 128 bands: the three scalings and products with their reductions took 430 us
+// in FP64, this and its sums 137.
+template <typename T, int TM, int TN, int WAVES_M>
+__global__ __launch_bounds__(kGemmThreads, 2) void k_force_product(
+    int64_t npw, int64_t nproj, int64_t nb, unsigned mt, unsigned nt,
+    const cplx<T>* __restrict__ psi, int64_t ldpsi, const cplx<T>* __restrict__ fdo,
+    int64_t ldf, const cplx<T>* __restrict__ proj, int64_t ldproj, const double* __restrict__ q,
+    double* __restrict__ partial) {
+  using G = GemmTile<T, TM, TN, WAVES_M>;
+  constexpr int NBM = G::NBM, NBN = G::NBN;
+  unsigned bm, bn, bs;
+  gemm_tile(blockIdx.x, mt, nt, 1, bm, bn, bs);
+  const int64_t m0 = (int64_t)bm * TM;
+  const int64_t n0 = (int64_t)bn * TN;
+  typename Mfma<T>::acc re[NBM][NBN], im[NBM][NBN];
+  gemm_accumulate<T, false, true, TM, TN, WAVES_M>(npw, nproj, m0, n0, 0, nb, psi, ldpsi, fdo,
+                                                   ldf, re, im);
+
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const int64_t row0 = m0 + (wave % WAVES_M) * G::WTM;
+  const int64_t col0 = n0 + (wave / WAVES_M) * G::WTN + (lane & 15);
+  double sum[NBN][3];
+#pragma unroll
+  for (int j = 0; j < NBN; ++j) sum[j][0] = sum[j][1] = sum[j][2] = 0.0;
+#pragma unroll
+  for (int i = 0; i < NBM; ++i)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int64_t row = row0 + 16 * i + Mfma<T>::row(lane, v);
+      if (row >= npw) continue;
+      const double q0 = q[3 * row], q1 = q[3 * row + 1], q2 = q[3 * row + 2];
+#pragma unroll
+      for (int j = 0; j < NBN; ++j) {
+        const int64_t col = col0 + 16 * j;
+        if (col >= nproj) continue;
+        const cplx<T> b = proj[row + col * ldproj];
+        const double z = (double)b.y * re[i][j][v] - (double)b.x * im[i][j][v];
+        sum[j][0] += q0 * z;
+        sum[j][1] += q1 * z;
+        sum[j][2] += q2 * z;
+      }
+    }
+  // the four lanes of a column
+  const int64_t parts = (int64_t)mt * WAVES_M;
+  const int64_t part = (int64_t)bm * WAVES_M + wave % WAVES_M;
+#pragma unroll
+  for (int j = 0; j < NBN; ++j) {
+    const int64_t col = col0 + 16 * j;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      double s = sum[j][c];
+      s += __shfl_xor(s, 16);
+      s += __shfl_xor(s, 32);
+      if (lane < 16 && col < nproj) partial[(c * nproj + col) * parts + part] = s;
+    }
+  }
+}
+
+// out[a, c] = 2 sum of the partials of atom a's projectors [off[a], off[a+1])
+__global__ __launch_bounds__(1024) void k_force_sum(const double* __restrict__ partial,
+                                                    int64_t nproj, int64_t parts,
+                                                    const int* __restrict__ off,
+                                                    double* __restrict__ out) {
+  __shared__ double sh[1024];
+  const int a = blockIdx.x, c = blockIdx.y, tid = threadIdx.x;
+  const int i0 = off[a];
+  const int64_t count = (int64_t)(off[a + 1] - i0) * parts;
+  const double* p = partial + (c * nproj + i0) * parts;
+  double s = 0.0;
+  for (int64_t e = tid; e < count; e += 1024) s += p[e];
+  sh[tid] = s;
+  __syncthreads();
+  for (int h = 512; h > 0; h >>= 1) {
+    if (tid < h) sh[tid] += sh[tid + h];
+    __syncthreads();
+  }
+  if (tid == 0) out[3 * a + c] = 2.0 * sh[0];
+}
+
 struct GemmVariant {
   int tm, tn, waves_m;
 };
@@ -610,6 +721,83 @@ int gemm_plan(int precision, int op_a, int64_t m, int64_t n, int64_t k, int64_t*
   out[2] = kVariants[sp.variant].tm;
   out[3] = kVariants[sp.variant].tn;
   return QEPW_OK;
+}
+
+// Of the 32 x 32 and the 64 x 64 tile the cheaper for the product by plan_cost:
+// 10 127 x 108 projectors x 60 bands in FP32 20.7 us with the large tile, 1.2 of
+// which a CU gets, 14.8 with the small one.
+static int force_variant(int precision, int64_t npw, int64_t nproj, int64_t nb) {
+  return plan_cost(precision, 0, npw, nproj, 1, nb) < plan_cost(precision, 1, npw, nproj, 1, nb)
+             ? 0
+             : 1;
+}
+
+static int64_t force_parts(int precision, int64_t npw, int64_t nproj, int64_t nb) {
+  const GemmVariant& v = kVariants[force_variant(precision, npw, nproj, nb)];
+  return (npw + v.tm - 1) / v.tm * v.waves_m;
+}
+
+// the weighted couplings (a multiple of 256 bytes), then the partial sums
+static size_t force_weighted_bytes(int precision, int64_t nproj, int64_t nb) {
+  const size_t elem = precision == QEPW_C128 ? sizeof(double2) : sizeof(float2);
+  return ((size_t)nproj * (size_t)nb * elem + 255) & ~(size_t)255;
+}
+
+size_t position_gradient_bytes(int precision, int64_t npw, int64_t nproj, int64_t nb) {
+  if (npw <= 0 || nproj <= 0 || nb < 0) return 0;
+  return force_weighted_bytes(precision, nproj, nb) +
+         (size_t)3 * nproj * force_parts(precision, npw, nproj, nb) * sizeof(double);
+}
+
+template <typename T>
+static int force_product_t(int64_t npw, int64_t nproj, int64_t nb, const void* psi,
+                           int64_t ldpsi, const cplx<T>* fdo, const void* proj, int64_t ldproj,
+                           const double* q, double* partial, hipStream_t stream) {
+  const int variant =
+      force_variant(std::is_same<T, double>::value ? QEPW_C128 : QEPW_C64, npw, nproj, nb);
+  const GemmVariant& v = kVariants[variant];
+  const int64_t mt = (npw + v.tm - 1) / v.tm, nt = (nproj + v.tn - 1) / v.tn;
+  if (mt > 0x7fffffff / nt) return QEPW_ERR_UNSUPPORTED;
+  const dim3 grid((unsigned)(mt * nt));
+  const cplx<T>* x = static_cast<const cplx<T>*>(psi);
+  const cplx<T>* b = static_cast<const cplx<T>*>(proj);
+  if (variant == 0)
+    hipLaunchKernelGGL((k_force_product<T, 32, 32, 2>), grid, dim3(kGemmThreads), 0, stream, npw,
+                       nproj, nb, (unsigned)mt, (unsigned)nt, x, ldpsi, fdo, nproj, b, ldproj, q,
+                       partial);
+  else
+    hipLaunchKernelGGL((k_force_product<T, 64, 64, 2>), grid, dim3(kGemmThreads), 0, stream, npw,
+                       nproj, nb, (unsigned)mt, (unsigned)nt, x, ldpsi, fdo, nproj, b, ldproj, q,
+                       partial);
+  return hipGetLastError() == hipSuccess ? QEPW_OK : QEPW_ERR_HIP;
+}
+
+int position_gradient(int precision, int64_t npw, int64_t nproj, int nb, const void* psi,
+                      int64_t ldpsi, const void* coupled, int64_t ldc, const double* f,
+                      const void* proj, int64_t ldproj, const double* q, const int* off,
+                      int natom, double* out, void* ws, size_t ws_bytes, hipStream_t stream) {
+  if (precision != QEPW_C128 && precision != QEPW_C64) return QEPW_ERR_ARG;
+  if (natom <= 0) return QEPW_OK;
+  if (natom > 0x7fffffff / 3) return QEPW_ERR_UNSUPPORTED;
+  if (ws_bytes < position_gradient_bytes(precision, npw, nproj, nb)) return QEPW_ERR_WORKSPACE;
+  double* partial = nullptr;
+  int64_t parts = 0;
+  if (npw > 0 && nproj > 0) {
+    parts = force_parts(precision, npw, nproj, nb);
+    partial = reinterpret_cast<double*>(static_cast<char*>(ws) +
+                                        force_weighted_bytes(precision, nproj, nb));
+    int rc = scale_rows(precision, coupled, ldc, nullptr, 0, f, ws, nproj, nproj, nb, stream);
+    if (rc != QEPW_OK) return rc;
+    rc = precision == QEPW_C128
+             ? force_product_t<double>(npw, nproj, nb, psi, ldpsi, static_cast<double2*>(ws),
+                                       proj, ldproj, q, partial, stream)
+             : force_product_t<float>(npw, nproj, nb, psi, ldpsi, static_cast<float2*>(ws), proj,
+                                      ldproj, q, partial, stream);
+    if (rc != QEPW_OK) return rc;
+  }
+  hipLaunchKernelGGL(k_force_sum, dim3((unsigned)natom, 3), dim3(1024), 0, stream, partial, nproj,
+                     parts, off, out);
+  return hipGetLastError() == hipSuccess ? QEPW_OK : QEPW_ERR_HIP;
 }
 
 // Products of commuting Hermitian matrices (the Newton-Schulz steps of the

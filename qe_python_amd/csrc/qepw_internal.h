@@ -76,6 +76,11 @@ int gemm_plan(int precision, int op_a, int64_t m, int64_t n, int64_t k, int64_t*
 int gemm(int precision, int op_a, int64_t m, int64_t n, int64_t k, const double* alpha,
          const void* a, int64_t lda, const void* b, int64_t ldb, const double* beta,
          void* c, int64_t ldc, void* workspace, size_t ws_bytes, hipStream_t stream);
+size_t position_gradient_bytes(int precision, int64_t npw, int64_t nproj, int64_t nb);
+int position_gradient(int precision, int64_t npw, int64_t nproj, int nb, const void* psi,
+                      int64_t ldpsi, const void* coupled, int64_t ldc, const double* f,
+                      const void* proj, int64_t ldproj, const double* q, const int* off,
+                      int natom, double* out, void* ws, size_t ws_bytes, hipStream_t stream);
 int herm_product(int n, const void* x, const void* y, const void* d, void* c, int64_t ld,
                  double alpha, double beta, hipStream_t stream);
 

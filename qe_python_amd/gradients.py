@@ -11,11 +11,13 @@ with the gradients
 * dE/dtau_a,c = 2 sum_n f_n Re sum_{i in a} conj(dO_c[i,n]) (D O)[i,n],
   O = B^H psi, dO_c = i B^H ((k+G)_c psi) -- the force branch of
   ``_nonlocal_derivatives`` (``qepy_pw/pw/scf.py:1521-1631``) with the
-  projectors recomputed from tau on the device instead of storing dB/dtau.
+  projectors recomputed from tau on the device instead of storing dB/dtau, and
+  summed over the bands first: 2 sum_G (k+G)_c sum_{i in a} Im(B conj(W))_Gi,
+  W = psi f (D O)^H, one product instead of one per direction.
 
 Everything runs through ``libqepw_hip.so`` (``qepw_apply_local``,
 ``qepw_gemm``, ``qepw_accumulate_density``, ``qepw_build_projectors``,
-``qepw_scale_rows``, ``qepw_projector_forces``); ``band_energy`` wraps the
+``qepw_scale_rows``, ``qepw_position_gradient``); ``band_energy`` wraps the
 forward and backward in a ``torch.autograd.Function``.  Both complex128 and
 complex64 storage are supported (FP64 accumulation of every reduction).
 """
@@ -118,18 +120,16 @@ class BandEnergyModel:
         """dE/dtau (natom, 3) float64."""
         nb = psi.shape[0]
         p = proj.shape[0]
-        scaled = torch.empty_like(psi)
-        d_overlap = torch.empty((3, nb, p), dtype=psi.dtype, device=self.device)
-        for c in range(3):
-            self.scale_rows(psi, scaled, s=self.gk[:, c], sstride=3)
-            dv.gemm(nat.OP_C, p, nb, self.npw, 1j, proj, scaled, 0.0, d_overlap[c],
-                    self.workspace)
+        lib = nat.load()
+        prec = dv.precision_code(psi.dtype)
         out = torch.empty((self.natom, 3), dtype=torch.float64, device=self.device)
-        rc = nat.load().qepw_projector_forces(
-            dv.precision_code(psi.dtype), d_overlap.data_ptr(), p, nb * p,
-            coupled.data_ptr(), dv.ld_of(coupled), weights.data_ptr(), nb,
-            self.offsets.data_ptr(), self.natom, out.data_ptr(), dv.stream_handle(self.device))
-        nat.check(rc, "qepw_projector_forces")
+        buf = self.workspace.get(lib.qepw_position_gradient_workspace(prec, self.npw, p, nb))
+        rc = lib.qepw_position_gradient(
+            prec, psi.data_ptr(), dv.ld_of(psi), nb, proj.data_ptr(), dv.ld_of(proj), p,
+            coupled.data_ptr(), dv.ld_of(coupled), weights.data_ptr(), self.gk.data_ptr(),
+            self.npw, self.offsets.data_ptr(), self.natom, out.data_ptr(), buf.data_ptr(),
+            buf.numel(), dv.stream_handle(self.device))
+        nat.check(rc, "qepw_position_gradient")
         return out
 
 

@@ -172,6 +172,53 @@ def test_medium_workload_central_differences():
     assert g32 == pytest.approx(fd, rel=1e-4)
 
 
+@pytest.mark.parametrize("dtype,tol", [(torch.complex128, 1e-12), (torch.complex64, 2e-5)])
+@pytest.mark.parametrize("npw,nch,natom,nb", [
+    (1, 1, 1, 1), (31, 1, 3, 2), (65, 8, 4, 15), (200, 11, 3, 17), (1030, 18, 8, 33),
+    (777, 13, 5, 0)])
+def test_position_gradient_at_tile_edges(dtype, tol, npw, nch, natom, nb):
+    """qepw_position_gradient (one product over the bands) against the sums
+    over dO_c = i B^H (q_c psi) in NumPy: one projector, either side of the 32
+    projectors where the tile changes, ragged rows, bands and projectors."""
+    from qe_python_amd import _native as nat
+    from qe_python_amd import device as dv
+    lib = nat.load()
+    rng = np.random.default_rng(npw + nb)
+    p = nch * natom
+
+    def block(rows, cols):
+        return rng.standard_normal((rows, cols)) + 1j * rng.standard_normal((rows, cols))
+    psi, proj, coupled = block(npw, nb), block(npw, p), block(p, nb)
+    q, f = rng.standard_normal((npw, 3)), rng.standard_normal(nb)
+    dev = [torch.from_numpy(np.ascontiguousarray(x.T)).to(DEV).to(dtype)
+           for x in (psi, proj, coupled)]
+    # the operands as stored (rounded to the block's precision)
+    psi, proj, coupled = (x.cpu().numpy().astype(complex).T for x in dev)
+    qd, fd = torch.from_numpy(q).to(DEV), torch.from_numpy(f).to(DEV)
+    off = torch.arange(0, p + 1, nch, dtype=torch.int32, device=DEV)
+    out = torch.full((natom, 3), float("nan"), dtype=torch.float64, device=DEV)
+    prec = dv.precision_code(dtype)
+    need = lib.qepw_position_gradient_workspace(prec, npw, p, nb)
+    ws = torch.empty(need, dtype=torch.uint8, device=DEV)
+
+    def call(size):
+        return lib.qepw_position_gradient(
+            prec, dev[0].data_ptr(), npw, nb, dev[1].data_ptr(), npw, p, dev[2].data_ptr(), p,
+            fd.data_ptr(), qd.data_ptr(), npw, off.data_ptr(), natom, out.data_ptr(),
+            ws.data_ptr(), size, dv.stream_handle(torch.device(DEV)))
+    with pytest.raises(Exception):
+        nat.check(call(need - 1), "short workspace")
+    nat.check(call(need), "qepw_position_gradient")
+    ref = np.empty((natom, 3))
+    for c in range(3):
+        d = 1j * proj.conj().T @ (q[:, c, None] * psi)
+        t = 2.0 * ((d.conj() * coupled).real @ f)
+        ref[:, c] = t.reshape(natom, nch).sum(1)
+    # rounding grows with the terms, which may cancel in one force
+    scale = max(np.linalg.norm(ref), 2.0 * np.sqrt(2.0 * npw * p * max(nb, 1)) / 10)
+    assert np.linalg.norm(out.cpu().numpy() - ref) <= tol * scale
+
+
 def test_argument_errors(small):
     from qe_python_amd.gradients import band_energy
     s, psi, f, model, _ = small
