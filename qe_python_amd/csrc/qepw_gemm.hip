@@ -608,7 +608,9 @@ static double plan_cost(int precision, int variant, int64_t m, int64_t n, int64_
   return t;
 }
 
-static SplitPlan built_in_plan(int precision, int op_a, int64_t m, int64_t n, int64_t k) {
+// a plan that needs no search, and no more scratch than callers that size
+// theirs by other means than qepw_gemm_workspace provide
+static SplitPlan fixed_plan(int op_a, int64_t m, int64_t n, int64_t k) {
   if (m <= 0 || n <= 0 || k <= 0) return finish_plan(0, 1, k);
   const bool ca = (op_a & QEPW_OP_C) != 0;
   const bool tall = ca && k > 2048;
@@ -637,10 +639,15 @@ static SplitPlan built_in_plan(int precision, int op_a, int64_t m, int64_t n, in
     const int64_t most = k / (tall ? 256 : 128);
     splits = want < most ? want : most;
   }
-  const SplitPlan fixed = finish_plan(variant, splits, k);
+  return finish_plan(variant, splits, k);
+}
+
+static SplitPlan built_in_plan(int precision, int op_a, int64_t m, int64_t n, int64_t k) {
+  const SplitPlan fixed = fixed_plan(op_a, m, n, k);
+  if (m <= 0 || n <= 0 || k <= 0) return fixed;
   // partial tiles stay within the static scratch (qepw_gemm_static) where the
   // fixed choice's do, and within four times that where they do not: with the
-  // operands of 512 x 192 x 78 805 at 1.2 GB, 21 splits take 1.12 ms, 85 1.00
+  // operands of 512 x 192 x 78 805 at 1.2 GB, 21 splits take 1.12 ms, 32 1.02
   const int64_t out_bytes = m * n * (precision == QEPW_C128 ? 16 : 8);
   const int64_t scratch = (int64_t)QEPW_GEMM_STATIC_SCRATCH;
   const bool over = fixed.splits > 1 && fixed.splits > scratch / out_bytes;
@@ -975,11 +982,16 @@ static int gemm_t(int op, int64_t m, int64_t n, int64_t k, const double* alpha,
                   void* c, int64_t ldc, void* ws, size_t ws_bytes, hipStream_t stream) {
   if (n == 1 && k > 0)
     return gemv_t<T>(op, m, k, alpha, a, lda, b, ldb, beta, c, ldc, ws, ws_bytes, stream);
-  const SplitPlan sp = split_plan(std::is_same<T, double>::value ? QEPW_C128 : QEPW_C64,
+  SplitPlan sp = split_plan(std::is_same<T, double>::value ? QEPW_C128 : QEPW_C64,
                                   op & (QEPW_OP_C | QEPW_OP_BC), m, n, k);
+  const auto bytes = [&](const SplitPlan& p) {
+    return p.splits > 1 ? (size_t)p.splits * m * n * sizeof(cplx<T>) : 0;
+  };
+  // a workspace of fixed size (the Rayleigh-Ritz steps') that the searched
+  // plan exceeds and the fixed one does not
+  if (ws_bytes < bytes(sp) && bytes(sp) > QEPW_GEMM_STATIC_SCRATCH) sp = fixed_plan(op, m, n, k);
   if (sp.splits > 65535) return QEPW_ERR_UNSUPPORTED;
-  const size_t need = sp.splits > 1 ? (size_t)sp.splits * m * n * sizeof(cplx<T>) : 0;
-  if (ws_bytes < need) return QEPW_ERR_WORKSPACE;
+  if (ws_bytes < bytes(sp)) return QEPW_ERR_WORKSPACE;
   const GemmVariant gv = kVariants[sp.variant];
   const int64_t mt = (m + gv.tm - 1) / gv.tm, nt = (n + gv.tn - 1) / gv.tn;
   if (mt > 0x7fffffff || nt > 65535 || mt * nt > 0x7fffffff / sp.splits)

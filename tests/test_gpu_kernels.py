@@ -145,6 +145,35 @@ def test_gemm_chosen_plans_at_tile_and_step_edges(prec, op):
         assert err < tol, (m, n, k, list(plan), err)
 
 
+def test_gemm_in_a_workspace_of_fixed_size():
+    """A product whose planned partials exceed the static scratch runs in the
+    Rayleigh-Ritz steps' workspace with fewer splits; less than 21 splits of
+    320 x 320 (the choice that needs no search) is refused."""
+    from qe_python_amd import _native as nat
+    from qe_python_amd import device as dv
+    lib = nat.load()
+    m, k = 320, 24000
+    rng = np.random.default_rng(3)
+    a = rand(rng, k, m)
+    ta = dev_block(a, torch.complex128)
+    tc = dev_block(np.zeros((m, m), complex), torch.complex128)
+    ws = torch.empty(max(lib.qepw_rr_workspace(m), lib.qepw_gemm_workspace(
+        nat.C128, nat.OP_C, m, m, k)), dtype=torch.uint8, device=DEV)
+    import ctypes
+    one, zero = (ctypes.c_double * 2)(1.0, 0.0), (ctypes.c_double * 2)(0.0, 0.0)
+    ref = a.conj().T @ a
+    for size in (lib.qepw_gemm_workspace(nat.C128, nat.OP_C, m, m, k), 21 * m * m * 16):
+        nat.check(lib.qepw_gemm(nat.C128, nat.OP_C, m, m, k, one, ta.data_ptr(), k,
+                                ta.data_ptr(), k, zero, tc.data_ptr(), m, ws.data_ptr(), size,
+                                dv.stream_handle(torch.device(DEV))), "qepw_gemm")
+        err = np.linalg.norm(host_block(tc) - ref) / np.linalg.norm(ref)
+        assert err < 1e-12, (size, err)
+    with pytest.raises(Exception):
+        nat.check(lib.qepw_gemm(nat.C128, nat.OP_C, m, m, k, one, ta.data_ptr(), k,
+                                ta.data_ptr(), k, zero, tc.data_ptr(), m, ws.data_ptr(),
+                                12 * m * m * 16, dv.stream_handle(torch.device(DEV))), "short")
+
+
 def test_gemm_split_k_is_deterministic():
     from qe_python_amd import _native as nat
     from qe_python_amd import device as dv
