@@ -285,6 +285,8 @@ static int plan_create_impl(const int32_t* miller, int64_t npw, int n1, int n2, 
   }
   p.sphere.plane64 = qepw::plane_choice<double>(p, p.sphere);
   p.sphere.plane32 = qepw::plane_choice<float>(p, p.sphere);
+  p.sphere.density64 = qepw::density_choice<double>(p, p.sphere);
+  p.sphere.density32 = qepw::density_choice<float>(p, p.sphere);
   *out = plan;
   return QEPW_OK;
 }

@@ -312,9 +312,6 @@ template <int N> struct TeamGeom {
   static constexpr int M = N / L;
   static constexpr int per_wave = 64 / M;
   static constexpr int teams = (kTeamThreads / 64) * per_wave;
-  // input slots kept by the pruned kernel: the first two and the last two
-  static constexpr unsigned all = (1u << L) - 1u;
-  static constexpr unsigned pruned = L >= 6 ? (0x3u | (0x3u << (L - 2))) : all;
 };
 
 // Slots of the team FFT of length n that hold any of the positions (bit s:
@@ -488,7 +485,7 @@ __global__ __launch_bounds__(kTeamThreads) void k_sticks_group(const StickGroupA
   }
 }
 
-// z lengths and density plane sides with a team kernel.
+// z lengths with a team kernel.
 #define QEPW_LINE_SIZES(X) \
   X(16) X(18) X(20) X(24) X(25) X(27) X(30) X(32) X(36) X(40) X(45) X(48) X(50) X(54) \
   X(60) X(64) X(72) X(75) X(80) X(81) X(90) X(96) X(100) X(108) X(120)
@@ -500,18 +497,6 @@ static int team_teams(int n) {
   QEPW_LINE_SIZES(QEPW_TEAMS_N)
 #undef QEPW_TEAMS_N
   return teams;
-}
-
-template <typename T>
-static size_t team_lds_bytes(int n, int nxc) {
-  size_t teams = 0;
-#define QEPW_TEAMS_OF(NN) if (n == NN) teams = TeamGeom<NN>::teams;
-  QEPW_LINE_SIZES(QEPW_TEAMS_OF)
-#undef QEPW_TEAMS_OF
-  // no team kernel for this length: the generic kernels run
-  if (teams == 0) return 0;
-  // active columns, the zero column of k_planes_team, one scratch line per team
-  return ((size_t)nxc + 1 + teams) * (size_t)(n + 1) * sizeof(cplx<T>);
 }
 
 // Launches the team z-stage kernel for n3 if one exists; false otherwise.
@@ -773,133 +758,10 @@ int apply_local_group(int count, const Plan* const* plans, int precision,
 // backward FFT (reference: accumulate_density_serial, _native_fft.pyx:
 // 2592-2648).  The backward z stage is apply_local's (the team kernel where
 // n3 has one, k_sticks_inverse otherwise); the plane stage
-// loops over a fixed slice of bands inside each workgroup and accumulates in
-// LDS / registers, writing one partial plane per (slice, z); a last kernel
-// sums the slices in a fixed order.  No atomics: results are reproducible.
-
-template <typename T, int N, bool PRUNE>
-__global__ __launch_bounds__(kTeamThreads) void k_density_team(
-    const cplx<T>* __restrict__ work, int64_t band_stride, int nst,
-    const int* __restrict__ colpos, const int* __restrict__ colmap, int nxc, int nb,
-    int bands_per_slice, const double* __restrict__ weights, double* __restrict__ partial,
-    int accumulate, const cplx<T>* __restrict__ tw) {
-  using G = TeamGeom<N>;
-  constexpr int L = G::L, M = G::M;
-  constexpr unsigned KEEP = PRUNE ? G::pruned : G::all;
-  // rows of a team: y = team + r * teams, r < R; each lane keeps the density
-  // of its outputs x = t + L k of those rows in registers across the bands
-  constexpr int R = (N + G::teams - 1) / G::teams;
-  extern __shared__ unsigned char smem_raw[];
-  constexpr int NP = N + 1;  // padded column stride and zero column, as in k_planes_team
-  cplx<T>* Q = reinterpret_cast<cplx<T>*>(smem_raw);
-  cplx<T>* scratch_all = Q + (nxc + 1) * NP;
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
-  const int team_in_wave = lane / M;
-  const int t = lane - team_in_wave * M;
-  const bool in_team = team_in_wave < G::per_wave;
-  const int team = wave * G::per_wave + team_in_wave;
-  cplx<T>* S = scratch_all + team * NP;
-  const int z = blockIdx.x;
-  const int slice = blockIdx.y;
-  const int b0 = slice * bands_per_slice;
-  const int b1 = min(nb, b0 + bands_per_slice);
-  const cplx<T> zero = mk<T>(T(0), T(0));
-  TeamTwiddles<T, N> twr;
-  twr.load(t, tw);
-  int cq[L];
-#pragma unroll
-  for (int s = 0; s < L; ++s) {
-    const int c = (t < M && ((KEEP >> s) & 1u)) ? colmap[t + M * s] : -1;
-    cq[s] = (c < 0 ? nxc : c) * NP;
-  }
-  double acc[R][M];
-#pragma unroll
-  for (int r = 0; r < R; ++r)
-#pragma unroll
-    for (int k = 0; k < M; ++k) acc[r][k] = 0.0;
-  // the zero column, read by the row pass at the inactive x positions (the
-  // column pass below never writes it; its closing barrier orders this)
-  for (int i = tid; i < NP; i += kTeamThreads) Q[nxc * NP + i] = zero;
-  for (int b = b0; b < b1; ++b) {
-    const cplx<T>* w = work + (int64_t)b * band_stride + (int64_t)z * nst;
-    const double wb = weights[b];
-    // backward y-FFT of every active column, its inputs read straight from
-    // the stick buffer (colpos: the stick at (c, y), or -1; every position of
-    // a column first, then every stick load), its outputs written to the
-    // column
-    if (in_team) {
-      for (int c = team; c < nxc; c += G::teams) {
-        if (c != team) wave_lds_sync();
-        cplx<T>* col = Q + c * NP;
-        const int* pos = colpos + c * N;
-        cplx<T> bb[L], a[M];
-        if (t < M) {
-          int st[L];
-#pragma unroll
-          for (int s = 0; s < L; ++s) st[s] = ((KEEP >> s) & 1u) ? pos[t + M * s] : -1;
-#pragma unroll
-          for (int s = 0; s < L; ++s) {
-            bb[s] = zero;
-            if ((KEEP >> s) & 1u) {
-              const cplx<T> v = w[st[s] >= 0 ? st[s] : 0];
-              bb[s] = st[s] >= 0 ? v : zero;
-            }
-          }
-        }
-        dif_front<T, N, +1>(t, S, twr, bb);
-        wave_lds_sync();
-        dif_back<T, N, +1>(t, S, a);
-        if (t < L) {
-#pragma unroll
-          for (int k = 0; k < M; ++k) col[t + L * k] = a[k];
-        }
-      }
-    }
-    __syncthreads();
-    // backward x-FFT of this team's rows, |psi|^2 accumulated in registers
-    if (in_team) {
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const int y = team + r * G::teams;
-        if (y < N) {
-          if (r > 0) wave_lds_sync();
-          cplx<T> bb[L], a[M];
-          if (t < M) {
-#pragma unroll
-            for (int s = 0; s < L; ++s)
-              bb[s] = ((KEEP >> s) & 1u) ? Q[cq[s] + y] : zero;
-          }
-          dif_front<T, N, +1>(t, S, twr, bb);
-          wave_lds_sync();
-          dif_back<T, N, +1>(t, S, a);
-          if (t < L) {
-#pragma unroll
-            for (int k = 0; k < M; ++k)
-              acc[r][k] += wb * ((double)a[k].x * (double)a[k].x +
-                                 (double)a[k].y * (double)a[k].y);
-          }
-        }
-      }
-    }
-    __syncthreads();
-  }
-  // (y, x) of the plane, (n3, n2, n1) layout: one writer per element
-  double* out = partial + ((int64_t)slice * gridDim.x + z) * N * N;
-  if (in_team && t < L) {
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int y = team + r * G::teams;
-      if (y < N) {
-#pragma unroll
-        for (int k = 0; k < M; ++k) {
-          const int i = y * N + t + L * k;
-          out[i] = (accumulate ? out[i] : 0.0) + acc[r][k];
-        }
-      }
-    }
-  }
-}
+// (qepw_plane.h; the kernels below where it does not serve the plan) loops
+// over a fixed slice of bands inside each workgroup and accumulates in
+// registers, writing one partial plane per (slice, z); a last kernel sums the
+// slices in a fixed order.  No atomics: results are reproducible.
 
 template <typename T>
 __global__ __launch_bounds__(kPlaneThreads) void k_density_plane(
@@ -1026,12 +888,6 @@ size_t density_workspace_bytes(const Plan& p, int precision, int nb) {
 }
 
 template <typename T>
-static size_t density_team_lds(int n, int nxc) {
-  // the density accumulates in registers: the plane kernel's LDS
-  return team_lds_bytes<T>(n, nxc);
-}
-
-template <typename T>
 int accumulate_density_t(const Plan& p, const void* vectors, int64_t ldv, int nb,
                          const double* weights, double scale, double* out, void* workspace,
                          size_t ws_bytes, hipStream_t stream) {
@@ -1040,9 +896,7 @@ int accumulate_density_t(const Plan& p, const void* vectors, int64_t ldv, int nb
   const size_t np = (size_t)p.n1 * p.n2;
   if (st.group * p.n3 > lds_fft_capacity(p.line[2], kStickThreads, kStickPts))
     return QEPW_ERR_UNSUPPORTED;
-  const size_t team_lds =
-      (p.n1 == p.n2 && st.d_colpos && st.d_colmap) ? density_team_lds<T>(p.n1, st.nxcols) : 0;
-  const bool team = team_lds > 0 && team_lds <= (size_t)kMaxLdsBytes;
+  const bool team = (sizeof(T) == 8 ? st.density64 : st.density32).waves > 0;
   // planes that neither the team kernel nor one workgroup's LDS can hold go
   // through the split stage's column lines, as in apply_local
   const bool split = !team && !generic_plane_fits<T>(p) && split_available<T>(p, st);
@@ -1080,6 +934,7 @@ int accumulate_density_t(const Plan& p, const void* vectors, int64_t ldv, int nb
                        stream, partial, 0, (int64_t)ngrid, scale, out);
     return hipGetLastError() == hipSuccess ? QEPW_OK : QEPW_ERR_HIP;
   }
+  int slices = 0;
   for (int b0 = 0; b0 < nb; b0 += chunk) {
     const int nbc = (nb - b0) < chunk ? (nb - b0) : chunk;
     const cplx<T>* src = static_cast<const cplx<T>*>(vectors) + (int64_t)b0 * ldv;
@@ -1089,36 +944,22 @@ int accumulate_density_t(const Plan& p, const void* vectors, int64_t ldv, int nb
       hipLaunchKernelGGL(k_sticks_inverse<T>, dim3(st.ngroups, nbc), dim3(kStickThreads),
                          stick_lds, stream, src, ldv, work, bstride, st.nst, p.n3, st.d_off,
                          st.d_gpos, st.group, p.line[2], twiddles<T>(p, 2));
-    const int per = (nbc + kDensitySlices - 1) / kDensitySlices;
-    const dim3 grid(p.n3, kDensitySlices);
-    const int acc = b0 > 0 ? 1 : 0;
     bool launched = false;
-    if (team) {
-#define QEPW_LAUNCH_DENSITY_K(NN, PR)                                                        \
-  do {                                                                                       \
-    allow_lds(reinterpret_cast<const void*>(&k_density_team<T, NN, PR>), team_lds);          \
-    hipLaunchKernelGGL((k_density_team<T, NN, PR>), grid, dim3(kTeamThreads), team_lds,     \
-                       stream, work, bstride, st.nst, st.d_colpos, st.d_colmap, st.nxcols,  \
-                       nbc, per, weights + b0, partial, acc, twiddles<T>(p, 0));             \
-  } while (0)
-#define QEPW_LAUNCH_DENSITY(NN)                                                              \
-  if (!launched && p.n1 == NN) {                                                             \
-    if (((st.xmask | st.ymask) & ~TeamGeom<NN>::pruned) == 0u)                                        \
-      QEPW_LAUNCH_DENSITY_K(NN, true);                                                       \
-    else                                                                                     \
-      QEPW_LAUNCH_DENSITY_K(NN, false);                                                      \
-    launched = true;                                                                         \
-  }
-      QEPW_LINE_SIZES(QEPW_LAUNCH_DENSITY)
-#undef QEPW_LAUNCH_DENSITY
-#undef QEPW_LAUNCH_DENSITY_K
-    }
+    if (team)
+      launched = launch_density_stage<T>(p, st, work, bstride, weights + b0, nbc, kDensitySlices,
+                                         &slices, b0 > 0, partial, stream);
+    // (the first chunk, the largest, sets the slices of all)
+    else if (slices == 0)
+      slices = std::min(kDensitySlices, nbc);
+    const int per = (nbc + slices - 1) / slices;
+    const dim3 grid(p.n3, slices);
+    const int acc = b0 > 0 ? 1 : 0;
     if (!launched && split) {
       const dim3 gcols((unsigned)((st.nxcols + gc - 1) / gc), (unsigned)p.n3, (unsigned)nbc);
       hipLaunchKernelGGL(k_split_cols_inverse<T>, gcols, dim3(kSplitThreads), lc, stream, work,
                          bstride, st.nst, st.d_colstart, st.d_stickq, st.nxcols, p.n2, tbuf,
                          tband, gc, p.line[1], twiddles<T>(p, 1));
-      const dim3 grows((unsigned)((p.n2 + gr - 1) / gr), (unsigned)p.n3, kDensitySlices);
+      const dim3 grows((unsigned)((p.n2 + gr - 1) / gr), (unsigned)p.n3, (unsigned)slices);
       hipLaunchKernelGGL(k_split_rows_density<T>, grows, dim3(kSplitThreads), lr, stream, tbuf,
                          tband, st.d_xcols, st.nxcols, p.n1, p.n2, p.n3, nbc, per, weights + b0,
                          partial, acc, gr, p.line[0], twiddles<T>(p, 0));
@@ -1131,7 +972,7 @@ int accumulate_density_t(const Plan& p, const void* vectors, int64_t ldv, int nb
                          twiddles<T>(p, 0), twiddles<T>(p, 1));
   }
   hipLaunchKernelGGL(k_sum_slices, dim3((unsigned)((ngrid + 255) / 256)), dim3(256), 0, stream,
-                     partial, kDensitySlices, (int64_t)ngrid, scale, out);
+                     partial, slices, (int64_t)ngrid, scale, out);
   return hipGetLastError() == hipSuccess ? QEPW_OK : QEPW_ERR_HIP;
 }
 

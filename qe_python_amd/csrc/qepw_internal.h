@@ -62,6 +62,11 @@ template <typename T> PlaneChoice plane_choice(const Plan& p, const StickTables&
 template <typename T>
 bool launch_plane_stage(const Plan& p, const StickTables& st, cplx<T>* work, int64_t bstride,
                         const T* V, int nb, hipStream_t stream);
+template <typename T> PlaneChoice density_choice(const Plan& p, const StickTables& st);
+template <typename T>
+bool launch_density_stage(const Plan& p, const StickTables& st, cplx<T>* work, int64_t bstride,
+                          const double* weights, int nb, int most, int* slices, bool accumulate,
+                          double* partial, hipStream_t stream);
 template <typename T>
 int launch_plane_group(int count, const Plan* const* plans, cplx<T>* const* work,
                        const int64_t* bstride, const T* const* V, const int* nb,

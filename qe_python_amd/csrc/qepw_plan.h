@@ -24,6 +24,8 @@ namespace qepw {
 struct PlaneChoice {
   int waves = 0;
   bool square = false, prune = false;
+  int hold = 0;         // density: workgroups of a CU
+  bool direct = false;  // density: the rows' exchange lines lie behind the columns
   size_t lds = 0;
 };
 
@@ -45,6 +47,7 @@ struct StickTables {
   unsigned xmask = 0;       // team-FFT input slots holding an active x
   unsigned ymask = 0;       // ... a stick's y
   PlaneChoice plane64, plane32;
+  PlaneChoice density64, density32;  // the density's
 };
 
 struct Plan {

@@ -82,8 +82,8 @@ template <typename T, int N> struct PlaneTwiddles<T, N, true> {
 // Backward (DIF) and forward (DIT) team FFTs of one line through its LDS line
 // S, split as in qepw_regfft.h: b, slots t + M s of lanes t < M; a, slots
 // t + L k of lanes t < L.
-template <typename T, int N>
-__device__ __forceinline__ void plane_backward(int t, cplx<T>* S, PlaneTwiddles<T, N>& tw,
+template <typename T, int N, typename TW>
+__device__ __forceinline__ void plane_backward(int t, cplx<T>* S, TW& tw,
                                                cplx<T> (&b)[PlaneLine<N>::L],
                                                cplx<T> (&a)[PlaneLine<N>::M]) {
   constexpr int L = PlaneLine<N>::L, M = PlaneLine<N>::M;
@@ -139,8 +139,8 @@ template <typename T> struct PlaneArgs {
 template <int N> struct PlaneLane {
   int t, team;
   bool on;
-  __device__ __forceinline__ PlaneLane() {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  __device__ __forceinline__ explicit PlaneLane(int tid = threadIdx.x) {
+    const int lane = tid & 63, wave = tid >> 6;
     const int i = lane / PlaneLine<N>::M;
     t = lane - i * PlaneLine<N>::M;
     on = i < PlaneLine<N>::per_wave;
@@ -151,17 +151,18 @@ template <int N> struct PlaneLane {
 // Backward y-FFT of every occupied column, in place in LDS: the column is the
 // team's exchange line.  Column nxc is zeroed: the row pass reads the
 // unoccupied x positions from it (and writes their discarded outputs to it).
-template <typename T, int N2, bool PRUNE>
+template <typename T, int N2, bool PRUNE, bool ZERO = true, typename TW>
 __device__ __forceinline__ void plane_cols_backward(const PlaneArgs<T>& g, const cplx<T>* w,
-                                                    cplx<T>* Q, int waves,
-                                                    PlaneTwiddles<T, N2>& tw) {
+                                                    cplx<T>* Q, int waves, TW& tw,
+                                                    int tid = threadIdx.x) {
   using G = PlaneLine<N2>;
   constexpr int L = G::L, M = G::M, NP = N2 + 1;
   constexpr unsigned KEEP = PRUNE ? G::pruned : G::all;
-  const PlaneLane<N2> ln;
+  const PlaneLane<N2> ln(tid);
   const int t = ln.t;
   const cplx<T> zero = mk<T>(T(0), T(0));
-  for (int i = threadIdx.x; i < NP; i += waves * 64) Q[g.nxc * NP + i] = zero;
+  if (ZERO)
+    for (int i = tid; i < NP; i += waves * 64) Q[g.nxc * NP + i] = zero;
   if (!ln.on) return;
   for (int c = ln.team; c < g.nxc; c += waves * G::per_wave) {
     cplx<T>* col = Q + c * NP;
@@ -197,10 +198,11 @@ __device__ __forceinline__ void plane_cols_backward(const PlaneArgs<T>& g, const
 // or the zero column's.  The same for every row of the plane.
 template <typename T, int N1, bool PRUNE>
 __device__ __forceinline__ void plane_row_slots(const PlaneArgs<T>& g, int np2,
-                                                int (&cq)[PlaneLine<N1>::L]) {
+                                                int (&cq)[PlaneLine<N1>::L],
+                                                int tid = threadIdx.x) {
   using G = PlaneLine<N1>;
   constexpr unsigned KEEP = PRUNE ? G::pruned : G::all;
-  const PlaneLane<N1> ln;
+  const PlaneLane<N1> ln(tid);
 #pragma unroll
   for (int s = 0; s < G::L; ++s) {
     const int c =
@@ -474,8 +476,232 @@ __global__ __launch_bounds__(64 * plane_group_waves<T>(), 3) void k_plane_group(
   }
 }
 
+// ---- density ----------------------------------------------------------------------
+// rho(r) += w_b |psi_b(r)|^2 over the bands of a slice: the backward half of the
+// plane stage, with each lane's outputs x = t + L k of its rows accumulated in
+// registers over the bands (FP64) and written once to the slice's partial plane.
+// Bound by the chain of each band (sticks, two FFT passes, two barriers) at the
+// waves that its registers and LDS leave a CU, eight to twelve.  Whole density of
+// 128 bands (or as many as 3e8 bytes of sticks hold), against a team kernel for
+// squares up to 120 and the Stockham and split stages for all else, in FP64 and
+// FP32, us: 36^2 44 / 34 as before, 60^2 145 / 104 -> 140 / 95, 72^2 189 / 122 ->
+// 173 / 119, 75^2 498 / 275 -> 397 / 244, 80^2 352 / 162 -> 342 / 152, 90^2 as
+// before, 96^2 566 / 290 -> 493 / 268, 120^2 663 / 332 -> 566 / 235, 128^2 1624 /
+// 1318 -> 795 / 495, 48 x 60 x 80 816 / 615 -> 188 / 102, 36 x 40 x 160 952 / 770
+// -> 272 / 153, 72 x 75 x 90 1707 / 1294 -> 943 / 370, 108 x 120 x 60 1835 / 1547
+// -> 1374 / 385.
+template <typename T> struct DensityArgs {
+  PlaneArgs<T> plane;   // V unused
+  int nb, per;          // bands, bands of a slice
+  int accumulate;       // add to the partial planes of an earlier chunk of bands
+  const double* weights;
+  double* partial;      // (slice, n3, n2, n1)
+};
+
+// Rows, RB per team, of one band; called by the whole workgroup (it
+// synchronises, and leaves the LDS free).  DIRECT: row by row through exchange
+// lines of their own behind the columns (Q + own), for planes whose LDS then
+// still leaves two workgroups a CU; else as in plane_rows, the rows read first
+// and the plane's storage reused.
+template <typename T, int N1, bool PRUNE, int RB, bool DIRECT, int A, typename TW>
+__device__ __forceinline__ void density_rows(cplx<T>* Q, int own, int n2, int waves, TW& tw,
+                                             const int (&cq)[PlaneLine<N1>::L], double wb,
+                                             double (&acc)[A], int tid = threadIdx.x) {
+  using G = PlaneLine<N1>;
+  constexpr int L = G::L, M = G::M, NP = N1 + 1;
+  constexpr unsigned KEEP = PRUNE ? G::pruned : G::all;
+  static_assert(RB * M <= A, "accumulators");
+  const PlaneLane<N1> ln(tid);
+  const int t = ln.t, team = ln.team, teams = waves * G::per_wave;
+  const cplx<T> zero = mk<T>(T(0), T(0));
+  cplx<T>* E = Q + (DIRECT ? own : 0) + team * NP;
+  cplx<T> rows[DIRECT ? 1 : RB][L];
+  auto read = [&](int r, int y) __attribute__((always_inline)) {
+    if (t < M) {
+#pragma unroll
+      for (int s = 0; s < L; ++s) rows[r][s] = ((KEEP >> s) & 1u) ? Q[cq[s] + y] : zero;
+    }
+  };
+  if constexpr (!DIRECT) {
+#pragma unroll
+    for (int r = 0; r < RB; ++r)
+      if (ln.on && team + r * teams < n2) read(r, team + r * teams);
+    __syncthreads();
+  }
+  if (ln.on) {
+#pragma unroll
+    for (int r = 0; r < RB; ++r) {
+      const int y = team + r * teams;
+      if (y < n2) {
+        cplx<T> a[M];
+        if (DIRECT) read(0, y);
+        if (r > 0) wave_lds_sync();  // the line is read across lanes above
+        plane_backward<T, N1>(t, E, tw, rows[DIRECT ? 0 : r], a);
+        if (t < L) {
+#pragma unroll
+          for (int k = 0; k < M; ++k)
+            acc[r * M + k] =
+                fma(wb, fma((double)a[k].x, (double)a[k].x, (double)a[k].y * (double)a[k].y),
+                    acc[r * M + k]);
+        }
+      }
+    }
+  }
+  __syncthreads();
+}
+
+template <typename T, int N1, int RB, int A>
+__device__ __forceinline__ void density_store(const DensityArgs<T>& d, int z, int slice, int waves,
+                                              const double (&acc)[A]) {
+  using G = PlaneLine<N1>;
+  const PlaneLane<N1> ln;
+  const int n2 = d.plane.n2;
+  double* out = d.partial + ((int64_t)slice * gridDim.x + z) * n2 * N1;
+  if (!ln.on || ln.t >= G::L) return;
+#pragma unroll
+  for (int r = 0; r < RB; ++r) {
+    const int y = ln.team + r * waves * G::per_wave;
+    if (y < n2) {
+#pragma unroll
+      for (int k = 0; k < G::M; ++k) {
+        const int i = y * N1 + ln.t + G::L * k;
+        out[i] = (d.accumulate ? out[i] : 0.0) + acc[r * G::M + k];
+      }
+    }
+  }
+}
+
+// Whether the square kernel's rows have exchange lines of their own.
+template <typename T> constexpr bool density_direct(int n, bool prune) {
+  return sizeof(T) == 8 ? n <= 72 || (prune && (n == 80 || n == 81 || n == 90)) : n <= 54;
+}
+
+// Whether the square kernel holds the twiddles of a line that the plane stage
+// loads (60^2, 128 bands: 154 us loaded, 144 held).
+template <typename T> constexpr bool density_held(int n) { return sizeof(T) == 8 && n <= 72; }
+
+// Waves of the square kernel's workgroup.
+template <typename T, int N, bool PRUNE> constexpr int density_waves() {
+  constexpr bool direct = density_direct<T>(N, PRUNE);
+  int w = N <= 72 ? 4 : direct || (N <= 80 && N != 75) ? 8 : 12;
+  while (w < 16) {
+    const int teams = w * PlaneLine<N>::per_wave;
+    const int rows = (N + teams - 1) / teams;
+    const int held = direct ? 0 : rows * plane_kept<N, PRUNE>();
+    if (rows * PlaneLine<N>::M <= 32 && held <= plane_row_budget<T>()) break;
+    w += 4;
+  }
+  return w;
+}
+
+// Waves a SIMD that its registers are bounded for: 72^2 in FP64 spills in three
+// waves' (128 bands: 234 us with three, 176 with two).
+template <typename T, int N, bool PRUNE> constexpr int density_simd_waves() {
+  constexpr int W = density_waves<T, N, PRUNE>();
+  return W > 12 ? 4 : sizeof(T) == 8 && N >= 60 && density_direct<T>(N, PRUNE) ? 2 : 3;
+}
+
+template <typename T, int N, bool PRUNE, int W>
+__global__ __launch_bounds__(64 * W, (density_simd_waves<T, N, PRUNE>())) void k_density_square(DensityArgs<T> d) {
+  extern __shared__ unsigned char smem_raw[];
+  cplx<T>* Q = reinterpret_cast<cplx<T>*>(smem_raw);
+  constexpr int teams = W * PlaneLine<N>::per_wave, RB = (N + teams - 1) / teams;
+  constexpr int A = RB * PlaneLine<N>::M;
+  const PlaneArgs<T>& g = d.plane;
+  const int z = blockIdx.x, b0 = blockIdx.y * d.per, b1 = min(d.nb, b0 + d.per);
+  PlaneTwiddles<T, N, !density_held<T>(N) && plane_lane_table(N, sizeof(T) == 8)> tw;
+  tw.load(PlaneLane<N>().t, g.tw1);
+  int cq[PlaneLine<N>::L];
+  plane_row_slots<T, N, PRUNE>(g, N + 1, cq);
+  double acc[A];
+#pragma unroll
+  for (int k = 0; k < A; ++k) acc[k] = 0.0;
+  constexpr bool DIRECT = density_direct<T>(N, PRUNE);
+  if (DIRECT)  // nothing overwrites the zero column
+    for (int i = threadIdx.x; i <= N; i += W * 64) Q[g.nxc * (N + 1) + i] = mk<T>(T(0), T(0));
+  for (int b = b0; b < b1; ++b) {
+    const cplx<T>* w = g.work + (int64_t)b * g.bstride + (int64_t)z * g.nst;
+    const double wb = d.weights[b];
+    plane_cols_backward<T, N, PRUNE, !DIRECT>(g, w, Q, W, tw);
+    __syncthreads();
+    density_rows<T, N, PRUNE, RB, DIRECT, A>(Q, (g.nxc + 1) * (N + 1), N, W, tw, cq, wb, acc);
+  }
+  density_store<T, N, RB, A>(d, z, blockIdx.y, W, acc);
+}
+
+// Any two lengths, chosen at run time as in k_plane_any; two rows per team.
+// Nothing of a length's tables and lane indexes may be held over the band loop
+// (the compiler would hold all lengths'): they are derived from an offset that
+// it takes to be new in every round.
+template <typename T, bool SMALL, bool DIRECT>
+__global__ __launch_bounds__(64 * kPlaneAnyWaves, 3) void k_density_any(DensityArgs<T> d) {
+  extern __shared__ unsigned char smem_raw[];
+  cplx<T>* Q = reinterpret_cast<cplx<T>*>(smem_raw);
+  constexpr int RB = 2, A = RB * (SMALL ? 12 : 16);
+  const int waves = blockDim.x >> 6;
+  const int z = blockIdx.x, b0 = blockIdx.y * d.per, b1 = min(d.nb, b0 + d.per);
+  double acc[A];
+#pragma unroll
+  for (int k = 0; k < A; ++k) acc[k] = 0.0;
+  for (int b = b0; b < b1; ++b) {
+    int tid = threadIdx.x, zero = 0;
+    asm volatile("" : "+v"(tid), "+s"(zero));
+    PlaneArgs<T> g = d.plane;
+    g.colpos += zero;
+    g.colmap += zero;
+    g.tw1 += zero;
+    g.tw2 += zero;
+    const cplx<T>* w = g.work + (int64_t)b * g.bstride + (int64_t)z * g.nst;
+    const int own = (g.nxc + 1) * (g.n2 + 1);
+    const double wb = d.weights[b];
+    switch (g.n2) {
+#define QEPW_PLANE_CASE(NN)                                                               \
+  case NN:                                                                                \
+    if constexpr (!SMALL || plane_any_small(NN)) {                                        \
+      PlaneTwiddles<T, NN> tw;                                                            \
+      tw.load(PlaneLane<NN>(tid).t, g.tw2);                                               \
+      plane_cols_backward<T, NN, true>(g, w, Q, waves, tw, tid);                          \
+    }                                                                                     \
+    break;
+      QEPW_TEAM_SIZES(QEPW_PLANE_CASE)
+#undef QEPW_PLANE_CASE
+      default: break;
+    }
+    __syncthreads();
+    switch (g.n1) {
+#define QEPW_PLANE_CASE(NN)                                                               \
+  case NN:                                                                                \
+    if constexpr (!SMALL || plane_any_small(NN)) {                                        \
+      PlaneTwiddles<T, NN> tw;                                                            \
+      tw.load(PlaneLane<NN>(tid).t, g.tw1);                                               \
+      int cq[PlaneLine<NN>::L];                                                           \
+      plane_row_slots<T, NN, true>(g, g.n2 + 1, cq, tid);                                 \
+      density_rows<T, NN, true, RB, DIRECT, A>(Q, own, g.n2, waves, tw, cq, wb, acc,      \
+                                               tid);                                      \
+    }                                                                                     \
+    break;
+      QEPW_TEAM_SIZES(QEPW_PLANE_CASE)
+#undef QEPW_PLANE_CASE
+      default: break;
+    }
+  }
+  const PlaneArgs<T>& g = d.plane;
+  switch (g.n1) {
+#define QEPW_PLANE_CASE(NN)                                                               \
+  case NN:                                                                                \
+    if constexpr (!SMALL || plane_any_small(NN))                                          \
+      density_store<T, NN, RB, A>(d, z, blockIdx.y, waves, acc);                          \
+    break;
+    QEPW_TEAM_SIZES(QEPW_PLANE_CASE)
+#undef QEPW_PLANE_CASE
+    default: break;
+  }
+}
+
 // ---- host side ------------------------------------------------------------------
 template <typename T> const cplx<T>* plane_twiddles(const Plan& p, int axis);
+static inline const double2* line_twiddles(const Plan& p, double) { return p.d_tw64[0]; }
+static inline const float2* line_twiddles(const Plan& p, float) { return p.d_tw32[0]; }
 
 template <typename T>
 static PlaneArgs<T> plane_args(const Plan& p, const StickTables& st, cplx<T>* work,
@@ -563,6 +789,107 @@ bool launch_plane_stage(const Plan& p, const StickTables& st, cplx<T>* work, int
   if (plane_any_small(p.n1) && plane_any_small(p.n2)) QEPW_PLANE_LAUNCH((k_plane_any<T, true>));
   QEPW_PLANE_LAUNCH((k_plane_any<T, false>));
 #undef QEPW_PLANE_LAUNCH
+  return false;
+}
+
+template <typename T> PlaneChoice density_choice(const Plan& p, const StickTables& st) {
+  // the plane stage's, with the waves that the density kernels take
+  PlaneChoice c = sizeof(T) == 8 ? st.plane64 : st.plane32;
+  if (c.waves == 0) return c;
+  int per1 = 0, w = 0, simd = 3;
+  bool direct = false;
+#define QEPW_PLANE_N(NN)                                                                        \
+  if (p.n1 == NN) {                                                                             \
+    per1 = PlaneLine<NN>::per_wave;                                                             \
+    w = c.prune ? density_waves<T, NN, true>() : density_waves<T, NN, false>();                 \
+    direct = density_direct<T>(NN, c.prune);                                                    \
+    simd = c.prune ? density_simd_waves<T, NN, true>() : density_simd_waves<T, NN, false>();    \
+  }
+  QEPW_TEAM_SIZES(QEPW_PLANE_N)
+#undef QEPW_PLANE_N
+  if (!c.square) {
+    w = 0;
+    simd = 3;
+    direct = true;
+    for (int v : {4, 8, 12}) {
+      if (p.n2 > 2 * v * per1) continue;
+      w = v;
+      break;
+    }
+  }
+  c.waves = w;
+  const size_t columns = (size_t)(st.nxcols + 1) * (p.n2 + 1), lines = (size_t)w * per1 * (p.n1 + 1);
+  c.lds = (direct ? columns + lines : std::max(columns, lines)) * sizeof(cplx<T>);
+  if (!c.square && c.lds > (size_t)kMaxLdsBytes) {
+    direct = false;
+    c.lds = std::max(columns, lines) * sizeof(cplx<T>);
+  }
+  c.direct = direct;
+  if (c.lds > (size_t)kMaxLdsBytes) c.waves = 0;
+  if (c.waves > 0)
+    c.hold = std::max(1, std::min(4 * simd / c.waves, (int)((size_t)(160 << 10) / c.lds)));
+  return c;
+}
+
+// Slices of the bands: every slice is a workgroup per plane that takes
+// ceil(nb / slices) bands; as many as give the fewest rounds of bands.
+static int density_slices(const PlaneChoice& c, int n3, int nb, int most) {
+  const int slots = 256 * c.hold;
+  int best = 1;
+  int64_t cost = INT64_MAX;
+  for (int s = 1; s <= most && s <= nb; ++s) {
+    const int64_t rounds = ((int64_t)n3 * s + slots - 1) / slots;
+    const int64_t t = rounds * ((nb + s - 1) / s);
+    if (t < cost) {
+      cost = t;
+      best = s;
+    }
+  }
+  return best;
+}
+
+// The partial density planes of nb bands; *slices of them are written (given
+// *slices > 0, that many).  False where the team stage does not serve the plan.
+template <typename T>
+bool launch_density_stage(const Plan& p, const StickTables& st, cplx<T>* work, int64_t bstride,
+                          const double* weights, int nb, int most, int* slices, bool accumulate,
+                          double* partial, hipStream_t stream) {
+  const PlaneChoice& c = sizeof(T) == 8 ? st.density64 : st.density32;
+  if (c.waves == 0) return false;
+  if (*slices == 0) *slices = density_slices(c, p.n3, nb, most);
+  DensityArgs<T> d{};
+  d.plane = plane_args<T>(p, st, work, bstride, nullptr);
+  if (c.square && density_held<T>(p.n1)) d.plane.tw1 = line_twiddles(p, T(0));
+  d.nb = nb;
+  d.per = (nb + *slices - 1) / *slices;
+  d.accumulate = accumulate ? 1 : 0;
+  d.weights = weights;
+  d.partial = partial;
+  const dim3 grid(p.n3, *slices);
+#define QEPW_DENSITY_LAUNCH(K)                                                          \
+  do {                                                                                  \
+    allow_lds(reinterpret_cast<const void*>(&K), c.lds);                                \
+    hipLaunchKernelGGL(K, grid, dim3(64 * c.waves), c.lds, stream, d);                  \
+    return true;                                                                        \
+  } while (0)
+  if (c.square) {
+#define QEPW_DENSITY_SQUARE(NN)                                                               \
+  if constexpr (NN <= 128) {                                                                  \
+    if (p.n1 == NN && c.prune)                                                                \
+      QEPW_DENSITY_LAUNCH((k_density_square<T, NN, true, density_waves<T, NN, true>()>));     \
+    if (p.n1 == NN)                                                                           \
+      QEPW_DENSITY_LAUNCH((k_density_square<T, NN, false, density_waves<T, NN, false>()>));   \
+  }
+    QEPW_TEAM_SIZES(QEPW_DENSITY_SQUARE)
+#undef QEPW_DENSITY_SQUARE
+    return false;
+  }
+  const bool small = plane_any_small(p.n1) && plane_any_small(p.n2);
+  if (small && c.direct) QEPW_DENSITY_LAUNCH((k_density_any<T, true, true>));
+  if (small) QEPW_DENSITY_LAUNCH((k_density_any<T, true, false>));
+  if (c.direct) QEPW_DENSITY_LAUNCH((k_density_any<T, false, true>));
+  QEPW_DENSITY_LAUNCH((k_density_any<T, false, false>));
+#undef QEPW_DENSITY_LAUNCH
   return false;
 }
 

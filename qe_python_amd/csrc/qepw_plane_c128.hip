@@ -14,5 +14,10 @@ template bool launch_plane_stage<double>(const Plan& p, const StickTables& st, d
 template int launch_plane_group<double>(int count, const Plan* const* plans, double2* const* work,
                                         const int64_t* bstride, const double* const* V,
                                         const int* nb, hipStream_t stream);
+template PlaneChoice density_choice<double>(const Plan& p, const StickTables& st);
+template bool launch_density_stage<double>(const Plan& p, const StickTables& st, double2* work,
+                                           int64_t bstride, const double* weights, int nb,
+                                           int most, int* slices, bool accumulate,
+                                           double* partial, hipStream_t stream);
 
 }  // namespace qepw

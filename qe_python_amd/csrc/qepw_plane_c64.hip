@@ -14,5 +14,10 @@ template bool launch_plane_stage<float>(const Plan& p, const StickTables& st, fl
 template int launch_plane_group<float>(int count, const Plan* const* plans, float2* const* work,
                                         const int64_t* bstride, const float* const* V,
                                         const int* nb, hipStream_t stream);
+template PlaneChoice density_choice<float>(const Plan& p, const StickTables& st);
+template bool launch_density_stage<float>(const Plan& p, const StickTables& st, float2* work,
+                                           int64_t bstride, const double* weights, int nb,
+                                           int most, int* slices, bool accumulate,
+                                           double* partial, hipStream_t stream);
 
 }  // namespace qepw

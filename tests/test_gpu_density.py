@@ -123,3 +123,49 @@ def test_density_on_split_stage_grids(shape):
     lhs = float(np.sum(vr * rho)) / np.prod(shape)
     rhs = float(np.sum(w * np.real(np.sum(coeff.conj() * hx, axis=0))))
     assert lhs == pytest.approx(rhs, rel=1e-11)
+
+
+@pytest.mark.parametrize("shape,dense", [
+    ((16, 16, 20), False), ((60, 60, 16), False), ((72, 72, 16), False), ((75, 75, 16), False),
+    ((80, 80, 16), False), ((90, 90, 16), False), ((96, 96, 16), False), ((40, 40, 16), True),
+    ((72, 72, 16), True), ((80, 80, 16), True), ((18, 16, 20), False), ((48, 60, 20), False),
+    ((90, 108, 16), False), ((108, 120, 16), False), ((30, 128, 16), False),
+    ((192, 50, 16), False), ((24, 30, 20), True)])
+def test_density_of_any_two_lengths(shape, dense):
+    """The density's plane kernels over square and rectangular planes, with and
+    without exchange lines of their own, for spheres that reach the ends of the
+    pruned slots and bases that fill the axes, with one band and a number that
+    no slice count divides, against NumPy's FFT."""
+    import torch
+
+    from qe_python_amd import device as dv
+    from qe_python_amd.basis import LocalPotentialWorkspace
+    rng = np.random.default_rng(53)
+    ax = [np.arange(-((n - 1) // 2), n // 2 + 1) if dense
+          else np.arange(-((n + 1) // 4), (n - 1) // 4 + 1) for n in shape]
+    m = np.stack(np.meshgrid(*ax, indexing="ij"), -1).reshape(-1, 3)
+    if not dense:   # an ellipsoid reaching the ends of each axis
+        half = np.array([len(a) / 2.0 for a in ax])
+        mid = np.array([(a[0] + a[-1]) / 2.0 for a in ax])
+        m = m[(((m - mid) / half) ** 2).sum(1) <= 1.0]
+    m = m[rng.permutation(len(m))].astype(np.int32)
+    ws = LocalPotentialWorkspace(m, shape)
+    for nb in (1, 19):
+        x = rng.standard_normal((len(m), nb)) + 1j * rng.standard_normal((len(m), nb))
+        w = rng.uniform(0.1, 2.0, nb)
+        ref = np.zeros(shape)
+        for b in range(nb):
+            grid = np.zeros(shape, complex)
+            grid[tuple((m % np.array(shape)).T)] = x[:, b]
+            ref += w[b] * np.abs(np.fft.ifftn(grid, norm="forward")) ** 2
+        rho = np.zeros(shape)
+        ws.accumulate_density(rho, x, w)
+        np.testing.assert_allclose(rho, ref, rtol=0, atol=1e-12 * np.abs(ref).max())
+        dev = torch.device("cuda", torch.cuda.current_device())
+        from qe_python_amd.diagonalization import _upload_block
+        psi32 = _upload_block(x, ws.plan.perm_device, ws.npw, dev, torch.complex64)
+        out32 = torch.empty(shape[::-1], dtype=torch.float64, device=dev)
+        ws._accumulate_device(psi32, torch.from_numpy(w).to(dev), out32)
+        assert dv.real_dtype(psi32.dtype) == torch.float32
+        np.testing.assert_allclose(out32.permute(2, 1, 0).cpu().numpy(), ref, rtol=0,
+                                   atol=2e-6 * np.abs(ref).max())
