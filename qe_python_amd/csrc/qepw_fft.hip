@@ -485,21 +485,19 @@ __global__ __launch_bounds__(kTeamThreads) void k_sticks_group(const StickGroupA
   }
 }
 
-// z lengths with a team kernel.
-#define QEPW_LINE_SIZES(X) \
-  X(16) X(18) X(20) X(24) X(25) X(27) X(30) X(32) X(36) X(40) X(45) X(48) X(50) X(54) \
-  X(60) X(64) X(72) X(75) X(80) X(81) X(90) X(96) X(100) X(108) X(120)
-
 // Teams per workgroup of the team FFT of length n (0: no team kernel).
 static int team_teams(int n) {
   int teams = 0;
 #define QEPW_TEAMS_N(NN) if (n == NN) teams = TeamGeom<NN>::teams;
-  QEPW_LINE_SIZES(QEPW_TEAMS_N)
+  QEPW_TEAM_SIZES(QEPW_TEAMS_N)
 #undef QEPW_TEAMS_N
   return teams;
 }
 
-// Launches the team z-stage kernel for n3 if one exists; false otherwise.
+// Launches the team z-stage kernel for n3 if one exists; false otherwise.  All
+// team lengths gain over the Stockham stage that took those above 120 (FFT phase
+// of 36 x 40 x n3, 128 bands, FP64 / FP32, us: n3 128 234 / 165 -> 199 / 126, 160
+// 270 / 190 -> 225 / 142, 192 316 / 221 -> 267 / 165).
 template <typename T>
 static bool launch_sticks_team(bool inverse, const Plan& p, const StickTables& st,
                                const cplx<T>* psi, int64_t ldpsi, cplx<T>* work,
@@ -519,7 +517,7 @@ static bool launch_sticks_team(bool inverse, const Plan& p, const StickTables& s
                          st.d_off, st.d_gpos, tw, inv_n);                                    \
     return true;                                                                             \
   }
-  QEPW_LINE_SIZES(QEPW_LAUNCH_STICKS)
+  QEPW_TEAM_SIZES(QEPW_LAUNCH_STICKS)
 #undef QEPW_LAUNCH_STICKS
   return false;
 }

@@ -18,6 +18,12 @@ inline void allow_lds(const void* kernel, size_t bytes) {
     (void)hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
 }
 
+// Line lengths with a team FFT.
+#define QEPW_TEAM_SIZES(X) \
+  X(16) X(18) X(20) X(24) X(25) X(27) X(30) X(32) X(36) X(40) X(45) X(48) X(50) X(54) \
+  X(60) X(64) X(72) X(75) X(80) X(81) X(90) X(96) X(100) X(108) X(120) X(128) X(135) \
+  X(144) X(150) X(160) X(180) X(192)
+
 // Grouped launches (qepw_apply_local_group): up to kMaxFftGroup problems whose
 // plane side and z length are among QEPW_GROUP_SIZES.
 #define QEPW_GROUP_SIZES(X) X(36) X(48) X(54) X(60) X(64) X(72) X(80) X(96)

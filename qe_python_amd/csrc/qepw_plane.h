@@ -309,12 +309,6 @@ __device__ __forceinline__ void plane_cols_forward(const PlaneArgs<T>& g, cplx<T
   }
 }
 
-// Line lengths with a team FFT.
-#define QEPW_TEAM_SIZES(X) \
-  X(16) X(18) X(20) X(24) X(25) X(27) X(30) X(32) X(36) X(40) X(45) X(48) X(50) X(54) \
-  X(60) X(64) X(72) X(75) X(80) X(81) X(90) X(96) X(100) X(108) X(120) X(128) X(135) \
-  X(144) X(150) X(160) X(180) X(192)
-
 // Elements of row data a lane may hold across the row pass.
 template <typename T> constexpr int plane_row_budget() { return sizeof(T) == 8 ? 16 : 36; }
 

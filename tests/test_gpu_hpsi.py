@@ -360,3 +360,34 @@ def test_plane_stage_of_any_two_lengths(shape, dense):
     ham32 = PlaneWaveHamiltonian(basis, np.zeros(shape, complex), (), real_potential=vr,
                                  precision="fp32")
     assert rel(ham32.apply(x), ref) <= 2e-6
+
+
+@pytest.mark.parametrize("n3", [128, 135, 144, 150, 160, 180, 192])
+def test_z_lines_of_the_largest_lengths(n3):
+    """The z stages' team kernels at their largest lengths, with a number of
+    sticks that fills no whole workgroup, and the density over them."""
+    from qe_python_amd.basis import LocalPotentialWorkspace, PlaneWaveBasis
+    from qe_python_amd.diagonalization import PlaneWaveHamiltonian
+    rng = np.random.default_rng(n3)
+    shape = (16, 18, n3)
+    ax = [np.arange(-((n - 1) // 4), (n - 1) // 4 + 1) for n in shape]
+    m = np.stack(np.meshgrid(*ax, indexing="ij"), -1).reshape(-1, 3)
+    m = m[((m / np.array([len(a) / 2.0 for a in ax])) ** 2).sum(1) <= 1.0]
+    m = m[rng.permutation(len(m))].astype(np.int32)
+    kin = 0.5 * (m.astype(float) ** 2).sum(1) / 100.0
+    basis = PlaneWaveBasis(m, m.astype(float), kin)
+    vr = rng.uniform(-1.0, 0.5, shape)
+    x = rng.standard_normal((len(m), 3)) + 1j * rng.standard_normal((len(m), 3))
+    ref = OracleHamiltonian(m, kin, shape, vr).apply(x)
+    ham = PlaneWaveHamiltonian(basis, np.zeros(shape, complex), (), real_potential=vr)
+    assert rel(ham.apply(x), ref) <= 1e-12
+    ham32 = PlaneWaveHamiltonian(basis, np.zeros(shape, complex), (), real_potential=vr,
+                                 precision="fp32")
+    assert rel(ham32.apply(x), ref) <= 2e-6
+    ws = LocalPotentialWorkspace(m, shape)
+    rho = np.zeros(shape)
+    ws.accumulate_density(rho, x, np.ones(3))
+    grid = np.zeros((3,) + shape, complex)
+    grid[(slice(None),) + tuple((m % np.array(shape)).T)] = x.T
+    dens = (np.abs(np.fft.ifftn(grid, axes=(1, 2, 3), norm="forward")) ** 2).sum(0)
+    np.testing.assert_allclose(rho, dens, rtol=0, atol=1e-12 * dens.max())
