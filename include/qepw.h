@@ -260,6 +260,13 @@ int qepw_restart_applied(int precision, const void* x, int64_t ldx, const void* 
 int qepw_permute_rows(int src_precision, int dst_precision, int direction,
                       const int32_t* perm, const void* src, int64_t lds, void* dst,
                       int64_t ldd, int64_t nrows, int nb, void* stream);
+/* The same with column b multiplied by cfac[b] (device double, rounded to the
+ * source's precision) on the way: the band-energy gradient 2 f_n H psi_n in the
+ * reference row order. */
+int qepw_permute_rows_scaled(int src_precision, int dst_precision, int direction,
+                             const int32_t* perm, const double* cfac, const void* src,
+                             int64_t lds, void* dst, int64_t ldd, int64_t nrows, int nb,
+                             void* stream);
 
 /*
  * dst[:, dst_cols[j]] = scale[j] * src[:, src_cols[j]] for j < ncols, nrows

@@ -73,6 +73,8 @@ SIGNATURES = [
                                                 c_void_p, c_int64, c_int64, c_int, c_void_p]),
     ("qepw_restart_applied", c_int, [c_int, c_void_p, c_int64, c_void_p, c_int64, c_void_p,
                                      c_void_p, c_int64, c_int64, c_int, c_void_p]),
+    ("qepw_permute_rows_scaled", c_int, [c_int, c_int, c_int, c_void_p, c_void_p, c_void_p,
+                                         c_int64, c_void_p, c_int64, c_int64, c_int, c_void_p]),
     ("qepw_permute_rows", c_int, [c_int, c_int, c_int, c_void_p, c_void_p, c_int64, c_void_p,
                                   c_int64, c_int64, c_int, c_void_p]),
     ("qepw_copy_columns", c_int, [c_int, c_int, c_void_p, c_int64, c_void_p, c_void_p, c_int64,

@@ -620,8 +620,21 @@ int qepw_permute_rows(int src_precision, int dst_precision, int direction, const
     return fail(QEPW_ERR_ARG, "qepw_permute_rows: bad argument");
   if (src == dst && perm) return fail(QEPW_ERR_ARG, "qepw_permute_rows: in-place permutation");
   return finish(qepw::permute_rows(src_precision, dst_precision, direction, perm, src, lds, dst,
-                                   ldd, nrows, nb, static_cast<hipStream_t>(stream)),
+                                   ldd, nrows, nb, nullptr, static_cast<hipStream_t>(stream)),
                 "qepw_permute_rows");
+}
+
+int qepw_permute_rows_scaled(int src_precision, int dst_precision, int direction,
+                             const int32_t* perm, const double* cfac, const void* src,
+                             int64_t lds, void* dst, int64_t ldd, int64_t nrows, int nb,
+                             void* stream) {
+  if (nb > 0 && (!src || !dst || !cfac || lds < nrows || ldd < nrows))
+    return fail(QEPW_ERR_ARG, "qepw_permute_rows_scaled: bad argument");
+  if (src == dst && perm)
+    return fail(QEPW_ERR_ARG, "qepw_permute_rows_scaled: in-place permutation");
+  return finish(qepw::permute_rows(src_precision, dst_precision, direction, perm, src, lds, dst,
+                                   ldd, nrows, nb, cfac, static_cast<hipStream_t>(stream)),
+                "qepw_permute_rows_scaled");
 }
 
 int qepw_copy_columns(int src_precision, int dst_precision, const void* src, int64_t lds,

@@ -113,7 +113,7 @@ int restart_applied(int precision, const void* x, int64_t ldx, const void* r, in
                     hipStream_t stream);
 int permute_rows(int src_precision, int dst_precision, int direction, const int* perm,
                  const void* src, int64_t lds, void* dst, int64_t ldd, int64_t nrows, int nb,
-                 hipStream_t stream);
+                 const double* cfac, hipStream_t stream);
 int row_real_dot(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t nrows,
                  int ncols, double scale, double* acc, hipStream_t stream);
 int copy_columns(int src_precision, int dst_precision, const void* src, int64_t lds,

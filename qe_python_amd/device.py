@@ -259,8 +259,17 @@ def restart_applied(x: torch.Tensor, r: torch.Tensor, e: torch.Tensor, hv: torch
 
 
 def permute_rows(direction: int, perm: torch.Tensor | None, src: torch.Tensor,
-                 dst: torch.Tensor, nrows: int) -> None:
-    """direction 0: dst[d] = src[perm[d]]; 1: dst[perm[d]] = src[d]."""
+                 dst: torch.Tensor, nrows: int, cfac: torch.Tensor | None = None) -> None:
+    """direction 0: dst[d] = src[perm[d]]; 1: dst[perm[d]] = src[d]; column b
+    scaled by the float64 cfac[b] on the way."""
+    if cfac is not None:
+        rc = nat.load().qepw_permute_rows_scaled(
+            precision_code(src.dtype), precision_code(dst.dtype), direction,
+            None if perm is None else perm.data_ptr(), cfac.data_ptr(), src.data_ptr(),
+            ld_of(src), dst.data_ptr(), ld_of(dst), nrows, src.shape[0],
+            stream_handle(src.device))
+        nat.check(rc, "qepw_permute_rows_scaled")
+        return
     rc = nat.load().qepw_permute_rows(precision_code(src.dtype), precision_code(dst.dtype),
                                       direction, None if perm is None else perm.data_ptr(),
                                       src.data_ptr(), ld_of(src), dst.data_ptr(), ld_of(dst),

@@ -17,7 +17,7 @@ with the gradients
 
 Everything runs through ``libqepw_hip.so`` (``qepw_apply_local``,
 ``qepw_gemm``, ``qepw_accumulate_density``, ``qepw_build_projectors``,
-``qepw_scale_rows``, ``qepw_position_gradient``); ``band_energy`` wraps the
+``qepw_permute_rows_scaled``, ``qepw_position_gradient``); ``band_energy`` wraps the
 forward and backward in a ``torch.autograd.Function``.  Both complex128 and
 complex64 storage are supported (FP64 accumulation of every reduction).
 """
@@ -93,14 +93,6 @@ class BandEnergyModel:
         dv.gemm(nat.OP_N, self.npw, nb, p, 1.0, proj, coupled, 1.0, hpsi, self.workspace)
         return hpsi, overlap, coupled
 
-    def scale_rows(self, src, dst, s=None, sstride=0, cfac=None):
-        rc = nat.load().qepw_scale_rows(
-            dv.precision_code(src.dtype), src.data_ptr(), dv.ld_of(src),
-            None if s is None else s.data_ptr(), sstride,
-            None if cfac is None else cfac.data_ptr(), dst.data_ptr(), dv.ld_of(dst),
-            self.npw, src.shape[0], dv.stream_handle(self.device))
-        nat.check(rc, "qepw_scale_rows")
-
     def density(self, psi, weights, scale):
         """scale * sum_b weights[b] |psi_b(r)|^2, (n3, n2, n1) float64."""
         lib = nat.load()
@@ -172,10 +164,9 @@ class _BandEnergy(torch.autograd.Function):
         wf = dv.upload(wf_host, model.device)
         grad_psi = grad_v = grad_tau = None
         if ctx.needs_input_grad[0]:
-            scaled = torch.empty_like(hpsi)
-            model.scale_rows(hpsi, scaled, cfac=dv.upload(2.0 * wf_host, model.device))
-            ref = torch.empty_like(scaled)
-            dv.permute_rows(1, model.plan.perm_device, scaled, ref, model.npw)
+            ref = torch.empty_like(hpsi)
+            dv.permute_rows(1, model.plan.perm_device, hpsi, ref, model.npw,
+                            cfac=dv.upload(2.0 * wf_host, model.device))
             grad_psi = ref.T.to(ctx.psi_dtype)
         if ctx.needs_input_grad[1]:
             n = float(np.prod(model.shape))
