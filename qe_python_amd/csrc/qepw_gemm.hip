@@ -813,20 +813,24 @@ int position_gradient(int precision, int64_t npw, int64_t nproj, int nb, const v
 // 16x16 tiles are computed, one per workgroup, and each is written together
 // with its conjugate transpose (the diagonal made real): C is exactly
 // Hermitian, which the conjugated loads of Y below rely on.  Y's element
-// (k, j) is read as conj(Y[j, k]), a contiguous run like X's (i, k).  The four
+// (k, j) is read as conj(Y[j, k]), a contiguous run like X's (i, k).  The eight
 // waves of a workgroup split K, each fetching its next kHermUnroll MFMA
 // steps while the current ones run, and their partial tiles are summed in LDS
-// in wave order, so results are reproducible.  Two steps in flight measured
-// fastest (n = 264 / 432 / 512: 7.1 / 15.2 / 21.4 us against 8.4 / 18.3 /
-// 26.3 us with eight; four and six in between).
+// in wave order, so results are reproducible.  Bound by each wave's chain of
+// loads up to n ~ 200, by the tiles' L2 reads above.  n = 32 / 128 / 264 / 432 /
+// 512 with four, eight and sixteen waves: 4.0 / 5.7 / 9.7 / 16.3 / 23.4, 3.9 /
+// 5.0 / 8.0 / 14.6 / 21.4 and 4.8 / 5.7 / 8.6 / 16.3 / 22.5 us a launch.  Two
+// steps in flight (with four waves n = 264 / 432 / 512 take 18-23% longer with
+// eight; four and six lie in between).
 constexpr int kHermUnroll = 2;
+constexpr int kHermWaves = 8;
 
-__global__ __launch_bounds__(256) void k_herm_product(
+__global__ __launch_bounds__(64 * kHermWaves) void k_herm_product(
     int n, const double2* __restrict__ X, const double2* __restrict__ Y,
     const double2* __restrict__ D, double2* __restrict__ C, int64_t ld, double alpha,
     double beta) {
-  constexpr int U = kHermUnroll;
-  __shared__ double2 part[4][256];
+  constexpr int U = kHermUnroll, W = kHermWaves;
+  __shared__ double2 part[W][256];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // tile (ti, tj), ti >= tj, of linear index b = ti (ti + 1) / 2 + tj
   const int b = blockIdx.x;
@@ -837,7 +841,7 @@ __global__ __launch_bounds__(256) void k_herm_product(
   const int m0 = 16 * ti, n0 = 16 * tj;
   // this wave's K steps (4 columns of K each): [s0, s1)
   const int steps = (n + 3) >> 2;
-  const int per = (steps + 3) >> 2;
+  const int per = (steps + W - 1) / W;
   const int s0 = min(steps, wave * per);
   const int s1 = min(steps, s0 + per);
   const int r = lane & 15, kq = lane >> 4;
@@ -898,10 +902,10 @@ __global__ __launch_bounds__(256) void k_herm_product(
   __syncthreads();
   const int er = tid & 15, ec = tid >> 4;
   const int gi = m0 + er, gj = n0 + ec;
-  if (gi >= n || gj >= n || gi < gj) return;
+  if (ec >= 16 || gi >= n || gj >= n || gi < gj) return;
   double sr = 0.0, si = 0.0;
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
+  for (int q = 0; q < W; ++q) {
     sr += part[q][tid].x;
     si += part[q][tid].y;
   }
@@ -925,8 +929,8 @@ int herm_product(int n, const void* x, const void* y, const void* d, void* c, in
   if (n <= 0) return QEPW_OK;
   if (ld < n) return QEPW_ERR_ARG;
   const int nt = (n + 15) / 16;
-  hipLaunchKernelGGL(k_herm_product, dim3((unsigned)(nt * (nt + 1) / 2)), dim3(256), 0,
-                     stream, n, static_cast<const double2*>(x), static_cast<const double2*>(y),
+  hipLaunchKernelGGL(k_herm_product, dim3((unsigned)(nt * (nt + 1) / 2)), dim3(64 * kHermWaves),
+                     0, stream, n, static_cast<const double2*>(x), static_cast<const double2*>(y),
                      static_cast<const double2*>(d), static_cast<double2*>(c), ld, alpha, beta);
   return hipGetLastError() == hipSuccess ? QEPW_OK : QEPW_ERR_HIP;
 }
