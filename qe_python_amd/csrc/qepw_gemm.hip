@@ -651,9 +651,13 @@ static SplitPlan built_in_plan(int precision, int op_a, int64_t m, int64_t n, in
   const int64_t out_bytes = m * n * (precision == QEPW_C128 ? 16 : 8);
   const int64_t scratch = (int64_t)QEPW_GEMM_STATIC_SCRATCH;
   const bool over = fixed.splits > 1 && fixed.splits > scratch / out_bytes;
-  // (no split below 256 columns, which take no longer than the second kernel)
-  const int64_t most =
-      k < 256 ? 1 : std::min(k / 32, (over ? 4 : 1) * scratch / out_bytes);
+  // A^H B of fewer than 256 columns stays unsplit: Gram matrices of small bases
+  // keep the order of their sums, which decides the pivot's sign where a basis is
+  // singular to the last bit.  A B is split down to chunks of 32 (the D coupling,
+  // 168 x 96 x 168 in FP32, with its h_psi: 172 us unsplit, 166 split)
+  const int64_t most = (op_a & QEPW_OP_C) && k < 256
+                           ? 1
+                           : std::min(k / 32, (over ? 4 : 1) * scratch / out_bytes);
   SplitPlan best = fixed;
   double cost = plan_cost(precision, fixed.variant, m, n, fixed.splits, fixed.kchunk);
   for (int v = 0; v < kNumVariants; ++v) {
