@@ -8,10 +8,11 @@
 //   A  k_sticks_inverse : gather the rows of ``group`` sticks (contiguous in
 //                         the device order) into LDS lines, backward z-FFT,
 //                         write the (n3, nst) stick buffer;
-//   B  k_planes         : one workgroup per (z-plane, band): load the plane's
-//                         active sticks into an n1 x n2 LDS plane, backward
-//                         y-FFT on active x columns only, backward x-FFT,
-//                         multiply by V(z, x, y), forward x-FFT, forward
+//   B  the xy planes    : one workgroup per (z-plane, band).  Team lengths take
+//                         qepw_plane.h; k_planes serves the others: load the
+//                         plane's active sticks into an n1 x n2 LDS plane,
+//                         backward y-FFT on active x columns only, backward
+//                         x-FFT, multiply by V(z, x, y), forward x-FFT, forward
 //                         y-FFT on active columns, store the active sticks;
 //   C  k_sticks_forward : forward z-FFT, gather the sphere rows, scale 1/N and
 //                         add T_G psi_G.
