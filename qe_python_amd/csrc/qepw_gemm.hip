@@ -357,17 +357,67 @@ __global__ __launch_bounds__(256) void k_reduce_splits(
 
 // One-column products (n = 1: a single band's projections and projector
 // sums) as matrix-vector passes instead of MFMA tiles with one live column.
-// Both write split-K partials part[s * m + i] that k_reduce_splits sums in a
-// fixed order and scales by alpha, beta.
-//   k_gemv_n: sum_{j in split s} A[i + j lda] b_j, one thread per row i;
-//   k_gemv_c: sum_{g in split s} conj(A[g + i lda]) b_g, one workgroup per
-//             (i, s) with a fixed-order tree sum.
-// b_j = B[j bstride], conjugated when CB.
+//   k_gemv_n: sum_j A[i + j lda] b_j, one workgroup per 64 rows, a lane a row;
+//             its sixteen waves take every sixteenth column;
+//   k_gemv_c: sum_g conj(A[g + i lda]) b_g, one workgroup per i with a
+//             fixed-order tree sum.
+// b_j = B[j bstride], conjugated when CB.  Both finish the sum in the workgroup and
+// scale it by alpha, beta.  Deep products (gemv_direct) take k_gemv_n_split or
+// SPLIT, 256 wide, whose partials part[s * m + i] k_reduce_splits sums in a fixed
+// order.  Bound by launches at a single band, by A's bytes above: an h_psi of 36^3
+// takes 82 -> 73 us with the three reductions gone; FP64 23 847 x 256 19.7 -> 17.3
+// us, its A^H 18.6 -> 17.2.
+template <typename T>
+__device__ __forceinline__ void gemv_store(cplx<T>* C, int64_t i, T sr, T si, T alpha_r, T alpha_i,
+                                           T beta_r, T beta_i) {
+  cplx<T> out;
+  out.x = alpha_r * sr - alpha_i * si;
+  out.y = alpha_r * si + alpha_i * sr;
+  if (beta_r != T(0) || beta_i != T(0)) {
+    const cplx<T> c = C[i];
+    out.x += beta_r * c.x - beta_i * c.y;
+    out.y += beta_r * c.y + beta_i * c.x;
+  }
+  C[i] = out;
+}
+
+constexpr int kGemvWaves = 16;
+
 template <typename T, bool CB>
-__global__ __launch_bounds__(256) void k_gemv_n(int64_t m, int64_t k, int64_t kchunk,
-                                                const cplx<T>* __restrict__ A, int64_t lda,
-                                                const cplx<T>* __restrict__ B, int64_t bstride,
-                                                cplx<T>* __restrict__ part) {
+__global__ __launch_bounds__(64 * kGemvWaves) void k_gemv_n(
+    int64_t m, int64_t k, const cplx<T>* __restrict__ A, int64_t lda,
+    const cplx<T>* __restrict__ B, int64_t bstride, cplx<T>* __restrict__ C, T alpha_r, T alpha_i,
+    T beta_r, T beta_i) {
+  __shared__ T shr[kGemvWaves][64], shi[kGemvWaves][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t i = (int64_t)blockIdx.x * 64 + lane;
+  const cplx<T>* row = A + (i < m ? i : m - 1);
+  T sr = T(0), si = T(0);
+#pragma unroll 4
+  for (int64_t j = wave; j < k; j += kGemvWaves) {
+    const cplx<T> a = row[j * lda];
+    const cplx<T> b = B[j * bstride];
+    const T bi = CB ? -b.y : b.y;
+    sr += a.x * b.x - a.y * bi;
+    si += a.x * bi + a.y * b.x;
+  }
+  shr[wave][lane] = sr;
+  shi[wave][lane] = si;
+  __syncthreads();
+  if (wave != 0 || i >= m) return;
+#pragma unroll
+  for (int w = 1; w < kGemvWaves; ++w) {
+    sr += shr[w][lane];
+    si += shi[w][lane];
+  }
+  gemv_store<T>(C, i, sr, si, alpha_r, alpha_i, beta_r, beta_i);
+}
+
+template <typename T, bool CB>
+__global__ __launch_bounds__(256) void k_gemv_n_split(int64_t m, int64_t k, int64_t kchunk,
+                                                      const cplx<T>* __restrict__ A, int64_t lda,
+                                                      const cplx<T>* __restrict__ B,
+                                                      int64_t bstride, cplx<T>* __restrict__ part) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= m) return;
   const int64_t j0 = (int64_t)blockIdx.y * kchunk;
@@ -384,18 +434,22 @@ __global__ __launch_bounds__(256) void k_gemv_n(int64_t m, int64_t k, int64_t kc
   part[(int64_t)blockIdx.y * m + i] = mk<T>(sr, si);
 }
 
-template <typename T, bool CB>
-__global__ __launch_bounds__(256) void k_gemv_c(int64_t m, int64_t k, int64_t kchunk,
-                                                const cplx<T>* __restrict__ A, int64_t lda,
-                                                const cplx<T>* __restrict__ B, int64_t bstride,
-                                                cplx<T>* __restrict__ part) {
-  __shared__ T shr[256], shi[256];
+template <typename T, bool CB, bool SPLIT>
+__global__ __launch_bounds__(SPLIT ? 256 : 1024) void k_gemv_c(
+    int64_t m, int64_t k, int64_t kchunk, const cplx<T>* __restrict__ A, int64_t lda,
+    const cplx<T>* __restrict__ B, int64_t bstride, cplx<T>* __restrict__ part, T alpha_r,
+    T alpha_i, T beta_r, T beta_i) {
+  constexpr int THREADS = SPLIT ? 256 : 1024;
+  __shared__ T shr[THREADS], shi[THREADS];
   const int64_t i = blockIdx.x;
-  const int64_t g0 = (int64_t)blockIdx.y * kchunk;
-  const int64_t g1 = g0 + kchunk < k ? g0 + kchunk : k;
+  const int64_t g0 = SPLIT ? (int64_t)blockIdx.y * kchunk : 0;
+  const int64_t g1 = SPLIT && g0 + kchunk < k ? g0 + kchunk : k;
   const cplx<T>* col = A + i * lda;
   T sr = T(0), si = T(0);
-  for (int64_t g = g0 + threadIdx.x; g < g1; g += 256) {
+  // (512 x 78 805 split: FP64 115 us, 126 unrolled by four; FP32 90 and 72)
+  constexpr int U = SPLIT && sizeof(T) == 8 ? 1 : 4;
+#pragma unroll U
+  for (int64_t g = g0 + threadIdx.x; g < g1; g += THREADS) {
     const cplx<T> a = col[g];
     const cplx<T> b = B[g * bstride];
     const T bi = CB ? -b.y : b.y;
@@ -406,18 +460,21 @@ __global__ __launch_bounds__(256) void k_gemv_c(int64_t m, int64_t k, int64_t kc
   shr[tid] = sr;
   shi[tid] = si;
   __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
+  for (int w = THREADS / 2; w > 0; w >>= 1) {
     if (tid < w) {
       shr[tid] += shr[tid + w];
       shi[tid] += shi[tid + w];
     }
     __syncthreads();
   }
-  if (tid == 0) part[(int64_t)blockIdx.y * m + i] = mk<T>(shr[0], shi[0]);
+  if (tid != 0) return;
+  if (SPLIT) part[(int64_t)blockIdx.y * m + i] = mk<T>(shr[0], shi[0]);
+  else gemv_store<T>(part, i, shr[0], shi[0], alpha_r, alpha_i, beta_r, beta_i);
 }
 
-// Splits of a one-column product: about 1024 workgroups in all, each split of
-// K at least 8 columns of A (k_gemv_n) or 1024 rows (k_gemv_c).
+// Splits of a one-column product, whose partials the caller's workspace holds:
+// about 1024 workgroups in all, each split of K at least 8 columns of A or, of A^H,
+// 1024 rows.
 struct GemvPlan {
   int64_t splits;
   int64_t kchunk;
@@ -432,6 +489,14 @@ static GemvPlan gemv_plan(bool ca, int64_t m, int64_t k) {
   if (splits < 1) splits = 1;
   const int64_t kchunk = (k + splits - 1) / splits;
   return {(k + kchunk - 1) / kchunk, kchunk};
+}
+
+// Whether a one-column product runs unsplit: where it fills the chip, or ends sooner
+// than a second kernel starts.  Beyond, split and unsplit: FP64 64 x 2000 13.9 and
+// 29.1 us, FP32 78 805 x 512 56 and 65; A^H FP64 64 x 100 000 21 and 35, 512 x 78 805
+// 115 and 122.
+static bool gemv_direct(bool ca, int64_t m, int64_t k) {
+  return ca ? k <= 8192 || (m >= 64 && k <= 32768) : k <= 384;
 }
 
 // Tile variants of k_cgemm: (TM, TN, WAVES_M).
@@ -961,26 +1026,42 @@ static int gemv_t(int op, int64_t m, int64_t k, const double* alpha, const void*
   const cplx<T>* pa = static_cast<const cplx<T>*>(a);
   const cplx<T>* pb = static_cast<const cplx<T>*>(b);
   cplx<T>* part = static_cast<cplx<T>*>(ws);
-  if (ca) {
-    const dim3 grid((unsigned)m, (unsigned)gp.splits);
+  cplx<T>* pc = static_cast<cplx<T>*>(c);
+  const T ar = (T)alpha[0], ai = (T)alpha[1], br = (T)beta[0], bi = (T)beta[1];
+  const bool direct = gemv_direct(ca, m, k);
+  if (!ca && direct) {
+    if ((m + 63) / 64 > 0x7fffffff) return QEPW_ERR_UNSUPPORTED;
+    const dim3 grid((unsigned)((m + 63) / 64));
     if (cb)
-      hipLaunchKernelGGL((k_gemv_c<T, true>), grid, dim3(256), 0, stream, m, k, gp.kchunk, pa,
-                         lda, pb, bstride, part);
+      hipLaunchKernelGGL((k_gemv_n<T, true>), grid, dim3(64 * kGemvWaves), 0, stream, m, k, pa,
+                         lda, pb, bstride, pc, ar, ai, br, bi);
     else
-      hipLaunchKernelGGL((k_gemv_c<T, false>), grid, dim3(256), 0, stream, m, k, gp.kchunk, pa,
-                         lda, pb, bstride, part);
+      hipLaunchKernelGGL((k_gemv_n<T, false>), grid, dim3(64 * kGemvWaves), 0, stream, m, k, pa,
+                         lda, pb, bstride, pc, ar, ai, br, bi);
+  } else if (!direct) {
+    const dim3 grid((unsigned)(ca ? m : (m + 255) / 256), (unsigned)gp.splits);
+    if (ca && cb)
+      hipLaunchKernelGGL((k_gemv_c<T, true, true>), grid, dim3(256), 0, stream, m, k, gp.kchunk,
+                         pa, lda, pb, bstride, part, ar, ai, br, bi);
+    else if (ca)
+      hipLaunchKernelGGL((k_gemv_c<T, false, true>), grid, dim3(256), 0, stream, m, k, gp.kchunk,
+                         pa, lda, pb, bstride, part, ar, ai, br, bi);
+    else if (cb)
+      hipLaunchKernelGGL((k_gemv_n_split<T, true>), grid, dim3(256), 0, stream, m, k, gp.kchunk,
+                         pa, lda, pb, bstride, part);
+    else
+      hipLaunchKernelGGL((k_gemv_n_split<T, false>), grid, dim3(256), 0, stream, m, k, gp.kchunk,
+                         pa, lda, pb, bstride, part);
+    hipLaunchKernelGGL(k_reduce_splits<T>, dim3((unsigned)((m + 63) / 64)), dim3(256), 0, stream,
+                       m, (int64_t)1, (int)gp.splits, part, pc, ldc, ar, ai, br, bi);
   } else {
-    const dim3 grid((unsigned)((m + 255) / 256), (unsigned)gp.splits);
     if (cb)
-      hipLaunchKernelGGL((k_gemv_n<T, true>), grid, dim3(256), 0, stream, m, k, gp.kchunk, pa,
-                         lda, pb, bstride, part);
+      hipLaunchKernelGGL((k_gemv_c<T, true, false>), dim3((unsigned)m), dim3(1024), 0, stream, m,
+                         k, k, pa, lda, pb, bstride, pc, ar, ai, br, bi);
     else
-      hipLaunchKernelGGL((k_gemv_n<T, false>), grid, dim3(256), 0, stream, m, k, gp.kchunk, pa,
-                         lda, pb, bstride, part);
+      hipLaunchKernelGGL((k_gemv_c<T, false, false>), dim3((unsigned)m), dim3(1024), 0, stream, m,
+                         k, k, pa, lda, pb, bstride, pc, ar, ai, br, bi);
   }
-  hipLaunchKernelGGL(k_reduce_splits<T>, dim3((unsigned)((m + 63) / 64)), dim3(256), 0, stream,
-                     m, (int64_t)1, (int)gp.splits, part, static_cast<cplx<T>*>(c), ldc,
-                     (T)alpha[0], (T)alpha[1], (T)beta[0], (T)beta[1]);
   return hipGetLastError() == hipSuccess ? QEPW_OK : QEPW_ERR_HIP;
 }
 

@@ -145,6 +145,34 @@ def test_gemm_chosen_plans_at_tile_and_step_edges(prec, op):
         assert err < tol, (m, n, k, list(plan), err)
 
 
+@pytest.mark.parametrize("prec", ["c128", "c64"])
+@pytest.mark.parametrize("op", ["N", "C", "NB", "CB"])
+def test_one_column_products_at_their_edges(prec, op):
+    """Matrix-vector products either side of 64 rows, 16 columns, and the
+    limits where they are split (A b above 384 columns, A^H b above 8192 rows
+    with fewer than 64 outputs and above 32768), against NumPy."""
+    from qe_python_amd import _native as nat
+    from qe_python_amd import device as dv
+    dtype = torch.complex128 if prec == "c128" else torch.complex64
+    code = (nat.OP_N if op[0] == "N" else nat.OP_C) | (nat.OP_BC if op.endswith("B") else 0)
+    ws = dv.Workspace(torch.device(DEV))
+    for m, k in [(1, 1), (63, 15), (64, 16), (65, 17), (1000, 256), (72, 72), (63, 8192),
+                 (63, 8193), (64, 8193), (1, 9000), (100, 384), (100, 385), (64, 32769)]:
+        rng = np.random.default_rng(m + k)
+        a = rand(rng, m, k) if op[0] == "N" else rand(rng, k, m)
+        b = rand(rng, 1, k) if op.endswith("B") else rand(rng, k, 1)
+        c = rand(rng, m, 1)
+        ta, tb = dev_block(a, dtype), dev_block(b, dtype)
+        bb = b.conj().T if op.endswith("B") else b
+        for alpha, beta in ((1.0, 0.0), (0.6 + 0.3j, -0.2 + 0.1j)):
+            tc = dev_block(c, dtype)
+            dv.gemm(code, m, 1, k, alpha, ta, tb, beta, tc, ws)
+            ref = alpha * ((a if op[0] == "N" else a.conj().T) @ bb) + beta * c
+            tol = 1e-12 if prec == "c128" else 2e-6 + 1e-7 * np.sqrt(k)
+            err = np.linalg.norm(host_block(tc) - ref) / np.linalg.norm(ref)
+            assert err < tol, (m, k, err)
+
+
 def test_gemm_in_a_workspace_of_fixed_size():
     """A product whose planned partials exceed the static scratch runs in the
     Rayleigh-Ritz steps' workspace with fewer splits; less than 21 splits of
