@@ -5,8 +5,7 @@
 // recursive decimation in time M = R*S:
 //   A_j1[k1] = DFT_S over j2 of v[j1 + R j2];
 //   X[k1 + S k2] = DFT_R over j1 of (w_M^(j1 k1) A_j1[k1]).
-// Twiddles are compile-time constants (a constexpr sine/cosine evaluated by
-// the compiler from their Taylor series after exact octant reduction).
+// Twiddles are compile-time constants (qepw_roots.h).
 //
 // team_fft<T, N, SIGN>: one line of length N = L*M (M >= L, both <= 16) by a
 // team of M lanes of one wave: lanes j1 < L take the M-point DFTs of the
@@ -17,74 +16,9 @@
 #pragma once
 
 #include "qepw_fft_lds.h"
+#include "qepw_roots.h"
 
 namespace qepw {
-
-// ---- compile-time unit roots -------------------------------------------
-constexpr double kPiD = 3.14159265358979323846264338327950288;
-
-constexpr double cx_sin_small(double x) {  // |x| <= pi/4
-  double term = x, sum = x;
-  for (int i = 1; i < 14; ++i) {
-    term *= -x * x / ((2.0 * i) * (2.0 * i + 1.0));
-    sum += term;
-  }
-  return sum;
-}
-constexpr double cx_cos_small(double x) {  // |x| <= pi/4
-  double term = 1.0, sum = 1.0;
-  for (int i = 1; i < 14; ++i) {
-    term *= -x * x / ((2.0 * i - 1.0) * (2.0 * i));
-    sum += term;
-  }
-  return sum;
-}
-// cos / sin of 2 pi k / n with k reduced exactly into an octant.
-constexpr double cx_cos2pi(int k, int n) {
-  k %= n;
-  if (k < 0) k += n;
-  // theta = 2 pi k / n = (pi/4) * (8k/n); octant o = floor(8k/n)
-  const int o = (8 * k) / n;
-  const double r = 2.0 * kPiD * (double)(8 * k - o * n) / (8.0 * n);  // in [0, pi/4)
-  switch (o) {
-    case 0: return cx_cos_small(r);
-    case 1: return cx_sin_small(kPiD / 4 - r);
-    case 2: return -cx_sin_small(r);
-    case 3: return -cx_cos_small(kPiD / 4 - r);
-    case 4: return -cx_cos_small(r);
-    case 5: return -cx_sin_small(kPiD / 4 - r);
-    case 6: return cx_sin_small(r);
-    default: return cx_cos_small(kPiD / 4 - r);
-  }
-}
-constexpr double cx_sin2pi(int k, int n) {
-  k %= n;
-  if (k < 0) k += n;
-  const int o = (8 * k) / n;
-  const double r = 2.0 * kPiD * (double)(8 * k - o * n) / (8.0 * n);
-  switch (o) {
-    case 0: return cx_sin_small(r);
-    case 1: return cx_cos_small(kPiD / 4 - r);
-    case 2: return cx_cos_small(r);
-    case 3: return cx_sin_small(kPiD / 4 - r);
-    case 4: return -cx_sin_small(r);
-    case 5: return -cx_cos_small(kPiD / 4 - r);
-    case 6: return -cx_cos_small(r);
-    default: return -cx_sin_small(kPiD / 4 - r);
-  }
-}
-
-template <int M> struct UnitRoots {
-  // w[k] = exp(+2 pi i k / M)
-  double c[M > 0 ? M : 1];
-  double s[M > 0 ? M : 1];
-  constexpr UnitRoots() : c(), s() {
-    for (int k = 0; k < M; ++k) {
-      c[k] = cx_cos2pi(k, M);
-      s[k] = cx_sin2pi(k, M);
-    }
-  }
-};
 
 constexpr int smallest_radix(int m) {
   return (m % 4 == 0) ? 4 : (m % 2 == 0) ? 2 : (m % 3 == 0) ? 3 : 5;
