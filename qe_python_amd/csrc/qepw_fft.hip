@@ -880,10 +880,35 @@ __global__ __launch_bounds__(kSplitThreads) void k_split_rows_density(
 
 constexpr int kDensitySlices = 16;
 
+template <typename T>
+static bool density_team(const StickTables& st) {
+  return (sizeof(T) == 8 ? st.density64 : st.density32).waves > 0;
+}
+
+// Planes that neither the team kernel nor one workgroup's LDS can hold go through
+// the split stage's column lines, as in apply_local.  (Not for the same plans: the
+// team kernel of the density takes two rows of a rectangle per team, that of the
+// plane stage up to three.)
+template <typename T>
+static bool density_split(const Plan& p, const StickTables& st) {
+  return !density_team<T>(st) && !generic_plane_fits<T>(p) && split_available<T>(p, st);
+}
+
+// Workspace of one band of the density: its sticks, and the column lines of the
+// split stage where that runs.
+template <typename T>
+static size_t density_band_bytes(const Plan& p) {
+  const StickTables& st = p.sphere;
+  size_t e = (size_t)p.n3 * (size_t)st.nst;
+  if (density_split<T>(p, st)) e += (size_t)split_band_elems(p, st);
+  return e * sizeof(cplx<T>);
+}
+
 size_t density_workspace_bytes(const Plan& p, int precision, int nb) {
   const size_t ngrid = (size_t)p.n1 * p.n2 * p.n3;
-  return apply_local_band_bytes(p, precision) * (size_t)(nb > 0 ? nb : 1) +
-         (size_t)kDensitySlices * ngrid * sizeof(double) + 256;
+  const size_t band = precision == QEPW_C128 ? density_band_bytes<double>(p)
+                                             : density_band_bytes<float>(p);
+  return band * (size_t)(nb > 0 ? nb : 1) + (size_t)kDensitySlices * ngrid * sizeof(double) + 256;
 }
 
 template <typename T>
@@ -895,18 +920,15 @@ int accumulate_density_t(const Plan& p, const void* vectors, int64_t ldv, int nb
   const size_t np = (size_t)p.n1 * p.n2;
   if (st.group * p.n3 > lds_fft_capacity(p.line[2], kStickThreads, kStickPts))
     return QEPW_ERR_UNSUPPORTED;
-  const bool team = (sizeof(T) == 8 ? st.density64 : st.density32).waves > 0;
-  // planes that neither the team kernel nor one workgroup's LDS can hold go
-  // through the split stage's column lines, as in apply_local
-  const bool split = !team && !generic_plane_fits<T>(p) && split_available<T>(p, st);
+  const bool team = density_team<T>(st);
+  const bool split = density_split<T>(p, st);
   if (!team && !split) {
     int rc = check_fft_limits<T>(p, st);
     if (rc) return rc;
   }
   const size_t partial_bytes = (size_t)kDensitySlices * ngrid * sizeof(double);
-  const size_t stick_band = (size_t)p.n3 * st.nst * sizeof(cplx<T>);
   const int64_t tband = split ? split_band_elems(p, st) : 0;
-  const size_t band_bytes = stick_band + (size_t)tband * sizeof(cplx<T>);
+  const size_t band_bytes = density_band_bytes<T>(p);
   if (ws_bytes < partial_bytes + band_bytes) return QEPW_ERR_WORKSPACE;
   double* partial = static_cast<double*>(workspace);
   cplx<T>* work = reinterpret_cast<cplx<T>*>(static_cast<char*>(workspace) + partial_bytes);

@@ -169,3 +169,49 @@ def test_density_of_any_two_lengths(shape, dense):
         assert dv.real_dtype(psi32.dtype) == torch.float32
         np.testing.assert_allclose(out32.permute(2, 1, 0).cpu().numpy(), ref, rtol=0,
                                    atol=2e-6 * np.abs(ref).max())
+
+
+@pytest.mark.parametrize("shape,dtype", [
+    ((96, 128, 16), "complex128"), ((75, 108, 16), "complex128"), ((120, 128, 16), "complex128"),
+    ((160, 120, 16), "complex64"), ((144, 144, 16), "complex64"), ((72, 75, 16), "complex64")])
+def test_density_in_the_quoted_workspace(shape, dtype):
+    """qepw_accumulate_density in exactly the bytes that
+    qepw_accumulate_density_workspace quotes, where the plane stage and the
+    density run on the same kernels and where they do not, against NumPy."""
+    import torch
+
+    from qe_python_amd import _native as nat
+    from qe_python_amd import device as dv
+    from qe_python_amd.basis import LocalPotentialWorkspace
+    from qe_python_amd.diagonalization import _upload_block
+    lib = nat.load()
+    dev = torch.device("cuda", torch.cuda.current_device())
+    torch_type = getattr(torch, dtype)
+    rng = np.random.default_rng(59)
+    ax = [np.arange(-((n + 1) // 4), (n - 1) // 4 + 1) for n in shape]
+    m = np.stack(np.meshgrid(*ax, indexing="ij"), -1).reshape(-1, 3)
+    half = np.array([len(a) / 2.0 for a in ax])
+    mid = np.array([(a[0] + a[-1]) / 2.0 for a in ax])
+    m = m[(((m - mid) / half) ** 2).sum(1) <= 1.0].astype(np.int32)
+    plan = LocalPotentialWorkspace(m, shape).plan
+    prec = dv.precision_code(torch_type)
+    for nb in (1, 3):
+        x = rng.standard_normal((len(m), nb)) + 1j * rng.standard_normal((len(m), nb))
+        w = rng.uniform(0.1, 2.0, nb)
+        psi = _upload_block(x, plan.perm_device, len(m), dev, torch_type)
+        wd = torch.from_numpy(w).to(dev)
+        out = torch.empty(shape[::-1], dtype=torch.float64, device=dev)
+        need = lib.qepw_accumulate_density_workspace(plan.handle, prec, nb)
+        ws = torch.empty(need, dtype=torch.uint8, device=dev)
+        nat.check(lib.qepw_accumulate_density(
+            plan.handle, prec, psi.data_ptr(), dv.ld_of(psi), nb, wd.data_ptr(), 1.0,
+            out.data_ptr(), ws.data_ptr(), need, dv.stream_handle(dev)),
+            "qepw_accumulate_density")
+        ref = np.zeros(shape)
+        for b in range(nb):
+            grid = np.zeros(shape, complex)
+            grid[tuple((m % np.array(shape)).T)] = x[:, b]
+            ref += w[b] * np.abs(np.fft.ifftn(grid, norm="forward")) ** 2
+        tol = 1e-12 if dtype == "complex128" else 2e-6
+        np.testing.assert_allclose(out.permute(2, 1, 0).cpu().numpy(), ref, rtol=0,
+                                   atol=tol * np.abs(ref).max())
