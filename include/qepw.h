@@ -142,8 +142,12 @@ int qepw_inverse_real(const qepw_plan* plan, const void* grid_g, double* out,
  * (v_mfma_f64_16x16x4f64 for QEPW_C128, v_mfma_f32_16x16x4f32 for QEPW_C64).
  * op_a = QEPW_OP_N: A is m x k;  QEPW_OP_C: A is k x m and op(A) = A^H;
  * or-ed with QEPW_OP_BC: B is n x k and op(B) = B^H (else B is k x n).
- * alpha, beta: host (re, im) pairs.  A^H B with large k is split over k with
- * a fixed-order (deterministic) reduction through ``workspace``.
+ * alpha, beta: host (re, im) pairs.  Products with few tiles are split over k
+ * with a fixed-order (deterministic) reduction through ``workspace``.  In a
+ * workspace smaller than qepw_gemm_workspace's bytes the product runs in panels
+ * with the same bits, down to 32 MiB or the bytes of a simpler split where those
+ * are fewer (less, or less than two outputs: QEPW_ERR_WORKSPACE); one that the
+ * simpler choice does not split runs unsplit, in another order of the sums.
  * Replaces: the zgemm bridge qepy_zgemm64 (qepy_pw/_native_fft.pyx:595-634)
  *   and its users projector_overlaps (:694-731, becp = beta^H psi) and
  *   add_projector_product (:782-836, Hpsi += beta (D becp)), plus the
@@ -180,11 +184,12 @@ int qepw_gemm_clear_rules(void);
  * QEPW_GEMM_STATIC_SCRATCH bytes (32 MiB) that each GPU the library runs on
  * holds until the process ends (qepw_gemm_static_scratch_bytes() returns the
  * size).  Same arguments, kernels and results as qepw_gemm (bitwise: the
- * same split plan and fixed-order reduction).  A product whose split-K
- * partials would exceed the array returns QEPW_ERR_WORKSPACE with a message
- * naming the size.  Calls that overlap on one GPU share its array and race;
- * the array needs no clearing between calls (every partial tile is written
- * before it is summed).  Call with the stream's device current.
+ * same split plan and fixed-order reduction, in panels where the partials
+ * exceed the array).  A product of which the array cannot hold two partial
+ * outputs returns QEPW_ERR_WORKSPACE with a message naming the size.  Calls
+ * that overlap on one GPU share its array and race; the array needs no clearing
+ * between calls (every partial tile is written before it is summed).  Call with
+ * the stream's device current.
  * No counterpart in the reference: this entry point is for callers that
  * cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc).

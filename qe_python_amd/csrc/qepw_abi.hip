@@ -536,7 +536,14 @@ int qepw_gemm_static(int precision, int op_a, int64_t m, int64_t n, int64_t k,
   if (precision != QEPW_C128 && precision != QEPW_C64)
     return fail(QEPW_ERR_ARG, "qepw_gemm_static: unknown precision");
   const size_t need = qepw::gemm_workspace_bytes(precision, op_a, m, n, k);
-  if (need > kStaticScratchBytes) {
+  void* ptr = nullptr;
+  if (need > 0) {
+    const int rc = static_scratch(&ptr);
+    if (rc != QEPW_OK) return rc;
+  }
+  const int rc = qepw::gemm(precision, op_a, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, ptr,
+                            need > 0 ? kStaticScratchBytes : 0, static_cast<hipStream_t>(stream));
+  if (rc == QEPW_ERR_WORKSPACE) {
     char msg[192];
     std::snprintf(msg, sizeof msg,
                   "qepw_gemm_static: this product needs %zu bytes of split-K scratch, more "
@@ -544,14 +551,7 @@ int qepw_gemm_static(int precision, int op_a, int64_t m, int64_t n, int64_t k,
                   need, kStaticScratchBytes);
     return fail(QEPW_ERR_WORKSPACE, msg);
   }
-  void* ptr = nullptr;
-  if (need > 0) {
-    const int rc = static_scratch(&ptr);
-    if (rc != QEPW_OK) return rc;
-  }
-  return finish(qepw::gemm(precision, op_a, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, ptr,
-                           need > 0 ? kStaticScratchBytes : 0, static_cast<hipStream_t>(stream)),
-                "qepw_gemm_static");
+  return finish(rc, "qepw_gemm_static");
 }
 
 int qepw_column_squared_norms(int precision, const void* v, int64_t ldv, int64_t nrows, int nb,

@@ -723,6 +723,12 @@ static SplitPlan built_in_plan(int precision, int op_a, int64_t m, int64_t n, in
   const int64_t most = (op_a & QEPW_OP_C) && k < 256
                            ? 1
                            : std::min(k / 32, (over ? 4 : 1) * scratch / out_bytes);
+  // ... of which one row or column of tiles has to fit the static scratch
+  // (split_panel)
+  const auto most_of = [&](const GemmVariant& v) {
+    const int64_t panel = std::min(std::min<int64_t>(v.tm, m) * n, m * std::min<int64_t>(v.tn, n));
+    return over ? std::min(most, scratch * m * n / (panel * out_bytes)) : most;
+  };
   SplitPlan best = fixed;
   double cost = plan_cost(precision, fixed.variant, m, n, fixed.splits, fixed.kchunk);
   for (int v = 0; v < kNumVariants; ++v) {
@@ -731,7 +737,7 @@ static SplitPlan built_in_plan(int precision, int op_a, int64_t m, int64_t n, in
     // unsplit, and the splits that give each CU one, two, ... eight tiles, up
     // to what the scratch holds and to chunks of 32 columns
     for (int per = 0; per <= 8; ++per) {
-      const int64_t s = per == 0 ? 1 : std::min(most, 256 * per / vt);
+      const int64_t s = per == 0 ? 1 : std::min(most_of(kVariants[v]), 256 * per / vt);
       if (s <= last) continue;
       last = s;
       const SplitPlan p = finish_plan(v, s, k);
@@ -1065,6 +1071,29 @@ static int gemv_t(int op, int64_t m, int64_t k, const double* alpha, const void*
   return hipGetLastError() == hipSuccess ? QEPW_OK : QEPW_ERR_HIP;
 }
 
+static size_t split_bytes(const SplitPlan& p, int64_t m, int64_t n, size_t elem) {
+  return p.splits > 1 ? (size_t)p.splits * m * n * elem : 0;
+}
+
+// A product whose partials exceed its workspace runs in panels of whole tiles, of
+// mp rows or np columns, one after the other with the same plan: the bits of the
+// result do not depend on the workspace.  False where the workspace is refused:
+// short of the fixed choice's partials, or of the static scratch where those
+// exceed it, unless two partial outputs already do.
+static bool split_panel(const SplitPlan& sp, const SplitPlan& fixed, int64_t m, int64_t n,
+                        size_t elem, size_t ws_bytes, int64_t* mp, int64_t* np) {
+  const size_t least = std::min(split_bytes(fixed, m, n, elem),
+                                std::max(QEPW_GEMM_STATIC_SCRATCH, 2 * (size_t)m * n * elem));
+  if (ws_bytes < least) return false;
+  const GemmVariant& v = kVariants[sp.variant];
+  const int64_t held = (int64_t)(ws_bytes / ((size_t)sp.splits * elem));
+  const int64_t rows = held / n / v.tm * v.tm, cols = held / m / v.tn * v.tn;
+  if (rows > 0) *mp = rows;
+  else if (cols > 0) *np = cols;
+  else return false;
+  return true;
+}
+
 template <typename T>
 static int gemm_t(int op, int64_t m, int64_t n, int64_t k, const double* alpha,
                   const void* a, int64_t lda, const void* b, int64_t ldb, const double* beta,
@@ -1073,27 +1102,33 @@ static int gemm_t(int op, int64_t m, int64_t n, int64_t k, const double* alpha,
     return gemv_t<T>(op, m, k, alpha, a, lda, b, ldb, beta, c, ldc, ws, ws_bytes, stream);
   SplitPlan sp = split_plan(std::is_same<T, double>::value ? QEPW_C128 : QEPW_C64,
                                   op & (QEPW_OP_C | QEPW_OP_BC), m, n, k);
-  const auto bytes = [&](const SplitPlan& p) {
-    return p.splits > 1 ? (size_t)p.splits * m * n * sizeof(cplx<T>) : 0;
-  };
-  // a workspace of fixed size (the Rayleigh-Ritz steps') that the searched
-  // plan exceeds and the fixed one does not
-  if (ws_bytes < bytes(sp) && bytes(sp) > QEPW_GEMM_STATIC_SCRATCH) sp = fixed_plan(op, m, n, k);
+  int64_t mp = m, np = n;
+  if (ws_bytes < split_bytes(sp, m, n, sizeof(cplx<T>))) {
+    const SplitPlan fixed = fixed_plan(op, m, n, k);
+    if (fixed.splits == 1 ||
+        !split_panel(sp, fixed, m, n, sizeof(cplx<T>), ws_bytes, &mp, &np)) {
+      if (ws_bytes < split_bytes(fixed, m, n, sizeof(cplx<T>))) return QEPW_ERR_WORKSPACE;
+      sp = fixed;
+    }
+  }
   if (sp.splits > 65535) return QEPW_ERR_UNSUPPORTED;
-  if (ws_bytes < bytes(sp)) return QEPW_ERR_WORKSPACE;
   const GemmVariant gv = kVariants[sp.variant];
-  const int64_t mt = (m + gv.tm - 1) / gv.tm, nt = (n + gv.tn - 1) / gv.tn;
-  if (mt > 0x7fffffff || nt > 65535 || mt * nt > 0x7fffffff / sp.splits)
-    return QEPW_ERR_UNSUPPORTED;
-  const dim3 grid((unsigned)(mt * nt * sp.splits));
   const T ar = (T)alpha[0], ai = (T)alpha[1], br = (T)beta[0], bi = (T)beta[1];
+  const bool ca = (op & QEPW_OP_C) != 0, cb = (op & QEPW_OP_BC) != 0;
   cplx<T>* part = static_cast<cplx<T>*>(ws);
-  const cplx<T>* pa = static_cast<const cplx<T>*>(a);
-  const cplx<T>* pb = static_cast<const cplx<T>*>(b);
-  cplx<T>* pc = static_cast<cplx<T>*>(c);
+  for (int64_t m0 = 0; m0 < m; m0 += mp)
+    for (int64_t n0 = 0; n0 < n; n0 += np) {
+      const int64_t mm = std::min(mp, m - m0), nn = std::min(np, n - n0);
+      const int64_t mt = (mm + gv.tm - 1) / gv.tm, nt = (nn + gv.tn - 1) / gv.tn;
+      if (mt > 0x7fffffff || nt > 65535 || mt * nt > 0x7fffffff / sp.splits)
+        return QEPW_ERR_UNSUPPORTED;
+      const dim3 grid((unsigned)(mt * nt * sp.splits));
+      const cplx<T>* pa = static_cast<const cplx<T>*>(a) + (ca ? m0 * lda : m0);
+      const cplx<T>* pb = static_cast<const cplx<T>*>(b) + (cb ? n0 : n0 * ldb);
+      cplx<T>* pc = static_cast<cplx<T>*>(c) + m0 + n0 * ldc;
 #define QEPW_GEMM_TILE(CA, CB, TM, TN, WM)                                                \
   hipLaunchKernelGGL((k_cgemm<T, CA, CB, TM, TN, WM>), grid, dim3(kGemmThreads), 0, stream, \
-                     m, n, k, sp.kchunk, (unsigned)mt, (unsigned)nt, (unsigned)sp.splits, pa, \
+                     mm, nn, k, sp.kchunk, (unsigned)mt, (unsigned)nt, (unsigned)sp.splits, pa, \
                      lda, pb, ldb, pc, ldc, part, ar, ai, br, bi)
 #define QEPW_GEMM_LAUNCH(CA, CB)                                   \
   do {                                                             \
@@ -1108,19 +1143,16 @@ static int gemm_t(int op, int64_t m, int64_t n, int64_t k, const double* alpha,
       default: QEPW_GEMM_TILE(CA, CB, 64, 16, 4); break;           \
     }                                                              \
   } while (0)
-  const bool ca = (op & QEPW_OP_C) != 0, cb = (op & QEPW_OP_BC) != 0;
-  if (ca && cb) QEPW_GEMM_LAUNCH(true, true);
-  else if (ca) QEPW_GEMM_LAUNCH(true, false);
-  else if (cb) QEPW_GEMM_LAUNCH(false, true);
-  else QEPW_GEMM_LAUNCH(false, false);
+      if (ca && cb) QEPW_GEMM_LAUNCH(true, true);
+      else if (ca) QEPW_GEMM_LAUNCH(true, false);
+      else if (cb) QEPW_GEMM_LAUNCH(false, true);
+      else QEPW_GEMM_LAUNCH(false, false);
 #undef QEPW_GEMM_LAUNCH
 #undef QEPW_GEMM_TILE
-  if (sp.splits > 1) {
-    const int64_t total = m * n;
-    hipLaunchKernelGGL(k_reduce_splits<T>, dim3((unsigned)((total + 63) / 64)), dim3(256),
-                       0, stream, m, n, (int)sp.splits, part, static_cast<cplx<T>*>(c), ldc,
-                       ar, ai, br, bi);
-  }
+      if (sp.splits > 1)
+        hipLaunchKernelGGL(k_reduce_splits<T>, dim3((unsigned)((mm * nn + 63) / 64)), dim3(256),
+                           0, stream, mm, nn, (int)sp.splits, part, pc, ldc, ar, ai, br, bi);
+    }
   return hipGetLastError() == hipSuccess ? QEPW_OK : QEPW_ERR_HIP;
 }
 

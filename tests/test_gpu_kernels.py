@@ -202,6 +202,64 @@ def test_gemm_in_a_workspace_of_fixed_size():
                                 12 * m * m * 16, dv.stream_handle(torch.device(DEV))), "short")
 
 
+@pytest.mark.parametrize("m,n,k", [(512, 192, 23847), (250, 384, 40001), (520, 1040, 5001),
+                                   (64, 768, 23847)])
+def test_gemm_bits_do_not_depend_on_the_workspace(m, n, k):
+    """Products A^H B whose planned partials exceed the static scratch (FP64's):
+    in the quoted workspace, in 32 MiB and in the static scratch they give the
+    same bits (panels of rows or, one tile high, columns with the same plan)."""
+    import ctypes
+
+    from qe_python_amd import _native as nat
+    from qe_python_amd import device as dv
+    lib = nat.load()
+    dtype, code = torch.complex128, nat.C128
+    limit = int(lib.qepw_gemm_static_scratch_bytes())
+    rng = np.random.default_rng(m + n)
+    a, b, c = rand(rng, k, m), rand(rng, k, n), rand(rng, m, n)
+    ta, tb = dev_block(a, dtype), dev_block(b, dtype)
+    alpha, beta = (ctypes.c_double * 2)(0.5, -0.25), (ctypes.c_double * 2)(1.0, 0.5)
+    need = int(lib.qepw_gemm_workspace(code, nat.OP_C, m, n, k))
+    assert need > limit
+    ws = torch.empty(need, dtype=torch.uint8, device=DEV)
+    out = []
+    for size in (need, limit, None):
+        tc = dev_block(c, dtype)
+        head = (code, nat.OP_C, m, n, k, alpha, ta.data_ptr(), k, tb.data_ptr(), k, beta,
+                tc.data_ptr(), m)
+        stream = dv.stream_handle(torch.device(DEV))
+        if size is None:
+            nat.check(lib.qepw_gemm_static(*head, stream), "qepw_gemm_static")
+        else:
+            nat.check(lib.qepw_gemm(*head, ws.data_ptr(), size, stream), "qepw_gemm")
+        out.append(host_block(tc))
+    ref = (0.5 - 0.25j) * (a.conj().T @ b) + (1.0 + 0.5j) * c
+    assert np.linalg.norm(out[0] - ref) / np.linalg.norm(ref) < 1e-12
+    assert np.array_equal(out[0], out[1]) and np.array_equal(out[0], out[2])
+
+
+def test_gemm_unsplit_without_a_workspace():
+    """A shallow product that the search splits still runs without a
+    workspace."""
+    import ctypes
+
+    from qe_python_amd import _native as nat
+    from qe_python_amd import device as dv
+    lib = nat.load()
+    m, n, k = 168, 96, 168
+    assert int(lib.qepw_gemm_workspace(nat.C64, nat.OP_N, m, n, k)) > 0
+    rng = np.random.default_rng(7)
+    a, b = rand(rng, m, k), rand(rng, k, n)
+    ta, tb = dev_block(a, torch.complex64), dev_block(b, torch.complex64)
+    tc = dev_block(np.zeros((m, n), complex), torch.complex64)
+    one, zero = (ctypes.c_double * 2)(1.0, 0.0), (ctypes.c_double * 2)(0.0, 0.0)
+    nat.check(lib.qepw_gemm(nat.C64, nat.OP_N, m, n, k, one, ta.data_ptr(), m, tb.data_ptr(), k,
+                            zero, tc.data_ptr(), m, None, 0,
+                            dv.stream_handle(torch.device(DEV))), "qepw_gemm")
+    err = np.linalg.norm(host_block(tc) - a @ b) / np.linalg.norm(a @ b)
+    assert err < 2e-6 + 1e-7 * np.sqrt(k)
+
+
 def test_gemm_split_k_is_deterministic():
     from qe_python_amd import _native as nat
     from qe_python_amd import device as dv
