@@ -202,6 +202,47 @@ def test_gemm_in_a_workspace_of_fixed_size():
                                 12 * m * m * 16, dv.stream_handle(torch.device(DEV))), "short")
 
 
+@pytest.mark.parametrize("prec,m,n,k", [
+    ("c64", 384, 160, 23847), ("c64", 384, 150, 35769), ("c64", 384, 192, 35769),
+    ("c64", 512, 40, 23847), ("c128", 512, 96, 47692), ("c128", 128, 128, 23847)])
+def test_gemm_rounds_like_short_chains(prec, m, n, k):
+    """A^H B against exact sums (operands of 18 bits, for complex128 of two such
+    halves, whose products add up exactly in float64).  A sum of c terms of
+    random sign in one accumulator is about sqrt(c / 2) roundings off; chains of
+    at most 256 columns, the sum of a split's chains and the sum of the splits
+    (by four waves) make sqrt(256 / 2 + chunk / 256 / 2 + splits / 8)."""
+    import ctypes
+
+    from qe_python_amd import _native as nat
+    from qe_python_amd import device as dv
+    lib = nat.load()
+    dtype = torch.complex128 if prec == "c128" else torch.complex64
+    rng = np.random.default_rng(m + n)
+
+    def halves(rows):
+        x = rng.uniform(-1.0, 1.0, (k, rows))
+        hi = np.round(x * 2.0 ** 17) / 2.0 ** 17
+        lo = np.round((x - hi) * 2.0 ** 34) / 2.0 ** 34
+        return hi, lo if prec == "c128" else np.zeros_like(lo)
+
+    def dot(x, y):   # x^T y as a sum and what it lacks
+        return x[0].T @ y[0], (x[0].T @ y[1] + x[1].T @ y[0]) + x[1].T @ y[1]
+    ar, ai, br, bi = halves(m), halves(m), halves(n), halves(n)
+    ta, tb = dev_block(sum(ar) + 1j * sum(ai), dtype), dev_block(sum(br) + 1j * sum(bi), dtype)
+    tc = dev_block(np.zeros((m, n), complex), dtype)
+    dv.gemm(nat.OP_C, m, n, k, 1.0, ta, tb, 0.0, tc, dv.Workspace(torch.device(DEV)))
+    got = host_block(tc).astype(complex)
+    (rr, rl), (ii, il), (ri, ril), (ir, irl) = dot(ar, br), dot(ai, bi), dot(ar, bi), dot(ai, br)
+    err = np.hypot(np.linalg.norm((got.real - (rr + ii)) - (rl + il)),
+                   np.linalg.norm((got.imag - (ri - ir)) - (ril - irl))) / np.linalg.norm(got)
+    plan = (ctypes.c_int64 * 4)()
+    nat.check(lib.qepw_gemm_plan(dv.precision_code(dtype), nat.OP_C, m, n, k, plan), "plan")
+    chunk = k / plan[1]
+    unit = 2.0 ** -53 if prec == "c128" else 2.0 ** -24
+    bound = unit * np.sqrt(256 / 2 + chunk / 256 / 2 + plan[1] / 8)
+    assert err < bound, (list(plan), err, bound)
+
+
 @pytest.mark.parametrize("m,n,k", [(512, 192, 23847), (250, 384, 40001), (520, 1040, 5001),
                                    (64, 768, 23847)])
 def test_gemm_bits_do_not_depend_on_the_workspace(m, n, k):
