@@ -411,9 +411,9 @@ __global__ __launch_bounds__(256) void k_reduce_splits(
 // One-column products (n = 1: a single band's projections and projector
 // sums) as matrix-vector passes instead of MFMA tiles with one live column.
 //   k_gemv_n: sum_j A[i + j lda] b_j, one workgroup per 64 rows, a lane a row;
-//             its sixteen waves take every sixteenth column;
+//             its sixteen waves take every sixteenth column, in two chains;
 //   k_gemv_c: sum_g conj(A[g + i lda]) b_g, one workgroup per i with a
-//             fixed-order tree sum.
+//             fixed-order tree sum of four chains a thread.
 // b_j = B[j bstride], conjugated when CB.  Both finish the sum in the workgroup and
 // scale it by alpha, beta.  Deep products (gemv_direct) take k_gemv_n_split or
 // SPLIT, 256 wide, whose partials part[s * m + i] k_reduce_splits sums in a fixed
@@ -434,7 +434,7 @@ __device__ __forceinline__ void gemv_store(cplx<T>* C, int64_t i, T sr, T si, T 
   C[i] = out;
 }
 
-constexpr int kGemvWaves = 16;
+constexpr int kGemvWaves = 16;  // k_gemv_n adds them in pairs
 
 template <typename T, bool CB>
 __global__ __launch_bounds__(64 * kGemvWaves) void k_gemv_n(
@@ -445,25 +445,41 @@ __global__ __launch_bounds__(64 * kGemvWaves) void k_gemv_n(
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t i = (int64_t)blockIdx.x * 64 + lane;
   const cplx<T>* row = A + (i < m ? i : m - 1);
-  T sr = T(0), si = T(0);
-#pragma unroll 4
-  for (int64_t j = wave; j < k; j += kGemvWaves) {
-    const cplx<T> a = row[j * lda];
-    const cplx<T> b = B[j * bstride];
-    const T bi = CB ? -b.y : b.y;
-    sr += a.x * b.x - a.y * bi;
-    si += a.x * bi + a.y * b.x;
+  constexpr int W = kGemvWaves;
+  T sr = T(0), si = T(0), tr = T(0), ti = T(0);
+  auto add = [&](T& pr, T& pi, const cplx<T> x, const cplx<T> y) __attribute__((always_inline)) {
+    const T yi = CB ? -y.y : y.y;
+    pr += x.x * y.x - x.y * yi;
+    pi += x.x * yi + x.y * y.x;
+  };
+  int64_t j = wave;
+  for (; j + 3 * W < k; j += 4 * W) {
+    cplx<T> x[4], y[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      x[u] = row[(j + u * W) * lda];
+      y[u] = B[(j + u * W) * bstride];
+    }
+    add(sr, si, x[0], y[0]);
+    add(tr, ti, x[1], y[1]);
+    add(sr, si, x[2], y[2]);
+    add(tr, ti, x[3], y[3]);
   }
-  shr[wave][lane] = sr;
-  shi[wave][lane] = si;
+  for (; j < k; j += W) add(sr, si, row[j * lda], B[j * bstride]);
+  shr[wave][lane] = sr + tr;
+  shi[wave][lane] = si + ti;
   __syncthreads();
   if (wave != 0 || i >= m) return;
+  T pr[4], pi[4];
 #pragma unroll
-  for (int w = 1; w < kGemvWaves; ++w) {
-    sr += shr[w][lane];
-    si += shi[w][lane];
+  for (int q = 0; q < 4; ++q) {
+    const int w = 4 * q;
+    pr[q] = (shr[w][lane] + shr[w + 1][lane]) + (shr[w + 2][lane] + shr[w + 3][lane]);
+    pi[q] = (shi[w][lane] + shi[w + 1][lane]) + (shi[w + 2][lane] + shi[w + 3][lane]);
   }
-  gemv_store<T>(C, i, sr, si, alpha_r, alpha_i, beta_r, beta_i);
+  pr[0] = (pr[0] + pr[1]) + (pr[2] + pr[3]);
+  pi[0] = (pi[0] + pi[1]) + (pi[2] + pi[3]);
+  gemv_store<T>(C, i, pr[0], pi[0], alpha_r, alpha_i, beta_r, beta_i);
 }
 
 template <typename T, bool CB>
@@ -498,7 +514,7 @@ __global__ __launch_bounds__(SPLIT ? 256 : 1024) void k_gemv_c(
   const int64_t g0 = SPLIT ? (int64_t)blockIdx.y * kchunk : 0;
   const int64_t g1 = SPLIT && g0 + kchunk < k ? g0 + kchunk : k;
   const cplx<T>* col = A + i * lda;
-  T sr = T(0), si = T(0);
+  T cr[4] = {}, ci[4] = {};
   // (512 x 78 805 split: FP64 115 us, 126 unrolled by four; FP32 90 and 72)
   constexpr int U = SPLIT && sizeof(T) == 8 ? 1 : 4;
 #pragma unroll U
@@ -506,9 +522,21 @@ __global__ __launch_bounds__(SPLIT ? 256 : 1024) void k_gemv_c(
     const cplx<T> a = col[g];
     const cplx<T> b = B[g * bstride];
     const T bi = CB ? -b.y : b.y;
-    sr += a.x * b.x + a.y * bi;
-    si += a.x * bi - a.y * b.x;
+    cr[0] += a.x * b.x + a.y * bi;
+    ci[0] += a.x * bi - a.y * b.x;
+    if constexpr (!SPLIT) {  // the next chain's turn: register names, unrolled
+      const T r = cr[0], i0 = ci[0];
+#pragma unroll
+      for (int u = 0; u < 3; ++u) {
+        cr[u] = cr[u + 1];
+        ci[u] = ci[u + 1];
+      }
+      cr[3] = r;
+      ci[3] = i0;
+    }
   }
+  const T sr = (cr[0] + cr[1]) + (cr[2] + cr[3]);
+  const T si = (ci[0] + ci[1]) + (ci[2] + ci[3]);
   const int tid = threadIdx.x;
   shr[tid] = sr;
   shi[tid] = si;

@@ -173,6 +173,58 @@ def test_one_column_products_at_their_edges(prec, op):
             assert err < tol, (m, k, err)
 
 
+def chunked_gemv(a, b, splits, threads):
+    """a (rows, k), b (k) complex64 summed in FP32 as a split product does:
+    chunks of K, in each the chains of ``threads`` threads and their tree sum;
+    the chunks by four waves, and those in order."""
+    f = np.float32
+    k = len(b)
+    chunk = -(-k // splits)
+    total = [[np.zeros(len(a), f), np.zeros(len(a), f)] for _ in range(4)]
+    for z in range(-(-k // chunk)):
+        part = np.zeros((2, threads, len(a)), f)
+        for g in range(z * chunk, min(k, (z + 1) * chunk), threads):
+            top = min(g + threads, min(k, (z + 1) * chunk))
+            x = a[:, g:top].T.astype(complex)
+            y = b[g:top, None].astype(complex)
+            re = (x.real * y.real - (x.imag * y.imag).astype(f).astype(float)).astype(f)
+            im = (x.real * y.imag + (x.imag * y.real).astype(f).astype(float)).astype(f)
+            part[0, :top - g] += re
+            part[1, :top - g] += im
+        h = threads // 2
+        while h:
+            part[:, :h] += part[:, h:2 * h]
+            h //= 2
+        for c in range(2):
+            total[z % 4][c] += part[c, 0]
+    return sum((t[0] for t in total[1:]), total[0][0]) + 1j * sum((t[1] for t in total[1:]),
+                                                                  total[0][1]).astype(complex)
+
+
+@pytest.mark.parametrize("op,m,k,splits,threads", [
+    ("N", 2951, 16, 2, 1), ("N", 2951, 168, 21, 1), ("N", 2951, 256, 32, 1), ("N", 2951, 384, 48, 1),
+    ("C", 64, 23847, 16, 256), ("C", 64, 10118, 10, 256)])
+def test_one_column_products_round_like_split_ones(op, m, k, splits, threads):
+    """Unsplit matrix-vector products in FP32 are no further from the exact sums
+    than chunks of 8 columns or 1024 rows summed apart (5% for the spread of
+    some 700 to 12 000 sums)."""
+    from qe_python_amd import _native as nat
+    from qe_python_amd import device as dv
+    ws = dv.Workspace(torch.device(DEV))
+    got = want = 0.0
+    for seed in range(2 if op == "N" else 12):
+        rng = np.random.default_rng(seed)
+        a, b = rand(rng, m, k).astype(np.complex64), rand(rng, k, 1).astype(np.complex64)
+        tc = dev_block(np.zeros((m, 1)), torch.complex64)
+        dv.gemm(nat.OP_N if op == "N" else nat.OP_C, m, 1, k, 1.0,
+                dev_block(a if op == "N" else a.conj().T, torch.complex64),
+                dev_block(b, torch.complex64), 0.0, tc, ws)
+        exact = (a.astype(complex) @ b.astype(complex))[:, 0]
+        got += np.linalg.norm(host_block(tc)[:, 0] - exact) ** 2
+        want += np.linalg.norm(chunked_gemv(a, b[:, 0], splits, threads) - exact) ** 2
+    assert got <= 1.05 ** 2 * want, (got / want) ** 0.5
+
+
 def test_gemm_in_a_workspace_of_fixed_size():
     """A product whose planned partials exceed the static scratch runs in the
     Rayleigh-Ritz steps' workspace with fewer splits; less than 21 splits of
