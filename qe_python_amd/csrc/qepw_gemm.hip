@@ -51,6 +51,7 @@ template <> struct Mfma<float> {
 };
 
 constexpr int kGemmThreads = 256;
+constexpr int64_t kMaxLaunch = 0xffffffff;  // threads of a launch
 constexpr int kPad = 1;
 // K depth of one LDS step: 16 columns, eight of the larger FP64 tiles (whose
 // steps are long enough, and whose LDS would halve the workgroups of a CU).
@@ -575,8 +576,10 @@ static GemvPlan gemv_plan(bool ca, int64_t m, int64_t k) {
 // Whether a one-column product runs unsplit: where it fills the chip, or ends sooner
 // than a second kernel starts.  Beyond, split and unsplit: FP64 64 x 2000 13.9 and
 // 29.1 us, FP32 78 805 x 512 56 and 65; A^H FP64 64 x 100 000 21 and 35, 512 x 78 805
-// 115 and 122.
+// 115 and 122.  (A launch runs fewer than 2^32 threads, and more wrap without an
+// error: the rows beyond take the split kernels, of 256 threads.)
 static bool gemv_direct(bool ca, int64_t m, int64_t k) {
+  if ((ca ? m : (m + 63) / 64) > kMaxLaunch / (64 * kGemvWaves)) return false;
   return ca ? k <= 8192 || (m >= 64 && k <= 32768) : k <= 384;
 }
 
@@ -920,7 +923,7 @@ static int force_product_t(int64_t npw, int64_t nproj, int64_t nb, const void* p
       force_variant(std::is_same<T, double>::value ? QEPW_C128 : QEPW_C64, npw, nproj, nb);
   const GemmVariant& v = kVariants[variant];
   const int64_t mt = (npw + v.tm - 1) / v.tm, nt = (nproj + v.tn - 1) / v.tn;
-  if (mt > 0x7fffffff / nt) return QEPW_ERR_UNSUPPORTED;
+  if (mt > kMaxLaunch / kGemmThreads / nt) return QEPW_ERR_UNSUPPORTED;
   const dim3 grid((unsigned)(mt * nt));
   const cplx<T>* x = static_cast<const cplx<T>*>(psi);
   const cplx<T>* b = static_cast<const cplx<T>*>(proj);
@@ -1117,7 +1120,6 @@ static int gemv_t(int op, int64_t m, int64_t k, const double* alpha, const void*
   const T ar = (T)alpha[0], ai = (T)alpha[1], br = (T)beta[0], bi = (T)beta[1];
   const bool direct = gemv_direct(ca, m, k);
   if (!ca && direct) {
-    if ((m + 63) / 64 > 0x7fffffff) return QEPW_ERR_UNSUPPORTED;
     const dim3 grid((unsigned)((m + 63) / 64));
     if (cb)
       hipLaunchKernelGGL((k_gemv_n<T, true>), grid, dim3(64 * kGemvWaves), 0, stream, m, k, pa,
@@ -1201,7 +1203,7 @@ static int gemm_t(int op, int64_t m, int64_t n, int64_t k, const double* alpha,
     for (int64_t n0 = 0; n0 < n; n0 += np) {
       const int64_t mm = std::min(mp, m - m0), nn = std::min(np, n - n0);
       const int64_t mt = (mm + gv.tm - 1) / gv.tm, nt = (nn + gv.tn - 1) / gv.tn;
-      if (mt > 0x7fffffff || nt > 65535 || mt * nt > 0x7fffffff / sp.splits)
+      if (mt > 0x7fffffff || nt > 65535 || mt * nt > kMaxLaunch / kGemmThreads / sp.splits)
         return QEPW_ERR_UNSUPPORTED;
       const dim3 grid((unsigned)(mt * nt * sp.splits));
       const cplx<T>* pa = static_cast<const cplx<T>*>(a) + (ca ? m0 * lda : m0);

@@ -225,6 +225,24 @@ def test_one_column_products_round_like_split_ones(op, m, k, splits, threads):
     assert got <= 1.05 ** 2 * want, (got / want) ** 0.5
 
 
+@pytest.mark.parametrize("op,m,k", [("C", (1 << 22) + 3, 2), ("N", (1 << 28) + 5, 1)])
+def test_one_column_products_of_the_most_rows(op, m, k):
+    """Outputs beyond 2^32 work-items of the workgroups of 1024 that short
+    matrix-vector products run in (small integers: exact)."""
+    from qe_python_amd import _native as nat
+    from qe_python_amd import device as dv
+    ramp = torch.arange(m, device=DEV) % 1000
+    a = torch.stack([ramp - 3 * j for j in range(k)]).to(torch.complex64)   # (k, m)
+    b = torch.arange(1, k + 1, device=DEV).to(torch.complex64)[None]
+    ref = sum((j + 1) * (ramp - 3 * j) for j in range(k))
+    c = torch.full((1, m), 7.0 + 0j, dtype=torch.complex64, device=DEV)
+    if op == "C":
+        a = a.T.contiguous()
+    dv.gemm(nat.OP_C if op == "C" else nat.OP_N, m, 1, k, 1.0, a, b, 0.0, c,
+            dv.Workspace(torch.device(DEV)))
+    assert torch.equal(c[0].real.long(), ref) and not torch.any(c[0].imag)
+
+
 def test_gemm_in_a_workspace_of_fixed_size():
     """A product whose planned partials exceed the static scratch runs in the
     Rayleigh-Ritz steps' workspace with fewer splits; less than 21 splits of
