@@ -659,14 +659,23 @@ static bool group_size(int n) {
   return false;
 }
 
+// Workgroups of a problem in the grouped stages.
+static int64_t group_planes(const Plan& p, int nb) { return (int64_t)p.n3 * nb; }
+static int64_t group_sticks(const Plan& p, int nb) {
+  const int teams = team_teams(p.n3);
+  return (int64_t)((p.sphere.nst + teams - 1) / teams) * nb;
+}
+
 // Whether a problem's FFT phase can join a grouped launch: square planes and
 // a z length among QEPW_GROUP_SIZES, the team plane path, its whole band
-// block in one workspace chunk.
+// block in one workspace chunk and one launch.
 template <typename T>
 static bool group_eligible(const Plan& p, int nb, size_t ws_bytes) {
   const StickTables& st = p.sphere;
   if (!(p.n1 == p.n2 && group_size(p.n1) && group_size(p.n3))) return false;
   if (plane_path<T>(p, st) != kPathTeam) return false;
+  if (group_planes(p, nb) > plane_group_most<T>() || group_sticks(p, nb) > kMaxLaunch / kTeamThreads)
+    return false;
   return (size_t)nb * band_bytes_t<T>(p, st) <= ws_bytes && nb <= 65535;
 }
 
@@ -676,7 +685,7 @@ int apply_local_group_t(int count, const Plan* const* plans, const void* const* 
                         const void* const* kinetics, void* const* results, const int64_t* ldr,
                         void* const* workspaces, const size_t* ws_bytes, hipStream_t stream) {
   // problems that cannot join run on their own; the rest in groups of at most
-  // kMaxFftGroup, three launches per group
+  // kMaxFftGroup and what a launch holds, three launches per group
   std::vector<int> members;
   for (int i = 0; i < count; ++i) {
     if (nb[i] <= 0) continue;
@@ -689,8 +698,15 @@ int apply_local_group_t(int count, const Plan* const* plans, const void* const* 
       if (rc != QEPW_OK) return rc;
     }
   }
-  for (size_t g0 = 0; g0 < members.size(); g0 += kMaxFftGroup) {
-    const int m = (int)std::min<size_t>(kMaxFftGroup, members.size() - g0);
+  int m = 0;
+  for (size_t g0 = 0; g0 < members.size(); g0 += m) {
+    int64_t planes = 0, sticks = 0;
+    for (m = 0; m < kMaxFftGroup && g0 + m < members.size(); ++m) {
+      const int i = members[g0 + m];
+      planes += group_planes(*plans[i], nb[i]);
+      sticks += group_sticks(*plans[i], nb[i]);
+      if (planes > plane_group_most<T>() || sticks > kMaxLaunch / kTeamThreads) break;
+    }
     StickGroupArgs<T> sa{};
     sa.count = m;
     size_t stick_lds = 0;
@@ -725,7 +741,6 @@ int apply_local_group_t(int count, const Plan* const* plans, const void* const* 
       gnb[j] = nb[i];
     }
     sa.start[m] = (int)stotal;
-    if (stotal > 0x7fffffff) return QEPW_ERR_UNSUPPORTED;
     allow_lds(reinterpret_cast<const void*>(&k_sticks_group<T, false>), stick_lds);
     allow_lds(reinterpret_cast<const void*>(&k_sticks_group<T, true>), stick_lds);
     hipLaunchKernelGGL((k_sticks_group<T, false>), dim3((unsigned)stotal), dim3(kTeamThreads),

@@ -51,7 +51,6 @@ template <> struct Mfma<float> {
 };
 
 constexpr int kGemmThreads = 256;
-constexpr int64_t kMaxLaunch = 0xffffffff;  // threads of a launch
 constexpr int kPad = 1;
 // K depth of one LDS step: 16 columns, eight of the larger FP64 tiles (whose
 // steps are long enough, and whose LDS would halve the workgroups of a CU).

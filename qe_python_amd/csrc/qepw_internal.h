@@ -10,6 +10,7 @@
 namespace qepw {
 
 constexpr int kMaxLdsBytes = 160 * 1024;
+constexpr int64_t kMaxLaunch = 0xffffffff;  // threads of a launch and dimension
 
 // Raises a kernel's dynamic LDS limit where a launch needs more than the 64 KB
 // every kernel may use (the call costs a microsecond of a launch).
@@ -73,6 +74,8 @@ template <typename T>
 bool launch_density_stage(const Plan& p, const StickTables& st, cplx<T>* work, int64_t bstride,
                           const double* weights, int nb, int most, int* slices, bool accumulate,
                           double* partial, hipStream_t stream);
+// Planes (of all bands and problems) of one grouped launch.
+template <typename T> int64_t plane_group_most();
 template <typename T>
 int launch_plane_group(int count, const Plan* const* plans, cplx<T>* const* work,
                        const int64_t* bstride, const T* const* V, const int* nb,

@@ -887,6 +887,10 @@ bool launch_density_stage(const Plan& p, const StickTables& st, cplx<T>* work, i
   return false;
 }
 
+template <typename T> int64_t plane_group_most() {
+  return kMaxLaunch / (64 * plane_group_waves<T>());
+}
+
 // The grouped plane stage of ``count`` square problems whose lengths are among
 // QEPW_GROUP_SIZES (nb bands each).
 template <typename T>
@@ -913,7 +917,7 @@ int launch_plane_group(int count, const Plan* const* plans, cplx<T>* const* work
                                  (size_t)plane_group_waves<T>() * per) *
                             (p.n1 + 1) * sizeof(cplx<T>));
   }
-  if (total > 0x7fffffff || lds > (size_t)kMaxLdsBytes) return QEPW_ERR_UNSUPPORTED;
+  if (total > plane_group_most<T>() || lds > (size_t)kMaxLdsBytes) return QEPW_ERR_UNSUPPORTED;
   g.start[count] = (int)total;
   allow_lds(reinterpret_cast<const void*>(&k_plane_group<T>), lds);
   hipLaunchKernelGGL(k_plane_group<T>, dim3((unsigned)total), dim3(64 * plane_group_waves<T>()),

@@ -391,3 +391,31 @@ def test_z_lines_of_the_largest_lengths(n3):
     grid[(slice(None),) + tuple((m % np.array(shape)).T)] = x.T
     dens = (np.abs(np.fft.ifftn(grid, axes=(1, 2, 3), norm="forward")) ** 2).sum(0)
     np.testing.assert_allclose(rho, dens, rtol=0, atol=1e-12 * dens.max())
+
+
+def test_grouped_bands_beyond_one_launch():
+    """Problems whose planes together pass 2^32 threads of the grouped plane
+    kernel (12 waves a plane in complex128), with one that passes them alone
+    (its bands run ungrouped): the same bits as problem by problem."""
+    import torch
+
+    from qe_python_amd import device as dv
+    from qe_python_amd.basis import LocalPotentialWorkspace
+    dev = torch.device("cuda", torch.cuda.current_device())
+    shape = (36, 36, 96)
+    m = np.array([[0, 0, 0], [1, 0, 2], [0, -1, 1], [-2, 3, 0], [1, 0, -5]], dtype=np.int32)
+    gen = torch.Generator(device=dev).manual_seed(5)
+    items, alone = [], []
+    for nb in (30000, 29000, 60000, 100):
+        plan = LocalPotentialWorkspace(m, shape).plan
+        x = torch.randn((nb, len(m)), dtype=torch.complex128, device=dev, generator=gen)
+        v = torch.randn(shape[::-1], dtype=torch.float64, device=dev, generator=gen)
+        kin = torch.rand(len(m), dtype=torch.float64, device=dev, generator=gen)
+        y, z = torch.full_like(x, 9.0), torch.full_like(x, 9.0)
+        items.append((plan, x, y, v, kin, dv.Workspace(dev)))
+        plan.apply_local(x, z, v, kin, dv.Workspace(dev))
+        alone.append(z)
+    assert 96 * 59000 * 768 > 1 << 32 and 96 * 60000 * 768 > 1 << 32
+    dv.DeviceFFTPlan.apply_local_group(items)
+    for (_, _, y, _, _, _), z in zip(items, alone):
+        assert torch.equal(y, z)
