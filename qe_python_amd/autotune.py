@@ -156,10 +156,15 @@ def tune(reps: int = 10, device=None, log=print):
 
 def load_table(path: Path | str | None = None) -> int:
     """Install a tuned table's rules (a rule replaces the built-in choice only
-    where it was measured faster).  Returns the number of rules set."""
+    where it was measured faster), or, without ``path`` and without a table at
+    ``TABLE``, the built-in choice alone.  Returns the number of rules set."""
     from . import device as dv
-    path = Path(path) if path is not None else TABLE
+    default = path is None
+    path = TABLE if default else Path(path)
     if not path.exists():
+        if default:
+            nat.load().qepw_gemm_clear_rules()
+            dv.forget_gemm_plans()
         return 0
     table = json.loads(path.read_text())
     lib = nat.load()
