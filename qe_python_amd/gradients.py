@@ -109,9 +109,17 @@ class BandEnergyModel:
         return out
 
     def position_gradient(self, psi, proj, coupled, weights):
-        """dE/dtau (natom, 3) float64."""
+        """dE/dtau (natom, 3) float64 from (nb, npw) device-order psi, the
+        packed projectors, D O and the float64 band weights."""
         nb = psi.shape[0]
         p = proj.shape[0]
+        if proj.dtype != psi.dtype or coupled.dtype != psi.dtype:
+            raise ValueError("psi, proj and coupled must share one complex dtype")
+        if weights.dtype != torch.float64 or weights.numel() < nb:
+            raise ValueError("one float64 weight per band is required")
+        if (p < self.natom * self.nch or psi.shape[1] < self.npw or proj.shape[1] < self.npw
+                or coupled.shape[0] < nb or coupled.shape[1] < p):
+            raise ValueError("psi, proj and coupled must be (nb, npw), (P, npw) and (nb, P)")
         lib = nat.load()
         prec = dv.precision_code(psi.dtype)
         out = torch.empty((self.natom, 3), dtype=torch.float64, device=self.device)

@@ -231,3 +231,22 @@ def test_argument_errors(small):
         band_energy(model, p, v[:-1], t, f)
     with pytest.raises(ValueError):
         band_energy(model, p, v, t, f[:-1])
+
+
+def test_position_gradient_checks_its_operands(small):
+    """BandEnergyModel.position_gradient refuses operands of another dtype or
+    smaller than the sizes that the kernel reads."""
+    s, psi, f, model, _ = small
+    nb, p = len(f), model.natom * model.nch
+    good = {"psi": torch.ones((nb, model.npw), dtype=torch.complex128, device=DEV),
+            "proj": torch.ones((p, model.npw), dtype=torch.complex128, device=DEV),
+            "coupled": torch.ones((nb, p), dtype=torch.complex128, device=DEV),
+            "weights": torch.ones(nb, dtype=torch.float64, device=DEV)}
+    assert model.position_gradient(**good).shape == (model.natom, 3)
+    bad = [("proj", good["proj"].to(torch.complex64)), ("coupled", good["coupled"].to(torch.complex64)),
+           ("weights", good["weights"].float()), ("weights", good["weights"][1:]),
+           ("psi", good["psi"][:, 1:]), ("proj", good["proj"][:, 1:]), ("proj", good["proj"][1:]),
+           ("coupled", good["coupled"][1:]), ("coupled", good["coupled"][:, 1:])]
+    for name, value in bad:
+        with pytest.raises(ValueError):
+            model.position_gradient(**{**good, name: value})
