@@ -93,6 +93,16 @@ class BandEnergyModel:
         dv.gemm(nat.OP_N, self.npw, nb, p, 1.0, proj, coupled, 1.0, hpsi, self.workspace)
         return hpsi, overlap, coupled
 
+    def scale_rows(self, src, dst, s=None, sstride=0, cfac=None):
+        """dst[b, g] = s[g sstride] cfac[b] src[b, g] (each factor optional):
+        with s one direction of k+G, the blocks of dO/dtau."""
+        rc = nat.load().qepw_scale_rows(
+            dv.precision_code(src.dtype), src.data_ptr(), dv.ld_of(src),
+            None if s is None else s.data_ptr(), sstride,
+            None if cfac is None else cfac.data_ptr(), dst.data_ptr(), dv.ld_of(dst),
+            self.npw, src.shape[0], dv.stream_handle(self.device))
+        nat.check(rc, "qepw_scale_rows")
+
     def density(self, psi, weights, scale):
         """scale * sum_b weights[b] |psi_b(r)|^2, (n3, n2, n1) float64."""
         lib = nat.load()

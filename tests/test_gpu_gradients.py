@@ -250,3 +250,30 @@ def test_position_gradient_checks_its_operands(small):
     for name, value in bad:
         with pytest.raises(ValueError):
             model.position_gradient(**{**good, name: value})
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.complex128, 1e-12), (torch.complex64, 2e-5)])
+def test_projector_forces_of_given_derivatives(small, dtype, tol):
+    """qepw_projector_forces on the blocks dO_c = i B^H (q_c psi), made with
+    BandEnergyModel.scale_rows, against position_gradient, which sums over the
+    bands first (bars of the gradients above)."""
+    from qe_python_amd import _native as nat
+    from qe_python_amd import device as dv
+    s, psi, f, model, _ = small
+    lib = nat.load()
+    nb, p = len(f), model.natom * model.nch
+    x = torch.from_numpy(np.ascontiguousarray(psi[model.plan.perm].T)).to(DEV).to(dtype)
+    proj = model.projectors(torch.tensor(s.projectors.positions, device=DEV), dtype)
+    v = torch.zeros(model.shape[::-1], dtype=dv.real_dtype(dtype), device=DEV)
+    _, _, coupled = model.apply(x, v, proj)
+    w = torch.tensor(f, device=DEV)
+    scaled, blocks = torch.empty_like(x), torch.empty((3, nb, p), dtype=dtype, device=DEV)
+    for c in range(3):
+        model.scale_rows(x, scaled, s=model.gk[:, c], sstride=3)
+        dv.gemm(nat.OP_C, p, nb, model.npw, 1j, proj, scaled, 0.0, blocks[c], model.workspace)
+    out = torch.full((model.natom, 3), float("nan"), dtype=torch.float64, device=DEV)
+    nat.check(lib.qepw_projector_forces(
+        dv.precision_code(dtype), blocks.data_ptr(), p, nb * p, coupled.data_ptr(),
+        dv.ld_of(coupled), w.data_ptr(), nb, model.offsets.data_ptr(), model.natom,
+        out.data_ptr(), dv.stream_handle(torch.device(DEV))), "qepw_projector_forces")
+    assert rel(out.cpu(), model.position_gradient(x, proj, coupled, w).cpu()) < tol
