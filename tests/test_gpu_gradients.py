@@ -277,3 +277,41 @@ def test_projector_forces_of_given_derivatives(small, dtype, tol):
         dv.ld_of(coupled), w.data_ptr(), nb, model.offsets.data_ptr(), model.natom,
         out.data_ptr(), dv.stream_handle(torch.device(DEV))), "qepw_projector_forces")
     assert rel(out.cpu(), model.position_gradient(x, proj, coupled, w).cpu()) < tol
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.complex128, 1e-12), (torch.complex64, 2e-5)])
+@pytest.mark.parametrize("npw,nch,natom,nb", [(12011, 29, 7, 97), (23847, 10, 25, 127)])
+def test_position_gradient_on_large_tiles(dtype, tol, npw, nch, natom, nb):
+    """qepw_position_gradient where the product runs on 64 x 64 tiles (the
+    workspace holds two partial sums a tile row), with ragged rows, bands and
+    projectors, against the sums over dO_c = i B^H (q_c psi) in NumPy."""
+    from qe_python_amd import _native as nat
+    from qe_python_amd import device as dv
+    lib = nat.load()
+    rng = np.random.default_rng(npw + nb)
+    p = nch * natom
+
+    def block(rows, cols):
+        x = rng.standard_normal((cols, rows)) + 1j * rng.standard_normal((cols, rows))
+        return torch.from_numpy(x).to(DEV).to(dtype)
+    psi, proj, coupled = block(npw, nb), block(npw, p), block(p, nb)
+    q, f = rng.standard_normal((npw, 3)), rng.standard_normal(nb)
+    qd, fd = torch.from_numpy(q).to(DEV), torch.from_numpy(f).to(DEV)
+    off = torch.arange(0, p + 1, nch, dtype=torch.int32, device=DEV)
+    out = torch.full((natom, 3), float("nan"), dtype=torch.float64, device=DEV)
+    prec, size = dv.precision_code(dtype), 16 if dtype == torch.complex128 else 8
+    need = lib.qepw_position_gradient_workspace(prec, npw, p, nb)
+    weighted = -(-p * nb * size // 256) * 256
+    assert need == weighted + 3 * p * 2 * -(-npw // 64) * 8
+    ws = torch.empty(need, dtype=torch.uint8, device=DEV)
+    nat.check(lib.qepw_position_gradient(
+        prec, psi.data_ptr(), npw, nb, proj.data_ptr(), npw, p, coupled.data_ptr(), p,
+        fd.data_ptr(), qd.data_ptr(), npw, off.data_ptr(), natom, out.data_ptr(),
+        ws.data_ptr(), need, dv.stream_handle(torch.device(DEV))), "qepw_position_gradient")
+    psi, proj, coupled = (x.cpu().numpy().astype(complex).T for x in (psi, proj, coupled))
+    ref = np.empty((natom, 3))
+    for c in range(3):
+        d = 1j * proj.conj().T @ (q[:, c, None] * psi)
+        ref[:, c] = (2.0 * ((d.conj() * coupled).real @ f)).reshape(natom, nch).sum(1)
+    scale = max(np.linalg.norm(ref), 2.0 * np.sqrt(2.0 * npw * p * nb) / 10)
+    assert np.linalg.norm(out.cpu().numpy() - ref) <= tol * scale
