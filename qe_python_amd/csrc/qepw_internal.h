@@ -57,10 +57,21 @@ int inverse_real(const Plan& p, const void* grid_g, void* out_real, void* worksp
                  size_t ws_bytes, hipStream_t stream);
 
 // qepw_plane_c128.hip, qepw_plane_c64.hip (the xy-plane stage, qepw_plane.h)
-// Whether the lines of length n load their twiddles instead of holding them:
-// held, FP64 lines spill or halve the waves a CU runs (96^2, 110 bands: 46 of
-// 168 registers' worth spilled); nine twiddles of lines up to 72 still fit (72^2,
-// 128 bands: 280 us held, 292 us loaded; 60^2: 216 and 209 us).
+// Whether the lines of length n load their twiddles instead of holding them.
+// Held, long FP64 lines spill or halve the waves a CU runs.  Squares, FFT phase of
+// 24 planes of 128 bands in FP64, loaded and held, us: 36^2 42.9 and 40, 48^2 62
+// and 62, 60^2 88 and 87, 72^2 100 and 96, 80^2 155 and 139, 81^2 178 and 156, but
+// 75^2 (fifteen twiddles) 221 and 284, 90^2 186 and 207, 96^2 215 and 231, 108^2 275
+// and 334, 128^2 452 and 683; FP32 72^2 75 and 66, 108^2 155 and 145, 128^2 346 and
+// 378.
+constexpr bool plane_square_table(int n, bool fp64) {
+  const int m = team_L(n) > 0 ? n / team_L(n) : 0;
+  return fp64 ? m > 10 || n > 81 : m >= 15;
+}
+// The kernels of any two lengths share their registers among all: FP64 lines hold
+// nine twiddles up to 72 and load all others (64 bands, loaded and held as above: 81
+// x 64 x 30 99 and 113 us, 50 x 64 x 40 79 and 85, 60 x 80 x 48 154 and 163, 36 x 40
+// x 160 120 and 118).
 constexpr bool plane_lane_table(int n, bool fp64) {
   const int m = team_L(n) > 0 ? n / team_L(n) : 0;
   return fp64 ? !(m == 9 && n <= 72) : m >= 15;

@@ -52,7 +52,8 @@ template <int N> struct PlaneLine {
 // The twiddles between the two halves of a team FFT, w_N^(t k) for lane t.
 // Held in registers (TeamTwiddles), or loaded where they are used from a table
 // in the order of the lanes ([k M + t] for the DIF half's k < L, N + [k L + t]
-// for the DIT half's k < M) that stays in the L1 (plane_lane_table).
+// for the DIT half's k < M) that stays in the L1 (plane_lane_table and, of the
+// squares, plane_square_table).
 template <typename T, int N, bool LOAD = plane_lane_table(N, sizeof(T) == 8)>
 struct PlaneTwiddles {
   TeamTwiddles<T, N> reg;
@@ -79,6 +80,9 @@ template <typename T, int N> struct PlaneTwiddles<T, N, true> {
   }
 };
 
+template <typename T, int N>
+using SquareTwiddles = PlaneTwiddles<T, N, plane_square_table(N, sizeof(T) == 8)>;
+
 // Backward (DIF) and forward (DIT) team FFTs of one line through its LDS line
 // S, split as in qepw_regfft.h: b, slots t + M s of lanes t < M; a, slots
 // t + L k of lanes t < L.
@@ -103,8 +107,8 @@ __device__ __forceinline__ void plane_backward(int t, cplx<T>* S, TW& tw,
   }
 }
 
-template <typename T, int N>
-__device__ __forceinline__ void plane_forward(int t, cplx<T>* S, PlaneTwiddles<T, N>& tw,
+template <typename T, int N, typename TW>
+__device__ __forceinline__ void plane_forward(int t, cplx<T>* S, TW& tw,
                                               cplx<T> (&a)[PlaneLine<N>::M],
                                               cplx<T> (&b)[PlaneLine<N>::L]) {
   constexpr int L = PlaneLine<N>::L, M = PlaneLine<N>::M;
@@ -214,9 +218,9 @@ __device__ __forceinline__ void plane_row_slots(const PlaneArgs<T>& g, int np2,
 // Rows, RB per team (RB teams >= n2): backward x-FFT (inputs only at occupied
 // columns), V, forward x-FFT (outputs only at occupied columns).  np2: the
 // LDS column stride.  Called by the whole workgroup (it synchronises).
-template <typename T, int N1, bool PRUNE, int RB>
+template <typename T, int N1, bool PRUNE, int RB, typename TW>
 __device__ __forceinline__ void plane_rows(const PlaneArgs<T>& g, int z, cplx<T>* Q, int n2,
-                                           int np2, int waves, PlaneTwiddles<T, N1>& tw,
+                                           int np2, int waves, TW& tw,
                                            const int (&cq)[PlaneLine<N1>::L]) {
   using G = PlaneLine<N1>;
   constexpr int L = G::L, M = G::M, NP = N1 + 1;
@@ -272,9 +276,9 @@ __device__ __forceinline__ void plane_rows(const PlaneArgs<T>& g, int z, cplx<T>
 // Forward y-FFT of every occupied column, in place; only the kept y slots,
 // which hold every stick, are computed, and the sticks among them go straight
 // to the stick buffer.
-template <typename T, int N2, bool PRUNE>
+template <typename T, int N2, bool PRUNE, typename TW>
 __device__ __forceinline__ void plane_cols_forward(const PlaneArgs<T>& g, cplx<T>* w, cplx<T>* Q,
-                                                   int waves, PlaneTwiddles<T, N2>& tw) {
+                                                   int waves, TW& tw) {
   using G = PlaneLine<N2>;
   constexpr int L = G::L, M = G::M, NP = N2 + 1;
   constexpr unsigned KEEP = PRUNE ? G::pruned : G::all;
@@ -322,9 +326,13 @@ template <int N, bool PRUNE> constexpr int plane_kept() {
 // waves, 403 with six): four while several workgroups share a CU (two are up to
 // 5% faster below 64^2, and slower for a few bands), twelve where an FP64
 // plane's LDS admits one or two per CU and four waves' rows would not fit
-// their registers (96^2: 864 us, 894 with three).  The kernels of four waves
-// before, with exchange lines of their own above 72^2, took: FP64 75^2 1007 us
-// (now 732), 80^2 662 (541), 90^2 1029 (797), 100^2 1298 (773), 108^2 1441
+// their registers.  24 planes of 128 bands in FP64, four (what the rows need where
+// that is more) and twelve, us: 60^2 88 and 114, 72^2 96 and 128, 80^2 155 and 164,
+// 75^2 (whose four waves' rows do not fit: eight) 249 and 221, 81^2 (eight) 162 and
+// 178, 90^2 190 and 186, 96^2 246 and 215, 128^2 569 and 452; FP32, four and eight,
+// 108^2 145 and 143, 120^2 180 and 161.  The kernels of four waves before, with
+// exchange lines of their own above 72^2, took: FP64 75^2 1007 us
+// (now 732), 80^2 662 (475), 90^2 1029 (797), 100^2 1298 (773), 108^2 1441
 // (890), 120^2 1348 (822), 128^2 in the split stage 3323 (1034); FP32 90^2 386
 // (322), 108^2 502 (380), 120^2 464 (361), 128^2 2640 (684).
 template <typename T, int N, bool PRUNE> constexpr int plane_waves() {
@@ -347,7 +355,7 @@ __device__ __forceinline__ void plane_square_body(const PlaneArgs<T>& g, int z, 
   cplx<T>* w = g.work + b * g.bstride + (int64_t)z * g.nst;
   constexpr int teams = W * PlaneLine<N>::per_wave;
   // the per-lane tables of all passes, fetched while the sticks are
-  PlaneTwiddles<T, N> tw;
+  SquareTwiddles<T, N> tw;
   tw.load(PlaneLane<N>().t, g.tw1);
   int cq[PlaneLine<N>::L];
   plane_row_slots<T, N, PRUNE>(g, N + 1, cq);
@@ -565,16 +573,19 @@ __device__ __forceinline__ void density_store(const DensityArgs<T>& d, int z, in
   }
 }
 
-// Whether the square kernel's rows have exchange lines of their own.
+// Whether the square kernel's rows have exchange lines of their own, measured
+// where the LDS holds them beside the columns: 24 planes of 128 bands, with and
+// without, us: FP64 60^2 71 and 87, 72^2 75 and 103, 80^2 101 and 106, 90^2 124 and
+// 128, 81^2 86 and 84, 75^2 118 and 122, 100^2 121 and 144 (the last two not taken);
+// FP32 40^2 35 and 38, 54^2 47 and 47, 72^2 62 and 68.
 template <typename T> constexpr bool density_direct(int n, bool prune) {
   return sizeof(T) == 8 ? n <= 72 || (prune && (n == 80 || n == 81 || n == 90)) : n <= 54;
 }
 
-// Whether the square kernel holds the twiddles of a line that the plane stage
-// loads (60^2, 128 bands: 154 us loaded, 144 held).
-template <typename T> constexpr bool density_held(int n) { return sizeof(T) == 8 && n <= 72; }
-
-// Waves of the square kernel's workgroup.
+// Waves of the square kernel's workgroup: four up to 72 (24 planes of 128 bands,
+// four and eight, us: FP64 27^2 30 and 32, 48^2 46 and 45, 60^2 71 and 63, 72^2 75
+// and 68; FP32 36^2 28 and 32, 72^2 68 and 58), then eight where the lines leave one
+// workgroup a CU (90^2 124, twelve 442: no room) or twelve (96^2 124, eight 123).
 template <typename T, int N, bool PRUNE> constexpr int density_waves() {
   constexpr bool direct = density_direct<T>(N, PRUNE);
   int w = N <= 72 ? 4 : direct || (N <= 80 && N != 75) ? 8 : 12;
@@ -603,7 +614,7 @@ __global__ __launch_bounds__(64 * W, (density_simd_waves<T, N, PRUNE>())) void k
   constexpr int A = RB * PlaneLine<N>::M;
   const PlaneArgs<T>& g = d.plane;
   const int z = blockIdx.x, b0 = blockIdx.y * d.per, b1 = min(d.nb, b0 + d.per);
-  PlaneTwiddles<T, N, !density_held<T>(N) && plane_lane_table(N, sizeof(T) == 8)> tw;
+  SquareTwiddles<T, N> tw;
   tw.load(PlaneLane<N>().t, g.tw1);
   int cq[PlaneLine<N>::L];
   plane_row_slots<T, N, PRUNE>(g, N + 1, cq);
@@ -693,13 +704,11 @@ __global__ __launch_bounds__(64 * kPlaneAnyWaves, 3) void k_density_any(DensityA
 }
 
 // ---- host side ------------------------------------------------------------------
-template <typename T> const cplx<T>* plane_twiddles(const Plan& p, int axis);
-static inline const double2* line_twiddles(const Plan& p, double) { return p.d_tw64[0]; }
-static inline const float2* line_twiddles(const Plan& p, float) { return p.d_tw32[0]; }
+template <typename T> const cplx<T>* plane_twiddles(const Plan& p, int axis, bool square);
 
 template <typename T>
 static PlaneArgs<T> plane_args(const Plan& p, const StickTables& st, cplx<T>* work,
-                               int64_t bstride, const T* V) {
+                               int64_t bstride, const T* V, bool square) {
   PlaneArgs<T> g{};
   g.work = work;
   g.bstride = bstride;
@@ -710,14 +719,16 @@ static PlaneArgs<T> plane_args(const Plan& p, const StickTables& st, cplx<T>* wo
   g.colpos = st.d_colpos;
   g.colmap = st.d_colmap;
   g.V = V;
-  g.tw1 = plane_twiddles<T>(p, 0);
-  g.tw2 = plane_twiddles<T>(p, 1);
+  g.tw1 = plane_twiddles<T>(p, 0, square);
+  g.tw2 = plane_twiddles<T>(p, 1, square);
   return g;
 }
 
 template <typename T> PlaneChoice plane_choice(const Plan& p, const StickTables& st) {
   PlaneChoice c;
-  if (!st.d_colpos || !st.d_colmap || !plane_twiddles<T>(p, 0) || !plane_twiddles<T>(p, 1))
+  const bool square = p.n1 == p.n2 && p.n1 <= 128;
+  if (!st.d_colpos || !st.d_colmap || !plane_twiddles<T>(p, 0, square) ||
+      !plane_twiddles<T>(p, 1, square))
     return c;
   int per1 = 0, per2 = 0, wprune = 0, wfull = 0, any_rows = 0;
   bool prune1 = false, prune2 = false;
@@ -737,7 +748,7 @@ template <typename T> PlaneChoice plane_choice(const Plan& p, const StickTables&
 #undef QEPW_PLANE_N
   if (per1 == 0 || per2 == 0) return c;
   c.prune = prune1 && prune2;
-  c.square = p.n1 == p.n2 && p.n1 <= 128;
+  c.square = square;
   if (c.square) {
     c.waves = c.prune ? wprune : wfull;
   } else if (c.prune) {
@@ -760,7 +771,7 @@ bool launch_plane_stage(const Plan& p, const StickTables& st, cplx<T>* work, int
                         const T* V, int nb, hipStream_t stream) {
   const PlaneChoice& c = sizeof(T) == 8 ? st.plane64 : st.plane32;
   if (c.waves == 0) return false;
-  const PlaneArgs<T> g = plane_args<T>(p, st, work, bstride, V);
+  const PlaneArgs<T> g = plane_args<T>(p, st, work, bstride, V, c.square);
   const dim3 grid(p.n3, nb);
 #define QEPW_PLANE_LAUNCH(K)                                                            \
   do {                                                                                  \
@@ -852,8 +863,7 @@ bool launch_density_stage(const Plan& p, const StickTables& st, cplx<T>* work, i
   if (c.waves == 0) return false;
   if (*slices == 0) *slices = density_slices(c, p.n3, nb, most);
   DensityArgs<T> d{};
-  d.plane = plane_args<T>(p, st, work, bstride, nullptr);
-  if (c.square && density_held<T>(p.n1)) d.plane.tw1 = line_twiddles(p, T(0));
+  d.plane = plane_args<T>(p, st, work, bstride, nullptr, c.square);
   d.nb = nb;
   d.per = (nb + *slices - 1) / *slices;
   d.accumulate = accumulate ? 1 : 0;
@@ -907,7 +917,7 @@ int launch_plane_group(int count, const Plan* const* plans, cplx<T>* const* work
     g.start[j] = (int)total;
     g.n3[j] = p.n3;
     g.prune[j] = c.prune ? 1 : 0;
-    g.plane[j] = plane_args<T>(p, p.sphere, work[j], bstride[j], V[j]);
+    g.plane[j] = plane_args<T>(p, p.sphere, work[j], bstride[j], V[j], true);
     total += (int64_t)p.n3 * nb[j];
     int per = 0;
 #define QEPW_PLANE_N(NN) if (p.n1 == NN) per = PlaneLine<NN>::per_wave;

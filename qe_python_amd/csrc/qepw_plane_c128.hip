@@ -3,8 +3,10 @@
 
 namespace qepw {
 
-template <> const double2* plane_twiddles<double>(const Plan& p, int axis) {
-  return plane_lane_table(axis == 0 ? p.n1 : p.n2, true) ? p.d_ltw64[axis] : p.d_tw64[axis];
+template <> const double2* plane_twiddles<double>(const Plan& p, int axis, bool square) {
+  const int n = axis == 0 ? p.n1 : p.n2;
+  return (square ? plane_square_table(n, true) : plane_lane_table(n, true)) ? p.d_ltw64[axis]
+                                                                          : p.d_tw64[axis];
 }
 
 template PlaneChoice plane_choice<double>(const Plan& p, const StickTables& st);

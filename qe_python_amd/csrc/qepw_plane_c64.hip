@@ -3,8 +3,10 @@
 
 namespace qepw {
 
-template <> const float2* plane_twiddles<float>(const Plan& p, int axis) {
-  return plane_lane_table(axis == 0 ? p.n1 : p.n2, false) ? p.d_ltw32[axis] : p.d_tw32[axis];
+template <> const float2* plane_twiddles<float>(const Plan& p, int axis, bool square) {
+  const int n = axis == 0 ? p.n1 : p.n2;
+  return (square ? plane_square_table(n, false) : plane_lane_table(n, false)) ? p.d_ltw32[axis]
+                                                                          : p.d_tw32[axis];
 }
 
 template PlaneChoice plane_choice<float>(const Plan& p, const StickTables& st);

@@ -419,3 +419,33 @@ def test_grouped_bands_beyond_one_launch():
     dv.DeviceFFTPlan.apply_local_group(items)
     for (_, _, y, _, _, _), z in zip(items, alone):
         assert torch.equal(y, z)
+
+
+@pytest.mark.parametrize("n", [27, 54, 75, 80, 81, 90])
+def test_square_planes_about_the_held_twiddles(n):
+    """Squares whose lines hold their twiddles and those that load them, in both
+    precisions, h_psi against the oracle and the density against NumPy."""
+    from qe_python_amd.basis import LocalPotentialWorkspace, PlaneWaveBasis
+    from qe_python_amd.diagonalization import PlaneWaveHamiltonian
+    rng = np.random.default_rng(n)
+    shape = (n, n, 16)
+    ax = [np.arange(-((q + 1) // 4), (q - 1) // 4 + 1) for q in shape]
+    m = np.stack(np.meshgrid(*ax, indexing="ij"), -1).reshape(-1, 3)
+    mid, half = (np.array([(a[0] + a[-1]) / 2.0 for a in ax]),
+                 np.array([len(a) / 2.0 for a in ax]))
+    m = m[(((m - mid) / half) ** 2).sum(1) <= 1.0].astype(np.int32)
+    kin = 0.5 * (m.astype(float) ** 2).sum(1) / 100.0
+    vr = rng.uniform(-1.0, 0.5, shape)
+    x = rng.standard_normal((len(m), 3)) + 1j * rng.standard_normal((len(m), 3))
+    ref = OracleHamiltonian(m, kin, shape, vr).apply(x)
+    basis = PlaneWaveBasis(m, m.astype(float), kin)
+    for precision, tol in (("fp64", 1e-12), ("fp32", 2e-6)):
+        ham = PlaneWaveHamiltonian(basis, np.zeros(shape, complex), (), real_potential=vr,
+                                   precision=precision)
+        assert rel(ham.apply(x), ref) <= tol
+    rho = np.zeros(shape)
+    LocalPotentialWorkspace(m, shape).accumulate_density(rho, x, np.ones(3))
+    grid = np.zeros((3,) + shape, complex)
+    grid[(slice(None),) + tuple((m % np.array(shape)).T)] = x.T
+    dens = (np.abs(np.fft.ifftn(grid, axes=(1, 2, 3), norm="forward")) ** 2).sum(0)
+    np.testing.assert_allclose(rho, dens, rtol=0, atol=1e-12 * dens.max())
