@@ -114,9 +114,9 @@ int qepw_apply_local_timed(const qepw_plan* plan, int precision, const void* vec
  * precision): arrays of ``count`` entries, the arguments of qepw_apply_local
  * per problem.  Problems whose grid lengths have a grouped kernel (square
  * planes of side and z length 36, 48, 54, 60, 64, 72, 80 or 96, the team plane
- * stage, all bands in one workspace) share three launches -- z-stage inverse,
- * planes, z-stage forward -- for up to 24 problems; the others run one by
- * one.  Results equal the one-problem calls bit for bit.  The batched form of
+ * stage, all bands in one workspace) share the launches -- z-stage inverse,
+ * planes (one launch per kind of plane kernel, one for sides up to 54 and 64), z-stage
+ * forward -- for up to 24 problems; the others run one by one.  Results equal the one-problem calls bit for bit.  The batched form of
  * the reference's per-k-point loop (qepy_pw/pw/scf.py:3340-3537) applying
  * H on each k-point's bands (LocalPotentialWorkspace.apply,
  * qepy_pw/basis.py:1354-1455).

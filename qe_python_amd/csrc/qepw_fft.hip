@@ -438,8 +438,8 @@ __global__ __launch_bounds__(kTeamThreads) void k_sticks_forward_team(
 // ---- one launch per stage for many problems --------------------------------
 // The h_psi FFT phase of up to kMaxFftGroup independent problems (k-points,
 // cells: each its own plan, bands, potential and workspace, in one precision)
-// runs as three launches in all.  Every problem's workgroups of a stage are
-// laid end to end along x (start[p] .. start[p + 1]); a workgroup finds its
+// runs as a launch per z stage and one per class of planes (plane_group_class).
+// Every problem's workgroups of a launch are laid end to end along x (start[p] .. start[p + 1]); a workgroup finds its
 // problem from that prefix, then runs the same register team FFT body as the
 // one-problem kernels for its grid length, chosen at run time among
 // QEPW_GROUP_SIZES.
@@ -659,6 +659,10 @@ static bool group_size(int n) {
   return false;
 }
 
+template <typename T> static const PlaneChoice& plane_choice_of(const Plan& p) {
+  return sizeof(T) == 8 ? p.sphere.plane64 : p.sphere.plane32;
+}
+
 // Workgroups of a problem in the grouped stages.
 static int64_t group_planes(const Plan& p, int nb) { return (int64_t)p.n3 * nb; }
 static int64_t group_sticks(const Plan& p, int nb) {
@@ -674,7 +678,8 @@ static bool group_eligible(const Plan& p, int nb, size_t ws_bytes) {
   const StickTables& st = p.sphere;
   if (!(p.n1 == p.n2 && group_size(p.n1) && group_size(p.n3))) return false;
   if (plane_path<T>(p, st) != kPathTeam) return false;
-  if (group_planes(p, nb) > plane_group_most<T>() || group_sticks(p, nb) > kMaxLaunch / kTeamThreads)
+  if (group_planes(p, nb) > plane_group_most(plane_choice_of<T>(p).waves) ||
+      group_sticks(p, nb) > kMaxLaunch / kTeamThreads)
     return false;
   return (size_t)nb * band_bytes_t<T>(p, st) <= ws_bytes && nb <= 65535;
 }
@@ -685,7 +690,8 @@ int apply_local_group_t(int count, const Plan* const* plans, const void* const* 
                         const void* const* kinetics, void* const* results, const int64_t* ldr,
                         void* const* workspaces, const size_t* ws_bytes, hipStream_t stream) {
   // problems that cannot join run on their own; the rest in groups of at most
-  // kMaxFftGroup and what a launch holds, three launches per group
+  // kMaxFftGroup and what a launch holds: the z stages and, of each class of planes
+  // (plane_group_class), the plane stage in one launch per group
   std::vector<int> members;
   for (int i = 0; i < count; ++i) {
     if (nb[i] <= 0) continue;
@@ -698,14 +704,18 @@ int apply_local_group_t(int count, const Plan* const* plans, const void* const* 
       if (rc != QEPW_OK) return rc;
     }
   }
+  const auto class_of = [&](int i) {
+    return plane_group_class(*plans[i], plane_choice_of<T>(*plans[i]), sizeof(T) == 8);
+  };
+  std::stable_sort(members.begin(), members.end(),
+                   [&](int x, int y) { return class_of(x) < class_of(y); });
   int m = 0;
   for (size_t g0 = 0; g0 < members.size(); g0 += m) {
-    int64_t planes = 0, sticks = 0;
+    int64_t sticks = 0;
     for (m = 0; m < kMaxFftGroup && g0 + m < members.size(); ++m) {
       const int i = members[g0 + m];
-      planes += group_planes(*plans[i], nb[i]);
       sticks += group_sticks(*plans[i], nb[i]);
-      if (planes > plane_group_most<T>() || sticks > kMaxLaunch / kTeamThreads) break;
+      if (sticks > kMaxLaunch / kTeamThreads) break;
     }
     StickGroupArgs<T> sa{};
     sa.count = m;
@@ -745,8 +755,18 @@ int apply_local_group_t(int count, const Plan* const* plans, const void* const* 
     allow_lds(reinterpret_cast<const void*>(&k_sticks_group<T, true>), stick_lds);
     hipLaunchKernelGGL((k_sticks_group<T, false>), dim3((unsigned)stotal), dim3(kTeamThreads),
                        stick_lds, stream, sa);
-    const int rc = launch_plane_group<T>(m, gplan, sa.work, sa.bstride, gV, gnb, stream);
-    if (rc != QEPW_OK) return rc;
+    for (int j0 = 0, j1; j0 < m; j0 = j1) {
+      const int i0 = members[g0 + j0];
+      const int64_t most = plane_group_most(plane_choice_of<T>(*plans[i0]).waves);
+      int64_t planes = 0;
+      for (j1 = j0; j1 < m; ++j1) {
+        planes += group_planes(*gplan[j1], gnb[j1]);
+        if (planes > most || class_of(members[g0 + j1]) != class_of(i0)) break;
+      }
+      const int rc = launch_plane_group<T>(j1 - j0, gplan + j0, sa.work + j0, sa.bstride + j0,
+                                           gV + j0, gnb + j0, stream);
+      if (rc != QEPW_OK) return rc;
+    }
     hipLaunchKernelGGL((k_sticks_group<T, true>), dim3((unsigned)stotal), dim3(kTeamThreads),
                        stick_lds, stream, sa);
   }

@@ -85,8 +85,17 @@ template <typename T>
 bool launch_density_stage(const Plan& p, const StickTables& st, cplx<T>* work, int64_t bstride,
                           const double* weights, int nb, int most, int* slices, bool accumulate,
                           double* partial, hipStream_t stream);
-// Planes (of all bands and problems) of one grouped launch.
-template <typename T> int64_t plane_group_most();
+// Planes (of all bands and problems) of one grouped launch, and the class of a
+// problem: those of one class share a launch (k_plane_group).  Lengths whose kernels
+// take up to 156 registers in FP64, or 117 in FP32, share a kernel (0); the others
+// have one each, which their registers would otherwise set for all.
+inline int64_t plane_group_most(int waves) { return kMaxLaunch / (64 * waves); }
+constexpr int plane_group_kind(int n, bool fp64) {
+  return (fp64 ? n <= 54 || n == 64 : n <= 72) ? 0 : n;
+}
+inline int plane_group_class(const Plan& p, const PlaneChoice& c, bool fp64) {
+  return (plane_group_kind(p.n1, fp64) * 16 + c.waves) * 2 + (c.prune ? 1 : 0);
+}
 template <typename T>
 int launch_plane_group(int count, const Plan* const* plans, cplx<T>* const* work,
                        const int64_t* bstride, const T* const* V, const int* nb,

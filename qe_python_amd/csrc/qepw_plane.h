@@ -437,40 +437,56 @@ __global__ __launch_bounds__(64 * kPlaneAnyWaves, 3) void k_plane_any(PlaneArgs<
 }
 
 // ---- one launch for many problems ---------------------------------------------
-// The plane stage of up to kMaxFftGroup square problems: workgroups of all
-// problems end to end along x, each finding its problem in a prefix table and
-// running the one-problem body of its length.
+// The plane stage of up to kMaxFftGroup square problems of one class
+// (plane_group_class): workgroups of all problems end to end along x, each finding
+// its problem in a prefix table and running the one-problem body of its length.
+// A class's lengths have the same waves, pruning and about the same registers: one
+// kernel for all, on the most waves that any length needs, took 1.2 - 2.4 times as
+// long (FFT phase, us: 24 problems of 36^3 with 16 bands, FP64 318 -> 160, FP32 240
+// -> 107; 8 of 72^3 with 32 bands 858 -> 601, 565 -> 335), and one of all lengths and both
+// prunings of the same waves 10 - 20% longer in FP32, whose waves it cuts to three a
+// SIMD.
 template <typename T> struct PlaneGroup {
   int count;
   int start[kMaxFftGroup + 1];
   int n3[kMaxFftGroup];
-  int prune[kMaxFftGroup];
   PlaneArgs<T> plane[kMaxFftGroup];
 };
 
-template <typename T> constexpr int plane_group_waves() {
-  int w = 0;
-#define QEPW_PLANE_CASE(NN)                            \
-  w = std::max(w, plane_waves<T, NN, true>());         \
-  w = std::max(w, plane_waves<T, NN, false>());
+template <typename T> constexpr bool plane_group_waves() {
+  bool ok = true;
+  const auto one = [](int w) { return w == 4 || w == 8 || w == 12; };
+#define QEPW_PLANE_CASE(NN) \
+  ok = ok && one(plane_waves<T, NN, true>()) && one(plane_waves<T, NN, false>());
   QEPW_GROUP_SIZES(QEPW_PLANE_CASE)
 #undef QEPW_PLANE_CASE
-  return w;
+  return ok;
 }
 
-template <typename T>
-__global__ __launch_bounds__(64 * plane_group_waves<T>(), 3) void k_plane_group(
+// Whether a length's kernel is of a group kernel's class.
+template <typename T, int N, int W, bool PRUNE, int KIND> constexpr bool plane_group_case() {
+  return plane_waves<T, N, PRUNE>() == W && plane_group_kind(N, sizeof(T) == 8) == KIND;
+}
+template <typename T, int W, bool PRUNE, int KIND> constexpr bool plane_group_any() {
+  bool any = false;
+#define QEPW_PLANE_CASE(NN) any = any || plane_group_case<T, NN, W, PRUNE, KIND>();
+  QEPW_GROUP_SIZES(QEPW_PLANE_CASE)
+#undef QEPW_PLANE_CASE
+  return any;
+}
+
+template <typename T, int W, bool PRUNE, int KIND>
+__global__ __launch_bounds__(64 * W, sizeof(T) == 4 && PRUNE ? 4 : 3) void k_plane_group(
     const PlaneGroup<T> g) {
-  constexpr int W = plane_group_waves<T>();
   const int p = group_of(g.start, g.count, blockIdx.x);
   const int l = blockIdx.x - g.start[p];
   const int z = l % g.n3[p];
   const int64_t b = l / g.n3[p];
   switch (g.plane[p].n1) {
-#define QEPW_PLANE_CASE(NN)                                                       \
-  case NN:                                                                        \
-    if (g.prune[p]) plane_square_body<T, NN, true, W>(g.plane[p], z, b);          \
-    else plane_square_body<T, NN, false, W>(g.plane[p], z, b);                    \
+#define QEPW_PLANE_CASE(NN)                                           \
+  case NN:                                                            \
+    if constexpr (plane_group_case<T, NN, W, PRUNE, KIND>())          \
+      plane_square_body<T, NN, PRUNE, W>(g.plane[p], z, b);           \
     break;
     QEPW_GROUP_SIZES(QEPW_PLANE_CASE)
 #undef QEPW_PLANE_CASE
@@ -897,42 +913,58 @@ bool launch_density_stage(const Plan& p, const StickTables& st, cplx<T>* work, i
   return false;
 }
 
-template <typename T> int64_t plane_group_most() {
-  return kMaxLaunch / (64 * plane_group_waves<T>());
-}
-
-// The grouped plane stage of ``count`` square problems whose lengths are among
-// QEPW_GROUP_SIZES (nb bands each).
+// The grouped plane stage of ``count`` square problems of one class whose lengths
+// are among QEPW_GROUP_SIZES (nb bands each).
 template <typename T>
 int launch_plane_group(int count, const Plan* const* plans, cplx<T>* const* work,
                        const int64_t* bstride, const T* const* V, const int* nb,
                        hipStream_t stream) {
+  static_assert(plane_group_waves<T>(), "waves of the group kernels");
   PlaneGroup<T> g{};
   g.count = count;
   int64_t total = 0;
   size_t lds = 0;
+  const auto choice = [](const Plan& p) -> const PlaneChoice& {
+    return sizeof(T) == 8 ? p.sphere.plane64 : p.sphere.plane32;
+  };
+  const int kind = plane_group_class(*plans[0], choice(*plans[0]), sizeof(T) == 8);
   for (int j = 0; j < count; ++j) {
     const Plan& p = *plans[j];
-    const PlaneChoice& c = sizeof(T) == 8 ? p.sphere.plane64 : p.sphere.plane32;
+    const PlaneChoice& c = choice(p);
+    if (plane_group_class(p, c, sizeof(T) == 8) != kind) return QEPW_ERR_UNSUPPORTED;
     g.start[j] = (int)total;
     g.n3[j] = p.n3;
-    g.prune[j] = c.prune ? 1 : 0;
     g.plane[j] = plane_args<T>(p, p.sphere, work[j], bstride[j], V[j], true);
     total += (int64_t)p.n3 * nb[j];
-    int per = 0;
-#define QEPW_PLANE_N(NN) if (p.n1 == NN) per = PlaneLine<NN>::per_wave;
-    QEPW_GROUP_SIZES(QEPW_PLANE_N)
-#undef QEPW_PLANE_N
-    lds = std::max(lds, std::max((size_t)(p.sphere.nxcols + 1),
-                                 (size_t)plane_group_waves<T>() * per) *
-                            (p.n1 + 1) * sizeof(cplx<T>));
+    lds = std::max(lds, c.lds);
   }
-  if (total > plane_group_most<T>() || lds > (size_t)kMaxLdsBytes) return QEPW_ERR_UNSUPPORTED;
+  const PlaneChoice& c = choice(*plans[0]);
+  const int length_kind = plane_group_kind(plans[0]->n1, sizeof(T) == 8);
+  if (total > plane_group_most(c.waves)) return QEPW_ERR_UNSUPPORTED;
   g.start[count] = (int)total;
-  allow_lds(reinterpret_cast<const void*>(&k_plane_group<T>), lds);
-  hipLaunchKernelGGL(k_plane_group<T>, dim3((unsigned)total), dim3(64 * plane_group_waves<T>()),
-                     lds, stream, g);
-  return QEPW_OK;
+#define QEPW_GROUP_KERNEL(W, PRUNE, KIND)                                                      \
+  if constexpr (plane_group_any<T, W, PRUNE, KIND>())                                          \
+    if (c.waves == W && c.prune == PRUNE && length_kind == KIND) {                             \
+      allow_lds(reinterpret_cast<const void*>(&k_plane_group<T, W, PRUNE, KIND>), lds);        \
+      hipLaunchKernelGGL((k_plane_group<T, W, PRUNE, KIND>), dim3((unsigned)total),            \
+                         dim3(64 * W), lds, stream, g);                                        \
+      return QEPW_OK;                                                                          \
+    }
+#define QEPW_GROUP_KIND(KIND)        \
+  QEPW_GROUP_KERNEL(4, true, KIND)   \
+  QEPW_GROUP_KERNEL(4, false, KIND)  \
+  QEPW_GROUP_KERNEL(8, true, KIND)   \
+  QEPW_GROUP_KERNEL(8, false, KIND)  \
+  QEPW_GROUP_KERNEL(12, true, KIND)  \
+  QEPW_GROUP_KERNEL(12, false, KIND)
+  QEPW_GROUP_KIND(0)
+  QEPW_GROUP_KIND(60)
+  QEPW_GROUP_KIND(72)
+  QEPW_GROUP_KIND(80)
+  QEPW_GROUP_KIND(96)
+#undef QEPW_GROUP_KIND
+#undef QEPW_GROUP_KERNEL
+  return QEPW_ERR_UNSUPPORTED;
 }
 
 }  // namespace qepw

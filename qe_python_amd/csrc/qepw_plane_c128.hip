@@ -13,7 +13,6 @@ template PlaneChoice plane_choice<double>(const Plan& p, const StickTables& st);
 template bool launch_plane_stage<double>(const Plan& p, const StickTables& st, double2* work,
                                          int64_t bstride, const double* V, int nb,
                                          hipStream_t stream);
-template int64_t plane_group_most<double>();
 template int launch_plane_group<double>(int count, const Plan* const* plans, double2* const* work,
                                         const int64_t* bstride, const double* const* V,
                                         const int* nb, hipStream_t stream);

@@ -13,7 +13,6 @@ template PlaneChoice plane_choice<float>(const Plan& p, const StickTables& st);
 template bool launch_plane_stage<float>(const Plan& p, const StickTables& st, float2* work,
                                          int64_t bstride, const float* V, int nb,
                                          hipStream_t stream);
-template int64_t plane_group_most<float>();
 template int launch_plane_group<float>(int count, const Plan* const* plans, float2* const* work,
                                         const int64_t* bstride, const float* const* V,
                                         const int* nb, hipStream_t stream);

@@ -395,8 +395,8 @@ def test_z_lines_of_the_largest_lengths(n3):
 
 def test_grouped_bands_beyond_one_launch():
     """Problems whose planes together pass 2^32 threads of the grouped plane
-    kernel (12 waves a plane in complex128), with one that passes them alone
-    (its bands run ungrouped): the same bits as problem by problem."""
+    kernel (four waves a plane), with one of more bands than a launch's second
+    dimension (it runs ungrouped): the same bits as problem by problem."""
     import torch
 
     from qe_python_amd import device as dv
@@ -406,7 +406,7 @@ def test_grouped_bands_beyond_one_launch():
     m = np.array([[0, 0, 0], [1, 0, 2], [0, -1, 1], [-2, 3, 0], [1, 0, -5]], dtype=np.int32)
     gen = torch.Generator(device=dev).manual_seed(5)
     items, alone = [], []
-    for nb in (30000, 29000, 60000, 100):
+    for nb in (65000, 64000, 63000, 70000, 100):
         plan = LocalPotentialWorkspace(m, shape).plan
         x = torch.randn((nb, len(m)), dtype=torch.complex128, device=dev, generator=gen)
         v = torch.randn(shape[::-1], dtype=torch.float64, device=dev, generator=gen)
@@ -415,7 +415,7 @@ def test_grouped_bands_beyond_one_launch():
         items.append((plan, x, y, v, kin, dv.Workspace(dev)))
         plan.apply_local(x, z, v, kin, dv.Workspace(dev))
         alone.append(z)
-    assert 96 * 59000 * 768 > 1 << 32 and 96 * 60000 * 768 > 1 << 32
+    assert 96 * (65000 + 64000 + 63000) * 256 > 1 << 32
     dv.DeviceFFTPlan.apply_local_group(items)
     for (_, _, y, _, _, _), z in zip(items, alone):
         assert torch.equal(y, z)
@@ -449,3 +449,36 @@ def test_square_planes_about_the_held_twiddles(n):
     grid[(slice(None),) + tuple((m % np.array(shape)).T)] = x.T
     dens = (np.abs(np.fft.ifftn(grid, axes=(1, 2, 3), norm="forward")) ** 2).sum(0)
     np.testing.assert_allclose(rho, dens, rtol=0, atol=1e-12 * dens.max())
+
+
+def test_grouped_problems_of_different_waves():
+    """Grouped problems whose plane kernels differ in their waves (96^2 beside
+    smaller planes in complex128; bases that fill the axes) in any order: the
+    same bits as problem by problem."""
+    import torch
+
+    from qe_python_amd import device as dv
+    from qe_python_amd.basis import LocalPotentialWorkspace
+    dev = torch.device("cuda", torch.cuda.current_device())
+    gen = torch.Generator(device=dev).manual_seed(11)
+    for dtype in (torch.complex128, torch.complex64):
+        items, alone = [], []
+        for n, n3, dense, nb in ((96, 36, False, 3), (36, 48, False, 5), (60, 36, True, 2),
+                                 (96, 48, False, 1), (72, 36, True, 2), (80, 36, False, 4),
+                                 (36, 36, True, 1)):
+            shape = (n, n, n3)
+            ax = [np.arange(-((q - 1) // 2), q // 2 + 1) if dense
+                  else np.arange(-((q - 1) // 4), (q - 1) // 4 + 1) for q in shape]
+            m = np.stack(np.meshgrid(*ax, indexing="ij"), -1).reshape(-1, 3)[::3].astype(np.int32)
+            plan = LocalPotentialWorkspace(m, shape).plan
+            x = torch.randn((nb, len(m)), dtype=dtype, device=dev, generator=gen)
+            real = dv.real_dtype(dtype)
+            v = torch.randn(shape[::-1], dtype=real, device=dev, generator=gen)
+            kin = torch.rand(len(m), dtype=real, device=dev, generator=gen)
+            y, z = torch.full_like(x, 9.0), torch.full_like(x, 9.0)
+            items.append((plan, x, y, v, kin, dv.Workspace(dev)))
+            plan.apply_local(x, z, v, kin, dv.Workspace(dev))
+            alone.append(z)
+        dv.DeviceFFTPlan.apply_local_group(items)
+        for (_, _, y, _, _, _), z in zip(items, alone):
+            assert torch.equal(y, z)
