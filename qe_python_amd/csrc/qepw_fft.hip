@@ -439,10 +439,10 @@ __global__ __launch_bounds__(kTeamThreads) void k_sticks_forward_team(
 // The h_psi FFT phase of up to kMaxFftGroup independent problems (k-points,
 // cells: each its own plan, bands, potential and workspace, in one precision)
 // runs as a launch per z stage and one per class of planes (plane_group_class).
-// Every problem's workgroups of a launch are laid end to end along x (start[p] .. start[p + 1]); a workgroup finds its
-// problem from that prefix, then runs the same register team FFT body as the
-// one-problem kernels for its grid length, chosen at run time among
-// QEPW_GROUP_SIZES.
+// Every problem's workgroups of a launch are laid end to end along x (start[p] ..
+// start[p + 1]); a workgroup finds its problem from that prefix, then runs the same
+// register team FFT body as the one-problem kernels for its grid length, chosen at run
+// time among QEPW_GROUP_SIZES.
 
 template <typename T> struct StickGroupArgs {
   int count;
