@@ -6,14 +6,13 @@
 //   op C : re += Ar Br + Ai Bi ;  im += Ar Bi - Ai Br
 // (op(B) = B^H is conjugated as it is staged into LDS).
 // using v_mfma_f64_16x16x4f64 (FP64) or v_mfma_f32_16x16x4f32 (FP32, FP32
-// accumulation).  A 256-thread workgroup owns a TILE x TILE output tile
-// (TILE = 64, or 32 for small outputs such as the reduced problem's square
-// products, where 64x64 tiles leave most CUs idle); each of its four waves
-// owns a quarter (2x2 or 1x1 MFMA blocks of 16x16) and walks K in steps of
-// 8 or 16 staged through LDS.  Tall-skinny A^H B products (K = npw up
-// to ~24k, M,N <= 512) are split over K: every split writes its partial tile
-// to the workspace and a second kernel sums the splits in fixed order, so
-// results are bitwise reproducible run to run.
+// accumulation).  A 256-thread workgroup owns a TM x TN output tile (kVariants:
+// eight shapes from 32 x 32 to 128 x 64); each of its four waves owns a part of
+// 16x16 MFMA blocks and walks K in steps of 8 or 16 staged through LDS.  Products
+// with few tiles (A^H B over K = npw above all) are split over K: every split
+// writes its partial tile to the workspace and a second kernel sums the splits in
+// fixed order, so results are bitwise reproducible run to run, and the plan depends
+// on the shape alone (a workspace below the quoted one: gemm_t).
 //
 // MFMA 16x16x4 operand layout (lane l of a wave64): A element (row l%16,
 // k l/16); B element (k l/16, col l%16).  Accumulator v of lane l holds
@@ -582,7 +581,6 @@ static bool gemv_direct(bool ca, int64_t m, int64_t k) {
   return ca ? k <= 8192 || (m >= 64 && k <= 32768) : k <= 384;
 }
 
-// Tile variants of k_cgemm: (TM, TN, WAVES_M).
 // The projector force, dE/dtau_a,c = 2 sum_n f_n Re sum_{i in a} conj(dO_c[i,n])
 // (D O)[i,n] with dO_c = i B^H (q_c psi), in one product over the bands instead of
 // three over the plane waves: with W = psi (f D O)^H (npw x P),
@@ -673,6 +671,7 @@ __global__ __launch_bounds__(1024) void k_force_sum(const double* __restrict__ p
   if (tid == 0) out[3 * a + c] = 2.0 * sh[0];
 }
 
+// Tile variants of k_cgemm: (TM, TN, WAVES_M).
 struct GemmVariant {
   int tm, tn, waves_m;
 };

@@ -1,5 +1,6 @@
 // The xy-plane stage on register "team" FFTs (qepw_regfft.h): one workgroup
-// per (z-plane, band), any pair of team lengths n1 (x) and n2 (y).
+// per (z-plane, band), any pair of team lengths n1 (x) and n2 (y) whose rows the
+// teams of twelve waves hold (plane_choice).
 //
 // LDS holds only the nxc occupied x columns of the plane, Q[c * NP2 + y], plus
 // one all-zero column:
@@ -378,7 +379,10 @@ __global__ __launch_bounds__(64 * W, W > 12 ? 4 : 3) void k_plane_square(PlaneAr
 // x 90 1751 / 1440 -> 458 / 277, 108 x 120 x 60 3857 / 3192 -> 926 / 386.
 constexpr int kPlaneAnyWaves = 12;
 // Rows per team of the run-time kernels: with six kept slots three FP64 rows
-// spill (90 x 108 x 60, 128 bands: 913 us with three, 685 us with two).
+// spill (90 x 108 x 60, 128 bands: 913 us with three, 685 us with two).  Planes of
+// more rows than that on twelve waves' teams (in FP64 n2 > 24 or 36 teams of a wave:
+// 120 x 128, 90 x 160, 108 x 128, 100 x 150) are left to the generic and split
+// stages, as they were.
 template <typename T, int N1> constexpr int plane_any_rows() {
   return sizeof(T) == 8 && plane_kept<N1, true>() > 4 ? 2 : 3;
 }

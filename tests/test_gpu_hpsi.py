@@ -482,3 +482,23 @@ def test_grouped_problems_of_different_waves():
         dv.DeviceFFTPlan.apply_local_group(items)
         for (_, _, y, _, _, _), z in zip(items, alone):
             assert torch.equal(y, z)
+
+
+@pytest.mark.parametrize("shape,fp64,fp32", [
+    ((128, 120, 16), True, True), ((96, 128, 16), True, True), ((75, 108, 16), True, True),
+    ((120, 128, 16), False, True), ((90, 160, 16), False, True), ((144, 144, 16), False, True)])
+def test_rectangles_on_the_team_stage(shape, fp64, fp32):
+    """Which large rectangles run on the team stage, whose workspace is the
+    sticks', and which take the split stage with its column lines."""
+    import torch
+
+    from qe_python_amd.basis import LocalPotentialWorkspace
+    ax = [np.arange(-((n + 1) // 4), (n - 1) // 4 + 1) for n in shape]
+    m = np.stack(np.meshgrid(*ax, indexing="ij"), -1).reshape(-1, 3)
+    half, mid = (np.array([len(a) / 2.0 for a in ax]),
+                 np.array([(a[0] + a[-1]) / 2.0 for a in ax]))
+    m = m[(((m - mid) / half) ** 2).sum(1) <= 1.0].astype(np.int32)
+    plan = LocalPotentialWorkspace(m, shape).plan
+    for dtype, size, team in ((torch.complex128, 16, fp64), (torch.complex64, 8, fp32)):
+        band = plan.workspace_bytes(dtype, 3) - plan.workspace_bytes(dtype, 2)
+        assert (band == plan.sticks * shape[2] * size) == team, (dtype, band)
